@@ -447,8 +447,9 @@ __device__ __forceinline__ double eval_terms(const TView& TV, const MolDesc& m, 
 // read with readlane and combined in a fixed order, so every lane gets the same value.
 template <int CTRL>
 __device__ __forceinline__ double dpp_d(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+  // every lane reads a lane of its own row, so no lane keeps an old value
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
   return __hiloint2double(hi, lo);
 }
 __device__ __forceinline__ double lane_d(double v, int lane) {
@@ -456,25 +457,11 @@ __device__ __forceinline__ double lane_d(double v, int lane) {
   const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
   return __hiloint2double(hi, lo);
 }
-constexpr int DPP_QUAD_XOR1 = 0xB1, DPP_QUAD_XOR2 = 0x4E, DPP_ROW_HALF_MIRROR = 0x141, DPP_ROW_MIRROR = 0x140;
-__device__ __forceinline__ double wsum(double v) {
-  v += dpp_d<DPP_QUAD_XOR1>(v);
-  v += dpp_d<DPP_QUAD_XOR2>(v);
-  v += dpp_d<DPP_ROW_HALF_MIRROR>(v);
-  v += dpp_d<DPP_ROW_MIRROR>(v);
-  return ((lane_d(v, 0) + lane_d(v, 16)) + lane_d(v, 32)) + lane_d(v, 48);
-}
-__device__ __forceinline__ double wmax(double v) {
-  v = fmax(v, dpp_d<DPP_QUAD_XOR1>(v));
-  v = fmax(v, dpp_d<DPP_QUAD_XOR2>(v));
-  v = fmax(v, dpp_d<DPP_ROW_HALF_MIRROR>(v));
-  v = fmax(v, dpp_d<DPP_ROW_MIRROR>(v));
-  return fmax(fmax(lane_d(v, 0), lane_d(v, 16)), fmax(lane_d(v, 32), lane_d(v, 48)));
-}
-
+constexpr int DPP_QUAD_XOR1 = 0xB1, DPP_QUAD_XOR2 = 0x4E, DPP_QUAD_REV = 0x1B, DPP_ROW_HALF_MIRROR = 0x141,
+              DPP_ROW_ROR8 = 0x128;
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
 }
 
 // four consecutive elements (t, j..j+3) of a symmetric matrix in padded packed storage
@@ -595,31 +582,111 @@ __device__ __forceinline__ void hcol_update4(float* col, const float2* AB, float
   }
 }
 
+// Sums (or maxima) of K values per lane over a wave at once. At each butterfly step a lane keeps
+// one of two values and sends the other to its partner, so the values left halve from step to
+// step instead of each going through all steps: 69 instructions for K = 8, against 248 for
+// eight separate wsum (of 16-28 per value, a third of them DPP moves). Lane bits 0-2 end up
+// selecting the value: value q is in lanes l with (l & (KP - 1)) == q. Each value's additions
+// pair the same lanes in the same order as wsum's (IEEE addition commutes), so the result has
+// the same bits.
+template <bool MAX>
+__device__ __forceinline__ double red_op(double a, double b) {
+  return MAX ? fmax(a, b) : a + b;
+}
+// lane l of a row receives lane l ^ X of the same row
+template <int X>
+__device__ __forceinline__ double row_xor(double v) {
+  if constexpr (X == 1) return dpp_d<DPP_QUAD_XOR1>(v);
+  if constexpr (X == 2) return dpp_d<DPP_QUAD_XOR2>(v);
+  if constexpr (X == 4) return dpp_d<DPP_QUAD_REV>(dpp_d<DPP_ROW_HALF_MIRROR>(v));  // l ^ 7, then ^ 3
+  return dpp_d<DPP_ROW_ROR8>(v);
+}
+template <int K, int X, bool MAX>
+__device__ __forceinline__ void red_step(const double (&v)[K], double (&r)[(K + 1) / 2], int lane) {
+  const bool up = (lane & X) != 0;
+#pragma unroll
+  for (int k = 0; k < K / 2; k++) {
+    const double keep = up ? v[2 * k + 1] : v[2 * k], send = up ? v[2 * k] : v[2 * k + 1];
+    r[k] = red_op<MAX>(keep, row_xor<X>(send));
+  }
+  if (K & 1) r[K / 2] = red_op<MAX>(v[K - 1], row_xor<X>(v[K - 1]));
+}
+// ((row 0 + row 1) + row 2) + row 3 of lane l's column, in every row
+template <bool MAX>
+__device__ __forceinline__ double red_rows(double v) {
+  const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+  const auto l2 = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);  // rows {0, 1} / {2, 3} in both halves
+  const auto h2 = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  const auto l01 = __builtin_amdgcn_permlane16_swap(l2[0], l2[0], false, false);
+  const auto h01 = __builtin_amdgcn_permlane16_swap(h2[0], h2[0], false, false);
+  const auto l23 = __builtin_amdgcn_permlane16_swap(l2[1], l2[1], false, false);
+  const auto h23 = __builtin_amdgcn_permlane16_swap(h2[1], h2[1], false, false);
+  const double r0 = __hiloint2double((int)h01[0], (int)l01[0]), r1 = __hiloint2double((int)h01[1], (int)l01[1]);
+  const double r2 = __hiloint2double((int)h23[0], (int)l23[0]), r3 = __hiloint2double((int)h23[1], (int)l23[1]);
+  return MAX ? fmax(fmax(r0, r1), fmax(r2, r3)) : ((r0 + r1) + r2) + r3;
+}
+// value q of v over the wave, in the lanes with (lane & 7) == q (K > 4), (lane & 3) == q (K > 2), ...
+template <int K, bool MAX>
+__device__ __forceinline__ double wave_red(const double (&v)[K], int lane) {
+  double a[(K + 1) / 2], b[(K + 3) / 4], c[(K + 7) / 8];
+  red_step<K, 1, MAX>(v, a, lane);
+  red_step<(K + 1) / 2, 2, MAX>(a, b, lane);
+  red_step<(K + 3) / 4, 4, MAX>(b, c, lane);
+  return red_rows<MAX>(red_op<MAX>(c[0], row_xor<8>(c[0])));
+}
+
 template <int NT>
 struct Reducer {
   static constexpr int NW = NT / 64;
   double* buf;  // RED_DOUBLES(NT) = 2 phases * NW * 8 doubles
   int phase;
-  // K values; bit k of MAXMASK selects max instead of sum
-  template <int K, int MAXMASK>
-  __device__ __forceinline__ void run(double (&v)[K]) {
-#pragma unroll
-    for (int k = 0; k < K; k++) v[k] = ((MAXMASK >> k) & 1) ? wmax(v[k]) : wsum(v[k]);
-    static_assert(K <= 8, "at most 8 values per reduction");
-    double* b = buf + phase * (NW * 8);
+  // K sums followed by KM maxima of v over the workgroup, at most 8 values in all: the waves'
+  // results meet in LDS (lane q writes and later adds up value q, in wave order), and every
+  // lane reads the totals from the lanes that hold them, as wave-uniform values.
+  template <int K, int KM>
+  __device__ __forceinline__ void run(double (&v)[K + KM]) {
+    constexpr int KT = K + KM;
+    static_assert(KT <= 8, "at most 8 values per reduction");
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) {
+    double s = 0.0, x = 0.0;
+    if constexpr (K > 0) {
+      double t[K];
 #pragma unroll
-      for (int k = 0; k < K; k++) b[w * 8 + k] = v[k];
+      for (int k = 0; k < K; k++) t[k] = v[k];
+      s = wave_red<K, false>(t, lane);
     }
-    __syncthreads();
+    if constexpr (KM > 0) {
+      double t[KM];
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-      double a = b[k];
-      for (int ww = 1; ww < NW; ww++) a = ((MAXMASK >> k) & 1) ? fmax(a, b[ww * 8 + k]) : a + b[ww * 8 + k];
-      v[k] = a;
+      for (int k = 0; k < KM; k++) t[k] = v[K + k];
+      x = wave_red<KM, true>(t, lane);
     }
-    phase ^= 1;
+    if constexpr (NW == 1) {
+      __syncthreads();  // orders the wave's LDS traffic, as callers expect of a reduction
+    } else {
+      // sums in the words 0..K-1 of a wave's eight, maxima in K..KT-1
+      double* b = buf + phase * (NW * 8);
+      if (K > 0 && lane < K) b[w * 8 + lane] = s;
+      if (KM > 0 && lane < KM) b[w * 8 + K + lane] = x;
+      __syncthreads();
+      if constexpr (K > 0) {
+        const int q = lane & 7;
+        s = b[q];
+#pragma unroll
+        for (int ww = 1; ww < NW; ww++) s += b[ww * 8 + q];
+      }
+      if constexpr (KM > 0) {
+        const int q = (K + lane) & 7;
+        x = b[q];
+#pragma unroll
+        for (int ww = 1; ww < NW; ww++) x = fmax(x, b[ww * 8 + q]);
+      }
+      phase ^= 1;
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) v[k] = lane_d(s, k);
+#pragma unroll
+    for (int k = 0; k < KM; k++) v[K + k] = lane_d(x, k);
   }
   __device__ __forceinline__ double sum(double a) {
     double v[1] = {a};
@@ -628,7 +695,7 @@ struct Reducer {
   }
   __device__ __forceinline__ double max(double a) {
     double v[1] = {a};
-    run<1, 1>(v);
+    run<0, 1>(v);
     return v[0];
   }
 };
@@ -981,7 +1048,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
         v3[1] += (double)d[i] * VG[i].y;
         v3[2] = fmax(v3[2], (double)(fabsf(d[i]) / fmaxf(fabsf(xs[i]), 1.0f)));
       }
-      R.template run<3, 4>(v3);
+      R.template run<2, 1>(v3);
       double slope = v3[1], test = v3[2];
       const double dn = sqrt(v3[0]);
       // a step longer than max_step is scaled down (:157-166); the scale goes into the
@@ -1090,7 +1157,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
         v2[0] = fmax(v2[0], (double)sg);
         v2[1] = fmax(v2[1], (double)sg * fmax((double)fabsf(xs[i]), 1.0));
       }
-      R.template run<2, 3>(v2);
+      R.template run<0, 2>(v2);
       while (v2[0] > GRAD_CAP) {  // scale_grad_serial, mmff_bfgs_header.metal:435-454
         gscale *= 0.5f;
         v2[0] *= 0.5;
