@@ -466,17 +466,17 @@ __device__ __forceinline__ float dpp_f(float v) {
 
 // four consecutive elements (t, j..j+3) of a symmetric matrix in padded packed storage
 // (column c at pcol(c), cb = pcol(t), pj = pcol(j)), with the matching gradient entries
-__device__ __forceinline__ void hrow_load4(const float* H, const float2* VG, int t, int cb, int j, int pj,
+__device__ __forceinline__ void hrow_load4(const float* H, const float* gv, int t, int cb, int j, int pj,
                                            float (&h)[4], float (&w)[4]) {
   const int p1 = pj + ((j + 4) & ~3), p2 = p1 + ((j + 5) & ~3), p3 = p2 + ((j + 6) & ~3);
   h[0] = H[j <= t ? cb + j : pj + t];
   h[1] = H[j + 1 <= t ? cb + j + 1 : p1 + t];
   h[2] = H[j + 2 <= t ? cb + j + 2 : p2 + t];
   h[3] = H[j + 3 <= t ? cb + j + 3 : p3 + t];
-  w[0] = VG[j].y;
-  w[1] = VG[j + 1].y;
-  w[2] = VG[j + 2].y;
-  w[3] = VG[j + 3].y;
+  w[0] = gv[j];
+  w[1] = gv[j + 1];
+  w[2] = gv[j + 2];
+  w[3] = gv[j + 3];
 }
 
 // one row of a column quad of the full Hessian gains a pending rank-2 update: column t's
@@ -504,7 +504,7 @@ __device__ __forceinline__ void hquad_dot(const float4& h, float g, float (&a)[4
 // dot products per update over these rows in lr (s.g, h.g), which the caller combines with
 // the column coefficients after summing the quad's lanes. HQ rows are loaded together.
 template <int HQ, int NU, int NPM>
-__device__ __forceinline__ void hquad_rows(float4* base, int nq, int j, int j1, const float2* VG,
+__device__ __forceinline__ void hquad_rows(float4* base, int nq, int j, int j1, const float* gv,
                                            const float2* const (&S)[NPM], const float (&cx)[NPM][4],
                                            const float (&cy)[NPM][4], float (&a)[4], float (&lr)[2][NPM]) {
   constexpr bool FLUSH = NU == NPM;
@@ -514,7 +514,7 @@ __device__ __forceinline__ void hquad_rows(float4* base, int nq, int j, int j1, 
     for (int u = 0; u < HQ; u++) h[u] = base[(size_t)(j + u) * nq];
 #pragma unroll
     for (int u = 0; u < HQ; u++) {
-      const float g = VG[j + u].y;
+      const float g = gv[j + u];
 #pragma unroll
       for (int k = 0; k < NU; k++) {
         const float2 w = S[k][j + u];
@@ -534,7 +534,7 @@ __device__ __forceinline__ void hquad_rows(float4* base, int nq, int j, int j1, 
   }
   for (; j < j1; j++) {
     float4 h = base[(size_t)j * nq];
-    const float g = VG[j].y;
+    const float g = gv[j];
 #pragma unroll
     for (int k = 0; k < NU; k++) {
       const float2 w = S[k][j];
@@ -552,16 +552,16 @@ __device__ __forceinline__ void hquad_rows(float4* base, int nq, int j, int j1, 
 
 // hquad_rows for the run-time count of pending updates (0..NPM)
 template <int HQ, int NPM, int NU = NPM>
-__device__ __forceinline__ void hquad_dispatch(int npend, float4* base, int nq, int j, int j1, const float2* VG,
+__device__ __forceinline__ void hquad_dispatch(int npend, float4* base, int nq, int j, int j1, const float* gv,
                                                const float2* const (&S)[NPM], const float (&cx)[NPM][4],
                                                const float (&cy)[NPM][4], float (&a)[4], float (&lr)[2][NPM]) {
   if constexpr (NU == 0) {
-    hquad_rows<HQ, 0, NPM>(base, nq, j, j1, VG, S, cx, cy, a, lr);
+    hquad_rows<HQ, 0, NPM>(base, nq, j, j1, gv, S, cx, cy, a, lr);
   } else {
     if (npend == NU)
-      hquad_rows<HQ, NU, NPM>(base, nq, j, j1, VG, S, cx, cy, a, lr);
+      hquad_rows<HQ, NU, NPM>(base, nq, j, j1, gv, S, cx, cy, a, lr);
     else
-      hquad_dispatch<HQ, NPM, NU - 1>(npend, base, nq, j, j1, VG, S, cx, cy, a, lr);
+      hquad_dispatch<HQ, NPM, NU - 1>(npend, base, nq, j, j1, gv, S, cx, cy, a, lr);
   }
 }
 
@@ -822,8 +822,8 @@ __host__ __device__ inline size_t nk_lds_bytes(int algo, int hm, int nt, int max
   size_t b = 16 * nw * sizeof(double) + 64 + 2 * (size_t)LBFGS_MAX_M * sizeof(double);
   b += (size_t)max_n * 8;  // gradient accumulators
   b += (size_t)max_n * 4 * 4;   // xs, d, xo, hd
-  b += (size_t)max_n * 16;      // V = {dg, g, pending xi, pending hd}
-  b += (size_t)max_n * 8;       // per-lane coefficients of the pending update
+  b += (size_t)max_n * 8;       // g, dg
+  b += (size_t)max_n * 16;      // a pending update: s, h, alpha, beta
   if (algo == MMFFHIP_BFGS && (hm == 1 || hm == 3)) b += (size_t)(hpend_for(nt) - 1) * max_n * 16;  // more pending updates
   if (algo == MMFFHIP_BFGS && hm == 3) b += nw * (size_t)sym_acc_floats(max_n) * 4;
   if (algo == MMFFHIP_LBFGS) {
@@ -868,21 +868,27 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
   int* s_int = (int*)(red + 16 * NW);
   double* lb_sc = (double*)(s_int + 16);  // rho[16], alpha[16]
   unsigned long long* gacc = (unsigned long long*)(lb_sc + 2 * LBFGS_MAX_M);
-  float2* VG = (float2*)(gacc + mn);  // {dg, g}
-  float2* SH = VG + mn;               // {s, h} of the last rank-2 update (s = x - x_old, h = H dg)
-  float* xs = (float*)(SH + mn);
+  float* gv = (float*)(gacc + mn);  // scaled gradient g
+  float* dgv = gv + mn;             // its last change dg
+  float* xs = dgv + mn;
   float* d = xs + mn;   // direction (also y2 = H g scratch)
   float* xo = d + mn;   // previous x, then xi = x - x_old
   float* hd = xo + mn;  // H dg (BFGS) / two-loop q (L-BFGS)
-  float2* AB = (float2*)(hd + mn);  // pending update U(t, j) = AB[t].x xi_j + AB[t].y hd_j
-  // global-Hessian BFGS keeps up to NPM pending updates (slot 0 in SH/AB, slot k >= 1 in XS)
-  // and writes H back once every NPM iterations
+  // A rank-2 update U(t, j) = alpha_t s_j + beta_t h_j (s = x - x_old, h = H dg) takes a slot of
+  // 4 mn floats. Global-Hessian BFGS keeps up to NPM pending updates and writes H back once
+  // every NPM iterations; the others apply theirs at once. The symmetric pass reads whole quads
+  // of s, h, alpha and beta (and of g) in one instruction, so it keeps the four in planes:
+  // one conflict-free 16-byte read per quad and plane, where {s, h} and {alpha, beta} pairs
+  // (and {dg, g}) took two 16-byte reads at a 32-byte stride, each a 2-way bank conflict. With
+  // pairs the LDS pipe was busy 63% of the n <= 360 launch of a 100,000-conformer ragged batch.
+  // The other placements read an update row by row and keep the pairs.
   constexpr bool LAZY = (HM == 1 || HM == 3) && ALGO == MMFFHIP_BFGS;
   constexpr int NPM = LAZY ? hpend_for(NT) : 1;
-  float2* XS = AB + mn;
-  auto sh_slot = [&](int k) { return k == 0 ? SH : XS + (size_t)(k - 1) * 2 * mn; };
-  auto ab_slot = [&](int k) { return k == 0 ? AB : XS + (size_t)(k - 1) * 2 * mn + mn; };
-  float* big = (float*)(XS + (size_t)(NPM - 1) * 2 * mn);
+  float* UP = hd + mn;
+  auto up_plane = [&](int k, int c) { return UP + (size_t)(4 * k + c) * mn; };  // c: s, h, alpha, beta
+  auto sh_slot = [&](int k) { return (float2*)up_plane(k, 0); };
+  auto ab_slot = [&](int k) { return (float2*)up_plane(k, 2); };
+  float* big = UP + (size_t)NPM * 4 * mn;
   float* H = HLDS ? big : P.hglob + (size_t)blockIdx.x * P.slot_floats;
   size_t big_floats = 0;
   if (HLDS) big_floats = ALGO == MMFFHIP_BFGS ? packed_floats(mn) : 2 * (size_t)P.m * mn;
@@ -962,9 +968,9 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
       // the padding rows of the last quad: zero gradient and update vectors, so that the
       // padding elements of H stay zero and add nothing to H v
       for (int i = n + tid; i < ((n + 3) & ~3); i += NT) {
-        VG[i] = make_float2(0.f, 0.f);
+        gv[i] = 0.f;
 #pragma unroll
-        for (int k = 0; k < NPM; k++) sh_slot(k)[i] = ab_slot(k)[i] = make_float2(0.f, 0.f);
+        for (int k = 0; k < 4 * NPM; k++) up_plane(0, k)[i] = 0.f;
       }
     }
     float psc = 1.0f;
@@ -1011,8 +1017,8 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
         mxg *= 0.5;
       }
       for (int i = tid; i < n; i += NT) {
-        VG[i] = make_float2(0.f, gread(gacc, i, m.n_atoms) * gscale);
-        SH[i] = make_float2(0.f, 0.f);
+        dgv[i] = 0.f;
+        gv[i] = gread(gacc, i, m.n_atoms) * gscale;
       }
     }
     psc = GRAD_SCALE_INIT / gscale;
@@ -1023,10 +1029,10 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
       if (pc && ALGO == MMFFHIP_BFGS) {
         const int a = i / 3;
         float sacc = 0.f;
-        for (int q = 0; q < 3; q++) sacc += h_init(pc, psc, i, 3 * a + q) * VG[3 * a + q].y;
+        for (int q = 0; q < 3; q++) sacc += h_init(pc, psc, i, 3 * a + q) * gv[3 * a + q];
         d[i] = -sacc;
       } else {
-        d[i] = -VG[i].y;
+        d[i] = -gv[i];
       }
     }
     double ss = 0.0;
@@ -1045,7 +1051,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
       for (int i = tid; i < n; i += NT) {
         xo[i] = xs[i];
         v3[0] += (double)d[i] * d[i];
-        v3[1] += (double)d[i] * VG[i].y;
+        v3[1] += (double)d[i] * gv[i];
         v3[2] = fmax(v3[2], (double)(fabsf(d[i]) / fmaxf(fabsf(xs[i]), 1.0f)));
       }
       R.template run<2, 1>(v3);
@@ -1126,7 +1132,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
           pc = nullptr;
           npend = 0;
           init_h();
-          for (int i = tid; i < n; i += NT) d[i] = -VG[i].y;
+          for (int i = tid; i < n; i += NT) d[i] = -gv[i];
           __syncthreads();
           continue;
         }
@@ -1165,7 +1171,8 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
       }
       for (int i = tid; i < n; i += NT) {
         const float gn = gread(gacc, i, m.n_atoms) * gscale;
-        VG[i] = make_float2(gn - VG[i].y, gn);
+        dgv[i] = gn - gv[i];
+        gv[i] = gn;
       }
       if (v2[1] / fmax(E * (double)gscale, 1.0) < (double)P.grad_tol) {  // :300-316
         status = 0;
@@ -1196,11 +1203,11 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
               int j = j0;
               if (j + 3 < j1) {
                 float h[4], w[4];
-                hrow_load4(H, VG, t, cb, j, pj, h, w);
+                hrow_load4(H, gv, t, cb, j, pj, h, w);
                 while (j + 7 < j1) {
                   float hn[4], wn[4];
                   const int pn = pcol(j + 4);
-                  hrow_load4(H, VG, t, cb, j + 4, pn, hn, wn);
+                  hrow_load4(H, gv, t, cb, j + 4, pn, hn, wn);
   #pragma unroll
                   for (int u = 0; u < 4; u++) {
                     a2[u] += h[u] * w[u];
@@ -1217,7 +1224,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
               }
               for (; j < j1; j++) {
                 const float hv = H[j <= t ? cb + j : pj + t];
-                a2[0] += hv * VG[j].y;
+                a2[0] += hv * gv[j];
                 pj += (j + 4) & ~3;
               }
               float s2 = (a2[0] + a2[1]) + (a2[2] + a2[3]);
@@ -1264,7 +1271,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
           }
           const int steps = nq <= 64 ? (Jw + G - 1) / G : nq < 64 + NW ? 2 * Jw : (Jw * nq + 63) >> 6;
           const bool flush = npend == NPM;
-          const float4* VG4 = (const float4*)VG;  // VG4[i] = {VG[2i], VG[2i + 1]}
+          const float4* gq = (const float4*)gv;
           float4* H4 = (float4*)H;
           for (int kk = 0; kk < steps; kk++) {
             if (j < Jw && L < nq) {
@@ -1276,14 +1283,13 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
                 if (flush) {
 #pragma unroll
                   for (int k = 0; k < NPM; k++) {
-                    const float4* sk = (const float4*)(sh_slot(k) + 4 * L);  // {s, h} of rows 4L..
-                    const float4* ak = (const float4*)(ab_slot(k) + 4 * M);  // {alpha, beta} of columns 4M..
-                    const float4 s01 = sk[0], s23 = sk[1], a01 = ak[0], a23 = ak[1];
-                    const float ux[4] = {a01.x, a01.z, a23.x, a23.z}, uy[4] = {a01.y, a01.w, a23.y, a23.w};
-                    hquad_upd(b0, make_float2(s01.x, s01.y), ux, uy);
-                    hquad_upd(b1, make_float2(s01.z, s01.w), ux, uy);
-                    hquad_upd(b2, make_float2(s23.x, s23.y), ux, uy);
-                    hquad_upd(b3, make_float2(s23.z, s23.w), ux, uy);
+                    const float4 sv = ((const float4*)up_plane(k, 0))[L], hv = ((const float4*)up_plane(k, 1))[L];
+                    const float4 av = ((const float4*)up_plane(k, 2))[M], bv = ((const float4*)up_plane(k, 3))[M];
+                    const float ux[4] = {av.x, av.y, av.z, av.w}, uy[4] = {bv.x, bv.y, bv.z, bv.w};
+                    hquad_upd(b0, make_float2(sv.x, hv.x), ux, uy);
+                    hquad_upd(b1, make_float2(sv.y, hv.y), ux, uy);
+                    hquad_upd(b2, make_float2(sv.z, hv.z), ux, uy);
+                    hquad_upd(b3, make_float2(sv.w, hv.w), ux, uy);
                   }
                   bp[0] = b0;
                   bp[nq] = b1;
@@ -1297,24 +1303,24 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
                 // registers while a lane's L stays fixed measured no faster: 119.9 against
                 // 118.9 ms on the medium workload; loading the next block's rows while this one
                 // is used spilled 76-244 bytes per lane and measured 125.1 against 119.5 ms.)
-                const float4 vm01 = VG4[2 * M], vm23 = VG4[2 * M + 1];
+                const float4 vm = gq[M];
                 float4* a4 = (float4*)(acc + cp * n4);
                 {
                   float4 v = a4[L];
-                  v.x += fmaf(b0.w, vm23.w, fmaf(b0.z, vm23.y, fmaf(b0.y, vm01.w, b0.x * vm01.y)));
-                  v.y += fmaf(b1.w, vm23.w, fmaf(b1.z, vm23.y, fmaf(b1.y, vm01.w, b1.x * vm01.y)));
-                  v.z += fmaf(b2.w, vm23.w, fmaf(b2.z, vm23.y, fmaf(b2.y, vm01.w, b2.x * vm01.y)));
-                  v.w += fmaf(b3.w, vm23.w, fmaf(b3.z, vm23.y, fmaf(b3.y, vm01.w, b3.x * vm01.y)));
+                  v.x += fmaf(b0.w, vm.w, fmaf(b0.z, vm.z, fmaf(b0.y, vm.y, b0.x * vm.x)));
+                  v.y += fmaf(b1.w, vm.w, fmaf(b1.z, vm.z, fmaf(b1.y, vm.y, b1.x * vm.x)));
+                  v.z += fmaf(b2.w, vm.w, fmaf(b2.z, vm.z, fmaf(b2.y, vm.y, b2.x * vm.x)));
+                  v.w += fmaf(b3.w, vm.w, fmaf(b3.z, vm.z, fmaf(b3.y, vm.y, b3.x * vm.x)));
                   a4[L] = v;
                 }
                 asm volatile("" ::: "memory");
                 if (s != 0) {
-                  const float4 vl01 = VG4[2 * L], vl23 = VG4[2 * L + 1];
+                  const float4 vl = gq[L];
                   float4 v = a4[M];
-                  v.x += fmaf(b3.x, vl23.w, fmaf(b2.x, vl23.y, fmaf(b1.x, vl01.w, b0.x * vl01.y)));
-                  v.y += fmaf(b3.y, vl23.w, fmaf(b2.y, vl23.y, fmaf(b1.y, vl01.w, b0.y * vl01.y)));
-                  v.z += fmaf(b3.z, vl23.w, fmaf(b2.z, vl23.y, fmaf(b1.z, vl01.w, b0.z * vl01.y)));
-                  v.w += fmaf(b3.w, vl23.w, fmaf(b2.w, vl23.y, fmaf(b1.w, vl01.w, b0.w * vl01.y)));
+                  v.x += fmaf(b3.x, vl.w, fmaf(b2.x, vl.z, fmaf(b1.x, vl.y, b0.x * vl.x)));
+                  v.y += fmaf(b3.y, vl.w, fmaf(b2.y, vl.z, fmaf(b1.y, vl.y, b0.y * vl.x)));
+                  v.z += fmaf(b3.z, vl.w, fmaf(b2.z, vl.z, fmaf(b1.z, vl.y, b0.z * vl.x)));
+                  v.w += fmaf(b3.w, vl.w, fmaf(b2.w, vl.z, fmaf(b1.w, vl.y, b0.w * vl.x)));
                   a4[M] = v;
                 }
                 asm volatile("" ::: "memory");
@@ -1346,13 +1352,12 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
 #pragma unroll
             for (int k = 0; k < NPM; k++) ds[k] = dh[k] = 0.0;
             for (int i = tid; i < n; i += NT) {
-              const double g = VG[i].y;
+              const double g = gv[i];
 #pragma unroll
               for (int k = 0; k < NPM; k++) {
                 if (k < npend) {
-                  const float2 u = sh_slot(k)[i];
-                  ds[k] += (double)u.x * g;
-                  dh[k] += (double)u.y * g;
+                  ds[k] += (double)up_plane(k, 0)[i] * g;
+                  dh[k] += (double)up_plane(k, 1)[i] * g;
                 }
               }
             }
@@ -1396,8 +1401,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
 #pragma unroll
                 for (int k = 0; k < NPM; k++)
                   if (k < npend) {
-                    const float2 ab = ab_slot(k)[t];
-                    y = fmaf(ab.y, fh[k], fmaf(ab.x, fs[k], y));
+                    y = fmaf(up_plane(k, 3)[t], fh[k], fmaf(up_plane(k, 2)[t], fs[k], y));
                   }
               }
               // H dg = H g_new - H g_old = H g_new + d_old
@@ -1447,7 +1451,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
             float lr[2][NPM];
 #pragma unroll
             for (int k = 0; k < NPM; k++) lr[0][k] = lr[1][k] = 0.f;
-            hquad_dispatch<HQ, NPM>(npend, base, nq, j0, j1, VG, S, cx, cy, a2, lr);
+            hquad_dispatch<HQ, NPM>(npend, base, nq, j0, j1, gv, S, cx, cy, a2, lr);
             // the pending updates' part of H g when they were not added element by element:
             // sum the dot products over the quad's lanes, then y_t += alpha_t (s.g) + beta_t (h.g)
             if (npend > 0 && npend < NPM) {
@@ -1485,14 +1489,14 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
         }
         double v6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         for (int i = tid; i < n; i += NT) {
-          const float2 v = VG[i];
+          const float g = gv[i], dg = dgv[i];
           const double xi = xo[i], h = hd[i];
-          v6[0] += (double)v.x * xi;
-          v6[1] += (double)v.x * h;
-          v6[2] += (double)v.x * v.x;
+          v6[0] += (double)dg * xi;
+          v6[1] += (double)dg * h;
+          v6[2] += (double)dg * dg;
           v6[3] += xi * xi;
-          v6[4] += xi * v.y;
-          v6[5] += h * v.y;
+          v6[4] += xi * g;
+          v6[5] += h * g;
         }
         R.template run<6, 0>(v6);
         const double fac = v6[0], fae = v6[1];
@@ -1503,14 +1507,20 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
           const double A = fi + fae * fi * fi, Bc = -fae * fi * fei, Cc = fae * fei * fei - fei;
           const double xig = v6[4], hdg = v6[5];
           // the new update goes behind the pending ones (slot 0 when H is kept updated)
-          float2* sh_new = sh_slot(LAZY ? npend : 0);
-          float2* ab_new = ab_slot(LAZY ? npend : 0);
+          const int slot = LAZY ? npend : 0;
           for (int t = tid; t < n; t += NT) {
             const double xi = xo[t], h = hd[t];
             const double al = A * xi + Bc * h, be = Bc * xi + Cc * h;
             d[t] = -(float)((double)d[t] + al * xig + be * hdg);
-            sh_new[t] = make_float2((float)xi, (float)h);
-            ab_new[t] = make_float2((float)al, (float)be);
+            if (SYM) {
+              up_plane(slot, 0)[t] = (float)xi;
+              up_plane(slot, 1)[t] = (float)h;
+              up_plane(slot, 2)[t] = (float)al;
+              up_plane(slot, 3)[t] = (float)be;
+            } else {
+              sh_slot(slot)[t] = make_float2((float)xi, (float)h);
+              ab_slot(slot)[t] = make_float2((float)al, (float)be);
+            }
           }
           npend++;
         } else {
@@ -1529,8 +1539,8 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
             const bool two = c2 != c1;
             const int l1 = (c1 + 4) >> 2, lb = l1 + (two ? (c2 + 4) >> 2 : 0);  // 4-row groups
             const int sb = (lb + lp - 1) >> lsh2, f0 = q * sb, f1 = min(lb, f0 + sb);
-            if (f0 < l1) hcol_update4(H + pcol(c1), AB, SH[c1], f0, min(f1, l1));
-            if (two && f1 > l1) hcol_update4(H + pcol(c2), AB, SH[c2], max(f0, l1) - l1, f1 - l1);
+            if (f0 < l1) hcol_update4(H + pcol(c1), ab_slot(0), sh_slot(0)[c1], f0, min(f1, l1));
+            if (two && f1 > l1) hcol_update4(H + pcol(c2), ab_slot(0), sh_slot(0)[c2], max(f0, l1) - l1, f1 - l1);
           }
           npend = 0;
           __syncthreads();
@@ -1538,19 +1548,19 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
       } else {
         // L-BFGS history and two-loop recursion (mmff_lbfgs_source_tg.metal:249-292)
         double ys = 0.0;
-        for (int i = tid; i < n; i += NT) ys += (double)VG[i].x * xo[i];
+        for (int i = tid; i < n; i += NT) ys += (double)dgv[i] * xo[i];
         ys = R.sum(ys);
         if (ys > 1e-10) {
           const int slot = hist_idx % M;
           for (int i = tid; i < n; i += NT) {
             S[(size_t)slot * mn + i] = xo[i];
-            Y[(size_t)slot * mn + i] = VG[i].x;
+            Y[(size_t)slot * mn + i] = dgv[i];
           }
           if (tid == 0) rho[slot] = 1.0 / ys;
           hist_idx++;
           if (hist_count < M) hist_count++;
         }
-        for (int i = tid; i < n; i += NT) hd[i] = VG[i].y;
+        for (int i = tid; i < n; i += NT) hd[i] = gv[i];
         __syncthreads();  // rho visible
         // The two-loop recursion with each axpy fused into the next dot product's pass (and
         // gamma's dots into the first pass, the gamma scaling into the last axpy of the first
