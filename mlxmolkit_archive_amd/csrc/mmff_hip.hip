@@ -137,19 +137,21 @@ __device__ __forceinline__ float from_fx(unsigned long long a) {
   return (float)((double)(long long)a * FX_UNIT);
 }
 
-// The accumulators of a conformer with N atoms are three planes of N words (x, y, z), so
-// lanes updating consecutive atoms touch consecutive 8-byte words (no bank conflicts); the
-// gradient of coordinate i = 3a + c is plane c, word a. The -g side of a pair term is an LDS
-// subtract (ds_sub_u64) of the same integer, so it needs no negation.
+// The accumulator of coordinate i = 3a + c is word i. Lanes updating consecutive atoms touch
+// 8-byte words 24 bytes apart, and 3 is coprime to the 32 double banks, so they meet no bank
+// twice; the three components are immediate offsets of one address (with three planes of N words
+// each component took an address addition of its own, 6 of a pair's 95 vector instructions). The
+// -g side of a pair term is an LDS subtract (ds_sub_u64) of the same integer, so it needs no
+// negation.
 template <bool G>
 struct LdsAcc {
   unsigned long long* g;
-  int N;
   __device__ __forceinline__ void add(int a, float x, float y, float z) {
     if (G) {
-      atomicAdd(&g[a], to_fx(x));
-      atomicAdd(&g[N + a], to_fx(y));
-      atomicAdd(&g[2 * N + a], to_fx(z));
+      unsigned long long* p = g + 3 * a;
+      atomicAdd(&p[0], to_fx(x));
+      atomicAdd(&p[1], to_fx(y));
+      atomicAdd(&p[2], to_fx(z));
     }
   }
   __device__ __forceinline__ static void sub(unsigned long long* p, unsigned long long v) {
@@ -159,21 +161,16 @@ struct LdsAcc {
   __device__ __forceinline__ void add_pair(int a, int b, float x, float y, float z) {
     if (G) {
       const unsigned long long fx = to_fx(x), fy = to_fx(y), fz = to_fx(z);
-      atomicAdd(&g[a], fx);
-      atomicAdd(&g[N + a], fy);
-      atomicAdd(&g[2 * N + a], fz);
-      sub(&g[b], fx);
-      sub(&g[N + b], fy);
-      sub(&g[2 * N + b], fz);
+      unsigned long long *p = g + 3 * a, *q = g + 3 * b;
+      atomicAdd(&p[0], fx);
+      atomicAdd(&p[1], fy);
+      atomicAdd(&p[2], fz);
+      sub(&q[0], fx);
+      sub(&q[1], fy);
+      sub(&q[2], fz);
     }
   }
 };
-
-// gradient of coordinate i (= 3a + c) from the accumulator planes of an N-atom conformer
-__device__ __forceinline__ float gread(const unsigned long long* g, int i, int N) {
-  const int a = i / 3;
-  return from_fx(g[(i - 3 * a) * N + a]);
-}
 
 // ------------------------------------------------------------------------------------
 // energy (+ gradient) of one conformer whose positions are in LDS, spread over NT lanes.
@@ -340,7 +337,7 @@ __device__ __forceinline__ TermData load_term(const TView& V, int t, int c1, int
 template <int FAM, bool G, bool PT, int NT, bool PREF = true>
 __device__ __forceinline__ double eval_terms(const TView& TV, const MolDesc& m, const float* xs,
                                              unsigned long long* gacc, int diel, uint32_t mask, double* et) {
-  LdsAcc<G> acc{gacc, m.n_atoms};
+  LdsAcc<G> acc{gacc};
   double e = 0.0;
   // bonded terms (one generic loop, next term prefetched when PREF)
   const int c1 = m.nb, c2 = c1 + m.na, c3 = c2 + m.nsb, c4 = c3 + m.noop, c5 = c4 + m.ntor;
@@ -741,7 +738,7 @@ __global__ void __launch_bounds__(NT) k_energy_grad(KBatch B, const float* __res
   }
   if (threadIdx.x == 0) e_out[c] = e;
   if (g_out)
-    for (int i = threadIdx.x; i < n; i += NT) g_out[off + i] = gread(gacc, i, m.n_atoms);
+    for (int i = threadIdx.x; i < n; i += NT) g_out[off + i] = from_fx(gacc[i]);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1010,7 +1007,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
     float gscale = GRAD_SCALE_INIT;
     {
       double mxg = 0.0;
-      for (int i = tid; i < n; i += NT) mxg = fmax(mxg, (double)fabsf(gread(gacc, i, m.n_atoms) * gscale));
+      for (int i = tid; i < n; i += NT) mxg = fmax(mxg, (double)fabsf(from_fx(gacc[i]) * gscale));
       mxg = R.max(mxg);
       while (mxg > GRAD_CAP) {
         gscale *= 0.5f;
@@ -1018,7 +1015,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
       }
       for (int i = tid; i < n; i += NT) {
         dgv[i] = 0.f;
-        gv[i] = gread(gacc, i, m.n_atoms) * gscale;
+        gv[i] = from_fx(gacc[i]) * gscale;
       }
     }
     psc = GRAD_SCALE_INIT / gscale;
@@ -1159,7 +1156,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
       n_grads++;
       double v2[2] = {0.0, 0.0};
       for (int i = tid; i < n; i += NT) {
-        const float sg = fabsf(gread(gacc, i, m.n_atoms) * gscale);
+        const float sg = fabsf(from_fx(gacc[i]) * gscale);
         v2[0] = fmax(v2[0], (double)sg);
         v2[1] = fmax(v2[1], (double)sg * fmax((double)fabsf(xs[i]), 1.0));
       }
@@ -1170,7 +1167,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
         v2[1] *= 0.5;
       }
       for (int i = tid; i < n; i += NT) {
-        const float gn = gread(gacc, i, m.n_atoms) * gscale;
+        const float gn = from_fx(gacc[i]) * gscale;
         dgv[i] = gn - gv[i];
         gv[i] = gn;
       }
@@ -1687,7 +1684,7 @@ __global__ void __launch_bounds__(NT) k_bb_fused(KBatch B, const float* __restri
       E = E_prev;
       continue;
     }
-    for (int i = tid; i < n; i += NT) g[i] = gread(gacc, i, m.n_atoms);
+    for (int i = tid; i < n; i += NT) g[i] = from_fx(gacc[i]);
     if (it > 0) {  // BB step :1041-1052
       double v2[2] = {0.0, 0.0};
       for (int i = tid; i < n; i += NT) {
@@ -1770,7 +1767,7 @@ __global__ void __launch_bounds__(NT) k_mm_init(KBatch B, MMState S, const float
   mm_eval<NT>(B, m, xs, gacc, R, E, n);
   for (int i = threadIdx.x; i < n; i += NT) {
     S.x[off + i] = xs[i];
-    S.g[off + i] = gread(gacc, i, m.n_atoms) * gsc;
+    S.g[off + i] = from_fx(gacc[i]) * gsc;
     if (mode == 0) S.bx[off + i] = xs[i];
   }
   if (threadIdx.x == 0) {
@@ -1899,7 +1896,7 @@ __global__ void __launch_bounds__(NT) k_mm_chunk(KBatch B, MMState S, int steps,
     }
     double sy = 0.0;
     for (int i = tid; i < n; i += NT) {
-      const float gn = gread(gacc, i, m.n_atoms) * gsc;
+      const float gn = from_fx(gacc[i]) * gsc;
       const float s = xn[i] - xs[i], y = gn - gs[i];
       S.S[sl * T + off + i] = s;
       S.Y[sl * T + off + i] = y;
