@@ -334,7 +334,8 @@ __device__ __forceinline__ TermData load_term(const TView& V, int t, int c1, int
 
 // PREF: load each bonded term's tables one step ahead (tables in global memory); with the
 // tables in LDS the loads are short and the prefetch only holds registers.
-template <int FAM, bool G, bool PT, int NT, bool PREF = true>
+// EV: the energies are used (otherwise only the gradient is).
+template <int FAM, bool G, bool PT, int NT, bool PREF = true, bool EV = true>
 __device__ __forceinline__ double eval_terms(const TView& TV, const MolDesc& m, const float* xs,
                                              unsigned long long* gacc, int diel, uint32_t mask, double* et) {
   LdsAcc<G> acc{gacc};
@@ -390,44 +391,46 @@ __device__ __forceinline__ double eval_terms(const TView& TV, const MolDesc& m, 
   // non-bonded pairs: two pairs per lane per step (independent dependency chains), the
   // next two loaded while the current two are computed. The loads are unconditional (index
   // clamped to the last pair; such duplicates are never used), so the wait before the
-  // current pairs' use leaves the next pairs' loads in flight.
+  // current pairs' use leaves the next pairs' loads in flight. Every step but the last is full
+  // for all lanes, so the loop counts in scalar registers and masks nothing.
   if ((mask & 96u) && m.npair > 0) {
     const float ke = (mask & 32u) ? 1.0f : 0.0f, kq = (mask & 64u) ? 1.0f : 0.0f;
-    const int np = m.npair, last = np - 1;
-    int u = threadIdx.x;
-    uint32_t ija = TV.pair_ij[min(u, last)], ijb = TV.pair_ij[min(u + NT, last)];
-    float4 pa = TV.pair_p[min(u, last)], pb = TV.pair_p[min(u + NT, last)];
+    const unsigned np = (unsigned)m.npair, last = np - 1;
+    struct Pair {
+      uint32_t ij;
+      float eps, qq, ir;
+    };
+    // 32-bit offsets from the (uniform) table bases
+    auto load = [&](unsigned u) {
+      u = min(u, last);
+      const float* q = (const float*)((const char*)TV.pair_p + 16u * u);
+      return Pair{*(const uint32_t*)((const char*)TV.pair_ij + 4u * u), q[1], q[2], q[3]};
+    };
     double ev_acc = 0.0, ee_acc = 0.0;
-    while (u < np) {
-      const int un = u + 2 * NT;
-      const uint32_t nija = TV.pair_ij[min(un, last)], nijb = TV.pair_ij[min(un + NT, last)];
-      const float4 npa = TV.pair_p[min(un, last)], npb = TV.pair_p[min(un + NT, last)];
-      float eva, eea;
-      t_pair<FAM, G>(xs, acc, (int)(ija & 0xffff), (int)(ija >> 16), pa.w, ke * pa.y, kq * pa.z, diel, eva, eea);
+    auto term = [&](const Pair& p) {
+      float ev = 0.f, ee = 0.f;
+      t_pair<FAM, G, EV>(xs, acc, (int)(p.ij & 0xffff), (int)(p.ij >> 16), p.ir, ke * p.eps, kq * p.qq, diel, ev, ee);
       // without per-term energies a pair's two parts are added in FP32 first (one rounding,
       // as small as the parts' own), then to the lane's FP64 sum
       if (PT) {
-        ev_acc += eva;
-        ee_acc += eea;
+        ev_acc += ev;
+        ee_acc += ee;
       } else {
-        ev_acc += (double)(eva + eea);
+        ev_acc += (double)(ev + ee);
       }
-      if (u + NT < np) {
-        float evb, eeb;
-        t_pair<FAM, G>(xs, acc, (int)(ijb & 0xffff), (int)(ijb >> 16), pb.w, ke * pb.y, kq * pb.z, diel, evb, eeb);
-        if (PT) {
-          ev_acc += evb;
-          ee_acc += eeb;
-        } else {
-          ev_acc += (double)(evb + eeb);
-        }
-      }
-      ija = nija;
-      ijb = nijb;
-      pa = npa;
-      pb = npb;
-      u = un;
+    };
+    unsigned u = threadIdx.x;
+    Pair pa = load(u), pb = load(u + NT);
+    for (unsigned left = (np - 1) / (2 * NT); left > 0; left--) {
+      const Pair na = load(u + 2 * NT), nb = load(u + 3 * NT);
+      term(pa);
+      term(pb);
+      pa = na;
+      pb = nb;
+      u += 2 * NT;
     }
+    if (u < np) term(pa);
+    if (u + NT < np) term(pb);
     e += ev_acc + ee_acc;
     if (PT) {
       et[5] += ev_acc;
@@ -1150,7 +1153,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
       if (!have_grad) {
         for (int i = tid; i < n; i += NT) gacc[i] = 0ull;
         __syncthreads();
-        eval_terms<FAM_TG, true, false, NT, TL == 0>(TV, m, xs, gacc, P.diel, 0x7fu, nullptr);
+        eval_terms<FAM_TG, true, false, NT, TL == 0, false>(TV, m, xs, gacc, P.diel, 0x7fu, nullptr);
         __syncthreads();
       }
       n_grads++;

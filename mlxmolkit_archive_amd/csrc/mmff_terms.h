@@ -332,36 +332,42 @@ __device__ __forceinline__ float t_torsion(const float* x, Acc& acc, int i1, int
 // eps = 0 / qqs = 0 switch a half off. diel = 1 (constant) or 2 (distance dependent, TG only).
 // Returns vdW energy in ev and ele energy in ee.
 // iR = 1 / R* (1 / max(R*, 1e-8) for the TG family), precomputed in the pair table.
-template <int FAM, bool G, class Acc>
+// The TG form writes its fused multiply-adds out, so that its rounding does not follow what the
+// compiler finds around it. EV says that the energies are used: the gradient alone keeps the
+// vdW part's last product unrounded, the two together the electrostatic part's.
+template <int FAM, bool G, bool EV, class Acc>
 __device__ __forceinline__ void t_pair(const float* x, Acc& acc, int i, int j, float iR, float eps, float qqs,
                                        int diel, float& ev, float& ee) {
   f3 d = ld(x, i) - ld(x, j);
-  float d2 = dot(d, d);
   if (FAM == FAM_TG) {
+    const float d2 = fmaf(d.z, d.z, fmaf(d.x, d.x, d.y * d.y));
     // four reciprocal-type operations per pair: 1/r (r = d2 / r), 1/(q + 0.07),
     // 1/(q^7 + 0.12) and 1/(r + 0.05), each shared by the energy and the gradient
     const float d2c = fmaxf(d2, 1e-16f);
     const float ir = rsqrtf(d2c);
     const float r = d2c * ir;
     const float q = r * iR;
-    const float q2 = q * q, q6 = q2 * q2 * q2, q7 = q6 * q;
-    const float rq = rcp(q + 0.07f);
+    const float q2 = q * q, q6 = q2 * q2 * q2;
+    const float rq = rcp(fmaf(r, iR, 0.07f));
     const float t = 1.07f * rq;
     const float t2 = t * t, t7 = t2 * t2 * t2 * t;
-    const float r7 = rcp(q7 + 0.12f);  // q >= 0: q7 + 0.12 >= 0.12
-    ev = eps * t7 * (1.12f * r7 - 2.0f);
-    const float dpd = r + 0.05f;
-    const float rd = rcp(dpd);  // dpd >= 0.05
+    const float r7 = rcp(fmaf(q6, q, 0.12f));  // q >= 0: q7 + 0.12 >= 0.12
+    const float rd = rcp(fmaf(d2c, ir, 0.05f));  // r + 0.05 >= 0.05
     const float qe = 332.0716f * qqs;
-    ee = diel == 2 ? qe * rd * rd : qe * rd;
+    if (EV) {
+      ev = eps * t7 * fmaf(1.12f, r7, -2.0f);
+      ee = (diel == 2 ? qe * rd : qe) * rd;
+    }
     if (G) {
       const float inv = r > 1e-8f ? ir : 0.0f;
-      const float dv = eps * iR * t7 * (-7.84f * q6 * r7 * r7 + (-7.84f * r7 + 14.0f) * rq);
-      const float de = diel == 2 ? -2.0f * qe * rd * rd * rd : -qe * rd * rd;
-      const float f = (dv + de) * inv;
+      const float c = eps * iR * t7, h = fmaf(fmaf(-7.84f, r7, 14.0f), rq, -7.84f * q6 * r7 * r7);
+      const float qd = diel == 2 ? (2.0f * qe) * rd : qe;
+      const float dd = EV ? fmaf(-qd * rd, rd, c * h) : fmaf(c, h, -(qd * rd * rd));
+      const float f = dd * inv;
       acc.add_pair(i, j, f * d.x, f * d.y, f * d.z);
     }
   } else {
+    const float d2 = dot(d, d);
     // shared reciprocals: 1/(rho + 0.07), 1/(rho^7 + 0.12), 1/(r + 0.05), 1/r
     const float r = sqrtf(d2) + M_KEPS;
     const float rho = r * iR;
