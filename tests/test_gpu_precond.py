@@ -56,6 +56,32 @@ def test_mlp_forward_backward_match_oracle():
     assert np.max(np.abs(gg - gr)) <= 1e-4 * np.max(np.abs(gr))
 
 
+@pytest.mark.parametrize("n", [1, 15, 64, 65, 130, 16385])
+def test_mlp_training_tiles_match_oracle(n):
+    """Partial, whole and several 64-atom tiles, and more tiles than workgroups (16,385 atoms).
+    Tolerances: a hidden unit is an FP32 sum of at most 105 products, relative error below
+    105 * 2^-24 = 6.3e-6 of its terms' size, and a gradient goes through five such sums, so
+    1e-4 of the largest entry covers them; without weights and without the gradient the loss
+    and blocks are the same bits."""
+    m = _model(7)
+    m.params[-(6 * 64 + 6):] = torch.from_numpy(np.random.default_rng(8).normal(0, 0.3, 6 * 64 + 6).astype(np.float32)).cuda()
+    f = _feat(n, 100 + n)
+    g = np.random.default_rng(n)
+    t = g.normal(0, 0.5, (n, 9)).astype(np.float32)
+    w = g.uniform(0.5, 2.0, n).astype(np.float32)
+    fd, td, wd = (torch.from_numpy(a).cuda() for a in (f, t, w))
+    loss, grad, blocks = m.loss_grad(fd, td, wd)
+    loss2, none, blocks2 = m.loss_grad(fd, td, None, want_grad=False)
+    torch.cuda.synchronize()
+    p = m.params.cpu().numpy().astype(np.float64)
+    Pr, _ = mo.forward(p, f)
+    _, per, gr = mo.loss_grad(p, f, t, w)
+    np.testing.assert_allclose(blocks.cpu().numpy(), Pr, rtol=1e-4, atol=1e-5)
+    np.testing.assert_allclose(loss.cpu().numpy(), per, rtol=1e-4, atol=1e-5)
+    assert np.max(np.abs(grad.cpu().numpy() - gr)) <= 1e-4 * np.max(np.abs(gr))
+    assert none is None and torch.equal(loss, loss2) and torch.equal(blocks, blocks2)
+
+
 def test_mlp_bf16_mfma_inference_matches_fp32():
     """BF16 operands, FP32 accumulation: blocks within bf16 rounding of the FP64 network;
     77 atoms exercise a partial 32-atom tile."""
