@@ -60,110 +60,174 @@ struct MlpW {
 };
 
 // ------------------------------------------------------------------------------------
-// inference on MFMA. LDS: W1 bf16 [64][112], W2 bf16 [64][64], W3 bf16 [32][64] (rows 6..31
-// zero), plus per wave an activation tile bf16 [32][112] and an output tile f32 [32][8].
+// Inference on MFMA, bound by reading the features (416 bytes per atom). A wave takes 32 atoms
+// at a time; the next tile's features (13 x 16 bytes per lane) are loaded into registers while
+// this one is computed. The products are formed transposed (A = weights, B = activations), so a
+// lane ends up with four consecutive units of one atom per register quad: one packed conversion
+// per two values and one 8-byte LDS write per four, where units in lanes took a rounding sequence
+// and a 2-byte write each. The first layer's weights stay in registers, the others in LDS. Row
+// strides of 58 and 34 words put the 32 rows of an 8-byte operand read in 32 different bank pairs.
 // v_mfma_f32_32x32x8_bf16 operand layout (wave64): lane l supplies A[l%32][4*(l/32)+0..3]
 // and B[4*(l/32)+0..3][l%32]; it receives D[8*(r/4) + 4*(l/32) + r%4][l%32], r = 0..15.
+// 500,003 atoms: 69 us (3.3 TB/s of features and blocks); 326 us with 4-byte feature loads and
+// units in lanes, 134 us with 16-byte loads and units in lanes.
 constexpr int INF_WAVES = 4;
-constexpr int INF_TILE_SHORTS = 32 * MLP_KPAD + 32 * 64 + 32 * 8 * 2;  // act, act2, out (f32)
-constexpr size_t INF_LDS = (size_t)(64 * MLP_KPAD + 64 * 64 + 32 * 64) * 2 + (size_t)INF_WAVES * INF_TILE_SHORTS * 2;
+constexpr int INF_LDX = 116, INF_LDH = 68;  // row strides (bf16) of features and hidden units
+constexpr int INF_WAVE_SHORTS = 32 * INF_LDX + 32 * INF_LDH + 2 * 32 * 9;  // features, hidden, blocks (f32)
+constexpr int INF_W23_SHORTS = 64 * INF_LDH + 32 * INF_LDH + 2 * 160;      // W2, W3, biases (f32)
+// W1 is staged where the waves' tiles go afterwards
+static_assert(64 * INF_LDX <= INF_WAVES * INF_WAVE_SHORTS, "staging area");
+constexpr size_t INF_LDS = 2 * (size_t)(INF_W23_SHORTS + INF_WAVES * INF_WAVE_SHORTS);
+constexpr int INF_GRID = 512;  // two workgroups per CU (registers), each taking tiles in turn
+static_assert(INF_LDS <= 65536, "no raised LDS limit needed");
+constexpr int INF_VEC = 32 * MLP_IN / 4 / 64;  // 16-byte feature loads per lane and tile (13)
 
-__device__ __forceinline__ bf16x4 ld4(const short* p) {
-  bf16x4 v;
-  v.x = p[0];
-  v.y = p[1];
-  v.z = p[2];
-  v.w = p[3];
-  return v;
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
-// D (32 x 32 block at column offset n0 of an [out][in] weight matrix Wt) += A (32 x K) * Wt^T
-template <int K>
-__device__ __forceinline__ f32x16 mfma_tile(const short* act, int act_ld, const short* wt, int w_ld, int n0, int lane) {
+// two floats as bf16, round to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+  const bf2 v = {(__bf16)a, (__bf16)b};
+  return __builtin_bit_cast(uint32_t, v);
+}
+
+// D[unit][atom] (32 x 32) = W (32 rows x 8 KS) times the transpose of the activations (rows of act)
+template <int KS, class WOP>
+__device__ __forceinline__ f32x16 mfma_tile(const WOP& w, const short* act, int act_ld, int lane) {
   f32x16 acc = {0.f};
-  const int r = lane & 31, kg = (lane >> 5) * 4;
+  const short* p = act + (lane & 31) * act_ld + (lane >> 5) * 4;
 #pragma unroll
-  for (int k = 0; k < K; k += 8) {
-    const bf16x4 a = ld4(act + r * act_ld + k + kg);
-    const bf16x4 b = ld4(wt + (n0 + r) * w_ld + k + kg);
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc, 0, 0, 0);
-  }
+  for (int k = 0; k < KS; k++)
+    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(w(k), *(const bf16x4*)(p + 8 * k), acc, 0, 0, 0);
   return acc;
 }
 
-// bias + ReLU, then store the 32 x 32 tile as bf16 activations at columns n0.. of act
-__device__ __forceinline__ void store_relu(f32x16 acc, const float* bias, int n0, short* act, int act_ld, int lane) {
-  const int col = lane & 31, rb = (lane >> 5) * 4;
+// bias + ReLU, then store the tile as bf16 activations at units n0.. of the atoms' rows of hid
+__device__ __forceinline__ void store_relu(const f32x16& acc, const float* bias, int n0, short* hid, int lane) {
+  short* row = hid + (lane & 31) * INF_LDH + n0 + 4 * (lane >> 5);
 #pragma unroll
-  for (int q = 0; q < 16; q++) {
-    const int row = 8 * (q >> 2) + rb + (q & 3);
-    act[row * act_ld + n0 + col] = to_bf16(fmaxf(acc[q] + bias[n0 + col], 0.f));
+  for (int q = 0; q < 4; q++) {
+    const float4 b = *(const float4*)(bias + n0 + 8 * q + 4 * (lane >> 5));
+    uint2 v;
+    v.x = pack_bf16(fmaxf(acc[4 * q] + b.x, 0.f), fmaxf(acc[4 * q + 1] + b.y, 0.f));
+    v.y = pack_bf16(fmaxf(acc[4 * q + 2] + b.z, 0.f), fmaxf(acc[4 * q + 3] + b.w, 0.f));
+    *(uint2*)(row + 8 * q) = v;
   }
 }
 
-__global__ void __launch_bounds__(64 * INF_WAVES) k_mlp_infer_bf16(MlpW W, const float* __restrict__ feat, int n_atoms,
-                                                                   float* __restrict__ blocks) {
+// VEC: the features are 16-byte aligned (rows are 26 x 16 bytes), so a tile is read in 16-byte
+// words; otherwise in 4-byte ones
+template <bool VEC>
+__global__ void __launch_bounds__(64 * INF_WAVES, 2)
+    k_mlp_infer_bf16(MlpW W, const float* __restrict__ feat, int n_atoms, float* __restrict__ blocks) {
   extern __shared__ __align__(16) unsigned char smem[];
-  short* w1 = (short*)smem;
-  short* w2 = w1 + 64 * MLP_KPAD;
-  short* w3 = w2 + 64 * 64;
-  short* tiles = w3 + 32 * 64;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  for (int i = tid; i < 64 * MLP_KPAD; i += blockDim.x) {
-    const int o = i / MLP_KPAD, k = i % MLP_KPAD;
-    w1[i] = to_bf16(k < MLP_IN ? W.w1[o * MLP_IN + k] : 0.f);
-  }
-  for (int i = tid; i < 64 * 64; i += blockDim.x) w2[i] = to_bf16(W.w2[i]);
-  for (int i = tid; i < 32 * 64; i += blockDim.x) w3[i] = to_bf16(i < MLP_OUT * 64 ? W.w3[i] : 0.f);
-  __syncthreads();
-  short* act = tiles + wv * INF_TILE_SHORTS;  // bf16 [32][112], later [32][64]
-  short* act2 = act + 32 * MLP_KPAD;            // bf16 [32][64]
-  float* outt = (float*)(act2 + 32 * 64);       // f32 [32][8]
-  const int n_tiles = (n_atoms + 31) / 32;
-  for (int t = blockIdx.x * INF_WAVES + wv; t < n_tiles; t += gridDim.x * INF_WAVES) {
-    const int a0 = t * 32;
-    // features of 32 atoms -> bf16 tile (rows past n_atoms are zero)
-    for (int i = lane; i < 32 * MLP_KPAD; i += 64) {
-      const int r = i / MLP_KPAD, k = i % MLP_KPAD;
-      const int a = a0 + r;
-      act[i] = to_bf16(a < n_atoms && k < MLP_IN ? feat[(size_t)a * MLP_IN + k] : 0.f);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c32 = lane & 31;
+  short* s2 = (short*)smem;                  // W2 [64][INF_LDH]
+  short* s3 = s2 + 64 * INF_LDH;             // W3 [32][INF_LDH], rows 6..31 zero
+  float* bias = (float*)(s3 + 32 * INF_LDH); // b1, b2, b3 padded to 32
+  short* tiles = (short*)(bias + 160);
+  bf16x4 w1a[MLP_KPAD / 8], w1b[MLP_KPAD / 8];
+  {
+    short* s1 = tiles;
+    for (int i = tid; i < 64 * MLP_KPAD; i += blockDim.x) {
+      const int o = i / MLP_KPAD, k = i % MLP_KPAD;
+      s1[o * INF_LDX + k] = to_bf16(k < MLP_IN ? W.w1[o * MLP_IN + k] : 0.f);
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    // layer 1: [32 x 112] x W1^T -> [32 x 64]
-    f32x16 h0 = mfma_tile<MLP_KPAD>(act, MLP_KPAD, w1, MLP_KPAD, 0, lane);
-    f32x16 h1 = mfma_tile<MLP_KPAD>(act, MLP_KPAD, w1, MLP_KPAD, 32, lane);
-    __builtin_amdgcn_wave_barrier();
-    store_relu(h0, W.b1, 0, act, 64, lane);  // reuse the tile as [32][64]
-    store_relu(h1, W.b1, 32, act, 64, lane);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    // layer 2: [32 x 64] x W2^T -> [32 x 64]
-    h0 = mfma_tile<64>(act, 64, w2, 64, 0, lane);
-    h1 = mfma_tile<64>(act, 64, w2, 64, 32, lane);
-    store_relu(h0, W.b2, 0, act2, 64, lane);
-    store_relu(h1, W.b2, 32, act2, 64, lane);
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    // layer 3: [32 x 64] x W3^T -> [32 x 32], columns 0..5 used
-    const f32x16 o = mfma_tile<64>(act2, 64, w3, 64, 0, lane);
-    {
-      const int col = lane & 31, rb = (lane >> 5) * 4;
-      if (col < MLP_OUT) {
+    for (int i = tid; i < 64 * 64; i += blockDim.x) s2[(i >> 6) * INF_LDH + (i & 63)] = to_bf16(W.w2[i]);
+    for (int i = tid; i < 32 * 64; i += blockDim.x)
+      s3[(i >> 6) * INF_LDH + (i & 63)] = to_bf16(i < MLP_OUT * 64 ? W.w3[i] : 0.f);
+    if (tid < 160) bias[tid] = tid < 64 ? W.b1[tid] : tid < 128 ? W.b2[tid - 64] : tid < 128 + MLP_OUT ? W.b3[tid - 128] : 0.f;
+    __syncthreads();
+    const short* p = s1 + c32 * INF_LDX + (lane >> 5) * 4;
 #pragma unroll
-        for (int q = 0; q < 16; q++) outt[(8 * (q >> 2) + rb + (q & 3)) * 8 + col] = o[q] + W.b3[col];
+    for (int k = 0; k < MLP_KPAD / 8; k++) {
+      w1a[k] = *(const bf16x4*)(p + 8 * k);
+      w1b[k] = *(const bf16x4*)(p + 32 * INF_LDX + 8 * k);
+    }
+    __syncthreads();  // the tiles below reuse the LDS
+  }
+  auto op1a = [&](int k) { return w1a[k]; };
+  auto op1b = [&](int k) { return w1b[k]; };
+  const short* p2 = s2 + c32 * INF_LDH + (lane >> 5) * 4;
+  auto op2a = [&](int k) { return *(const bf16x4*)(p2 + 8 * k); };
+  auto op2b = [&](int k) { return *(const bf16x4*)(p2 + 32 * INF_LDH + 8 * k); };
+  const short* p3 = s3 + c32 * INF_LDH + (lane >> 5) * 4;
+  auto op3 = [&](int k) { return *(const bf16x4*)(p3 + 8 * k); };
+  short* act = tiles + wv * INF_WAVE_SHORTS;  // bf16 [32][INF_LDX]
+  short* hid = act + 32 * INF_LDX;            // bf16 [32][INF_LDH]
+  float* blk = (float*)(hid + 32 * INF_LDH);  // outputs [32][8], then blocks [32][9]
+  for (int i = lane; i < 32 * (MLP_KPAD - MLP_IN); i += 64)
+    act[(i >> 3) * INF_LDX + MLP_IN + (i & 7)] = 0;  // the padding columns of the first layer
+  const int n_tiles = (n_atoms + 31) / 32, step = gridDim.x * INF_WAVES;
+  int t = blockIdx.x * INF_WAVES + wv;
+  float4 f[INF_VEC];
+  auto fetch = [&](int tile) {
+    const size_t left = ((size_t)n_atoms - (size_t)tile * 32) * (MLP_IN / 4);  // 16-byte words to the end
+    const float4* src = (const float4*)feat + (size_t)tile * (32 * MLP_IN / 4);
+#pragma unroll
+    for (int v = 0; v < INF_VEC; v++) {
+      const int i = v * 64 + lane;
+      if (VEC) {
+        f[v] = (size_t)i < left ? src[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+      } else {
+        const float* p = (const float*)src + 4 * i;
+        f[v] = (size_t)i < left ? make_float4(p[0], p[1], p[2], p[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
       }
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    if (lane < 32 && a0 + lane < n_atoms) {
-      float blk[9];
-      chol_block(outt + lane * 8, blk);
-      float* dst = blocks + (size_t)(a0 + lane) * 9;
+  };
+  if (t < n_tiles) fetch(t);
+  for (; t < n_tiles; t += step) {
+    const int a0 = t * 32;
+    // features of 32 atoms -> bf16 tile (rows past n_atoms are zero)
 #pragma unroll
-      for (int q = 0; q < 9; q++) dst[q] = blk[q];
+    for (int v = 0; v < INF_VEC; v++) {
+      const int i = v * 64 + lane, r = i / (MLP_IN / 4), k = 4 * (i - r * (MLP_IN / 4));
+      uint2 b;
+      b.x = pack_bf16(f[v].x, f[v].y);
+      b.y = pack_bf16(f[v].z, f[v].w);
+      *(uint2*)(act + r * INF_LDX + k) = b;
     }
-    __builtin_amdgcn_wave_barrier();
+    if (t + step < n_tiles) fetch(t + step);
+    wave_lds_fence();
+    // layer 1: [32 x 112] x W1^T -> [32 x 64]
+    f32x16 h0 = mfma_tile<MLP_KPAD / 8>(op1a, act, INF_LDX, lane), h1 = mfma_tile<MLP_KPAD / 8>(op1b, act, INF_LDX, lane);
+    store_relu(h0, bias, 0, hid, lane);
+    store_relu(h1, bias, 32, hid, lane);
+    wave_lds_fence();
+    // layer 2: [32 x 64] x W2^T -> [32 x 64], over the same rows once both products have read them
+    h0 = mfma_tile<8>(op2a, hid, INF_LDH, lane);
+    h1 = mfma_tile<8>(op2b, hid, INF_LDH, lane);
+    wave_lds_fence();
+    store_relu(h0, bias + 64, 0, hid, lane);
+    store_relu(h1, bias + 64, 32, hid, lane);
+    wave_lds_fence();
+    // layer 3: [32 x 64] x W3^T -> [32 x 32], units 0..5 used: 0-3 in the lower half's first
+    // quad, 4 and 5 in the upper half's
+    const f32x16 o = mfma_tile<8>(op3, hid, INF_LDH, lane);
+    if (lane < 32)
+      *(float4*)(blk + c32 * 8) = make_float4(o[0] + bias[128], o[1] + bias[129], o[2] + bias[130], o[3] + bias[131]);
+    else
+      *(float2*)(blk + c32 * 8 + 4) = make_float2(o[0] + bias[132], o[1] + bias[133]);
+    wave_lds_fence();
+    float b[9];
+    if (lane < 32) chol_block(blk + lane * 8, b);
+    wave_lds_fence();
+    if (lane < 32) {
+#pragma unroll
+      for (int q = 0; q < 9; q++) blk[lane * 9 + q] = b[q];
+    }
+    wave_lds_fence();
+    const int n_out = 9 * min(32, n_atoms - a0);
+    float* dst = blocks + (size_t)a0 * 9;
+#pragma unroll
+    for (int v = 0; v < 5; v++) {
+      const int i = v * 64 + lane;
+      if (i < n_out) dst[i] = blk[i];
+    }
+    wave_lds_fence();
   }
 }
 
@@ -452,14 +516,15 @@ int mmffhip_mlp_infer(const float* params, const float* feat, int32_t n_atoms, f
   if (n_atoms == 0) return MMFFHIP_OK;
   if (!params || !feat || !blocks) return perr(MMFFHIP_ERR_ARG, "params, feat and blocks are required");
   const MlpW W = mlp_weights(params);
-  const int tiles = (n_atoms + 31) / 32;
-  const int grid = (tiles + INF_WAVES - 1) / INF_WAVES < 1024 ? (tiles + INF_WAVES - 1) / INF_WAVES : 1024;
-  if (INF_LDS > 65536 &&
-      hipFuncSetAttribute((const void*)&k_mlp_infer_bf16, hipFuncAttributeMaxDynamicSharedMemorySize, (int)INF_LDS) !=
-          hipSuccess)
-    return perr(MMFFHIP_ERR_HIP, "hipFuncSetAttribute failed");
-  hipLaunchKernelGGL(k_mlp_infer_bf16, dim3(grid), dim3(64 * INF_WAVES), INF_LDS, (hipStream_t)stream, W, feat,
-                     n_atoms, blocks);
+  const int tiles = (n_atoms + 31) / 32, need = (tiles + INF_WAVES - 1) / INF_WAVES;
+  const int grid = need < INF_GRID ? need : INF_GRID;
+  const bool vec = ((uintptr_t)feat & 15) == 0;
+  if (vec)
+    hipLaunchKernelGGL(k_mlp_infer_bf16<true>, dim3(grid), dim3(64 * INF_WAVES), INF_LDS, (hipStream_t)stream, W, feat,
+                       n_atoms, blocks);
+  else
+    hipLaunchKernelGGL(k_mlp_infer_bf16<false>, dim3(grid), dim3(64 * INF_WAVES), INF_LDS, (hipStream_t)stream, W, feat,
+                       n_atoms, blocks);
   return hipGetLastError() == hipSuccess ? MMFFHIP_OK : perr(MMFFHIP_ERR_HIP, "launch failed");
 }
 

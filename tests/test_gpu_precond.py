@@ -96,6 +96,25 @@ def test_mlp_bf16_mfma_inference_matches_fp32():
         assert np.median(err) < 1e-2 and err.max() < 5e-2, (n, np.median(err), err.max())
 
 
+@pytest.mark.parametrize("n", [1, 31, 33, 65541])
+def test_mlp_inference_tiles_and_alignment(n):
+    """Partial tiles and more tiles than waves (65,541 atoms), with the features on a 16-byte
+    boundary and one float past it: the same blocks, within bf16 rounding (2^-9 per operand; the
+    bounds of the test above) of the FP64 network."""
+    m = _model(9)
+    m.params[-(6 * 64 + 6):] = torch.from_numpy(np.random.default_rng(6).normal(0, 0.2, 6 * 64 + 6).astype(np.float32)).cuda()
+    f = _feat(n, 50 + n)
+    fd = torch.from_numpy(f).cuda()
+    off = torch.empty(n * mo.N_IN + 1, dtype=torch.float32, device="cuda")[1:].view(n, mo.N_IN)
+    off.copy_(fd)
+    b, b_off = m.blocks(fd), m.blocks(off)
+    torch.cuda.synchronize()
+    assert fd.data_ptr() % 16 == 0 and off.data_ptr() % 16 == 4 and torch.equal(b, b_off)
+    Pr, _ = mo.forward(m.params.cpu().numpy().astype(np.float64), f)
+    err = np.abs(b.cpu().numpy() - Pr).max(axis=1) / np.abs(Pr).max(axis=1)
+    assert np.median(err) < 1e-2 and err.max() < 5e-2, (n, np.median(err), err.max())
+
+
 def test_hessian_blocks_match_oracle_finite_differences(small_wl):
     from mlxmolkit_archive_amd import engine
     from mlxmolkit_archive_amd.precond import hessian_diag_blocks
