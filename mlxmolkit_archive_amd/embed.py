@@ -151,10 +151,17 @@ def embed_device(params_list: Sequence, z_list: Sequence[np.ndarray], conf_count
     out = torch.empty(total, dtype=torch.float32, device=device)
     if len(conf_mol) == 0:
         return out
+    # longest first: a conformer's cost grows with the square of its atoms, and the last ones to
+    # start decide when the launch ends (each conformer writes at its own offset, so results are
+    # the same)
+    by_size = np.argsort(-n_atoms, kind="stable")
+    first = np.cumsum(counts) - counts
+    k = counts[by_size]
+    order = np.arange(len(conf_mol)) + np.repeat(first[by_size] - (np.cumsum(k) - k), k)
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(device)  # noqa: E731
     bufs = [t(desc.reshape(-1)), t(ij.view(np.int32) if len(ij) else np.zeros(1, np.int32)),
-            t(dd if len(dd) else np.zeros(1, np.float32)), t(conf_mol), t(off.astype(np.int32)),
-            t(sd.view(np.int64))]
+            t(dd if len(dd) else np.zeros(1, np.float32)), t(conf_mol[order]), t(off[order].astype(np.int32)),
+            t(sd[order].view(np.int64))]
     _lib.check(L.mmffhip_embed(*(int(b.data_ptr()) for b in bufs), len(conf_mol), int(n_atoms.max()), float(noise),
                                int(out.data_ptr()), _lib.stream_ptr(stream)))
     # the staging tensors must outlive the asynchronous launch

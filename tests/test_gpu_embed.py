@@ -99,3 +99,34 @@ def test_device_embedder_noise_and_minimization():
     print(f"\nBFGS from device starts: status0 {np.mean(st == 0):.3f}, mean iterations "
           f"{res.counters.cpu().numpy()[:, 0].mean():.1f}, energy range {e.min():.1f}..{e.max():.1f}")
     assert np.mean(st == 0) >= 0.95 and np.isfinite(e).all()
+
+
+def _chain(n):
+    """Restraint table of an n-atom zigzag: 1-2 and 1-3 springs, walls between atoms 3 to 9 apart."""
+    i, j, d = [], [], []
+    for k in range(n):
+        for s in range(1, 10):
+            if k + s < n:
+                i.append(k), j.append(k + s), d.append(1.5 if s == 1 else 2.5 if s == 2 else -3.0)
+    ij = np.array(i, np.uint32) | (np.array(j, np.uint32) << 16)
+    return ij.astype(np.uint32), np.array(d, np.float32)
+
+
+@pytest.mark.parametrize("n", [1, 2, 20, 65, 131])
+def test_embedding_does_not_depend_on_the_batch(n):
+    """A molecule alone, and beside one so large that its coordinates leave no LDS for the waves'
+    queues of active restraints: the same geometry. The two kernels add the same energies in
+    another order, so they take the same steps unless two energies agree to rounding; 1e-5 A
+    allows one float rounding of a coordinate (2^-23 of at most 40 A). Up to 1,279 atoms fit."""
+    from types import SimpleNamespace
+    from mlxmolkit_archive_amd.embed import embed_device
+    big = 1279
+    tabs = [_chain(n), _chain(big)]
+    ps = [SimpleNamespace(n_atoms=n), SimpleNamespace(n_atoms=big)]
+    seeds = np.array([5, 6, 7], np.uint64)
+    alone = embed_device(ps[:1], [None], [2], seeds=seeds[:2], noise=0.1, tables=tabs[:1]).cpu().numpy()
+    both = embed_device(ps, [None] * 2, [2, 1], seeds=seeds, noise=0.1, tables=tabs).cpu().numpy()
+    assert alone.shape == (6 * n,) and np.isfinite(both).all()
+    assert np.abs(alone - both[:6 * n]).max() <= 1e-5
+    with pytest.raises(RuntimeError, match="too large"):
+        embed_device([SimpleNamespace(n_atoms=big + 1)], [None], [1], seeds=seeds[:1], tables=[_chain(n)])
