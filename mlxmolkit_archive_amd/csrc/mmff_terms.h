@@ -305,9 +305,20 @@ __device__ __forceinline__ float t_torsion(const float* x, Acc& acc, int i1, int
     float n1n2 = sqrtf(dot(c1, c1) * dot(c2, c2) + M_KEPS);
     float sw = dot(mv, c2) / n1n2, cw = dot(c1, c2) / n1n2;
     float om = atan2f(sw, cw);
-    float e = 0.5f * (V1 * (1.0f + cosf(om)) + V2 * (1.0f - cosf(2.0f * om)) + V3 * (1.0f + cosf(3.0f * om)));
+    // one argument reduction per angle serves its sine and cosine (the same values as sinf, cosf)
+    float s1, c1o, s2, c2o, s3, c3o;
     if (G) {
-      float dE = 0.5f * (-V1 * sinf(om) + 2.0f * V2 * sinf(2.0f * om) - 3.0f * V3 * sinf(3.0f * om));
+      sincosf(om, &s1, &c1o);
+      sincosf(2.0f * om, &s2, &c2o);
+      sincosf(3.0f * om, &s3, &c3o);
+    } else {
+      c1o = cosf(om);
+      c2o = cosf(2.0f * om);
+      c3o = cosf(3.0f * om);
+    }
+    float e = 0.5f * (V1 * (1.0f + c1o) + V2 * (1.0f - c2o) + V3 * (1.0f + c3o));
+    if (G) {
+      float dE = 0.5f * (-V1 * s1 + 2.0f * V2 * s2 - 3.0f * V3 * s3);
       f3 rij = p1 - p2, rkj = p3 - p2, rkl = p3 - p4;
       f3 m = cross(rij, rkj), n = cross(rkj, rkl);
       float msq = dot(m, m) + M_KEPS, nsq = dot(n, n) + M_KEPS;
