@@ -333,6 +333,61 @@ __device__ __forceinline__ TermData load_term(const TView& V, int t, int c1, int
   return d;
 }
 
+// non-bonded pairs: two pairs per lane per step (independent dependency chains), the
+// next two loaded while the current two are computed. The loads are unconditional (index
+// clamped to the last pair; such duplicates are never used), so the wait before the
+// current pairs' use leaves the next pairs' loads in flight. Every step but the last is full
+// for all lanes, so the loop counts in scalar registers and masks nothing.
+template <int FAM, bool G, bool PT, int NT, bool EV>
+__device__ __forceinline__ double eval_pairs(const TView& TV, const MolDesc& m, const float* xs, LdsAcc<G>& acc,
+                                             int diel, uint32_t mask, double* et) {
+  if ((mask & 96u) && m.npair > 0) {
+    const float ke = (mask & 32u) ? 1.0f : 0.0f, kq = (mask & 64u) ? 1.0f : 0.0f;
+    const unsigned np = (unsigned)m.npair, last = np - 1;
+    struct Pair {
+      uint32_t ij;
+      float eps, qq, ir;
+    };
+    // 32-bit offsets from the (uniform) table bases
+    auto load = [&](unsigned u) {
+      u = min(u, last);
+      const float* q = (const float*)((const char*)TV.pair_p + 16u * u);
+      return Pair{*(const uint32_t*)((const char*)TV.pair_ij + 4u * u), q[1], q[2], q[3]};
+    };
+    double ev_acc = 0.0, ee_acc = 0.0;
+    auto term = [&](const Pair& p) {
+      float ev = 0.f, ee = 0.f;
+      t_pair<FAM, G, EV>(xs, acc, (int)(p.ij & 0xffff), (int)(p.ij >> 16), p.ir, ke * p.eps, kq * p.qq, diel, ev, ee);
+      // without per-term energies a pair's two parts are added in FP32 first (one rounding,
+      // as small as the parts' own), then to the lane's FP64 sum
+      if (PT) {
+        ev_acc += ev;
+        ee_acc += ee;
+      } else {
+        ev_acc += (double)(ev + ee);
+      }
+    };
+    unsigned u = threadIdx.x;
+    Pair pa = load(u), pb = load(u + NT);
+    for (unsigned left = (np - 1) / (2 * NT); left > 0; left--) {
+      const Pair na = load(u + 2 * NT), nb = load(u + 3 * NT);
+      term(pa);
+      term(pb);
+      pa = na;
+      pb = nb;
+      u += 2 * NT;
+    }
+    if (u < np) term(pa);
+    if (u + NT < np) term(pb);
+    if (PT) {
+      et[5] += ev_acc;
+      et[6] += ee_acc;
+    }
+    return ev_acc + ee_acc;
+  }
+  return 0.0;
+}
+
 // PREF: load each bonded term's tables one step ahead (tables in global memory); with the
 // tables in LDS the loads are short and the prefetch only holds registers.
 // EV: the energies are used (otherwise only the gradient is).
@@ -389,56 +444,75 @@ __device__ __forceinline__ double eval_terms(const TView& TV, const MolDesc& m, 
     if (PREF) cur = nxt;
     t = tn;
   }
-  // non-bonded pairs: two pairs per lane per step (independent dependency chains), the
-  // next two loaded while the current two are computed. The loads are unconditional (index
-  // clamped to the last pair; such duplicates are never used), so the wait before the
-  // current pairs' use leaves the next pairs' loads in flight. Every step but the last is full
-  // for all lanes, so the loop counts in scalar registers and masks nothing.
-  if ((mask & 96u) && m.npair > 0) {
-    const float ke = (mask & 32u) ? 1.0f : 0.0f, kq = (mask & 64u) ? 1.0f : 0.0f;
-    const unsigned np = (unsigned)m.npair, last = np - 1;
-    struct Pair {
-      uint32_t ij;
-      float eps, qq, ir;
+  e += eval_pairs<FAM, G, PT, NT, EV>(TV, m, xs, acc, diel, mask, et);
+  return e;
+}
+
+// eval_terms for kernels whose results do not hang on the order of the energy sum (single points;
+// the descents, where the energy only guards): the bonded terms go to the waves in tasks of 64
+// terms of one type, the heaviest types first and the waves taken back and forth, so no wave runs
+// several types' code for parts of its lanes and the waves finish together. The minimizers that
+// compare energies trial by trial keep eval_terms' fixed order. With the generic bonded loop,
+// which also held the next term's parameters in registers (83 now against 103 for the MEGA
+// kernel): 12,139 ragged MEGA energies and gradients 143 -> 123 us, 2,500 TG energies with terms
+// 14.9 -> 13.0 us, the Barzilai-Borwein descent of 1,000 conformers 6.08 -> 4.65 ms.
+template <int FAM, bool G, bool PT, int NT>
+__device__ __forceinline__ double eval_tasks(const TView& V, const MolDesc& m, const float* xs,
+                                             unsigned long long* gacc, int diel, uint32_t mask, double* et) {
+  constexpr int NW = NT / 64;
+  LdsAcc<G> acc{gacc};
+  double e = 0.0;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // first task of each type after the torsions
+  const int t1 = (m.ntor + 63) >> 6, t2 = t1 + ((m.nsb + 63) >> 6), t3 = t2 + ((m.na + 63) >> 6),
+            t4 = t3 + ((m.noop + 63) >> 6), t5 = t4 + ((m.nb + 63) >> 6);
+  for (int k = 0; k * NW < t5; k++) {
+    const int t = (k & 1) ? (k + 1) * NW - 1 - w : k * NW + w;
+    auto add = [&](int kind, float v) {
+      e += v;
+      if (PT) et[kind] += v;
     };
-    // 32-bit offsets from the (uniform) table bases
-    auto load = [&](unsigned u) {
-      u = min(u, last);
-      const float* q = (const float*)((const char*)TV.pair_p + 16u * u);
-      return Pair{*(const uint32_t*)((const char*)TV.pair_ij + 4u * u), q[1], q[2], q[3]};
-    };
-    double ev_acc = 0.0, ee_acc = 0.0;
-    auto term = [&](const Pair& p) {
-      float ev = 0.f, ee = 0.f;
-      t_pair<FAM, G, EV>(xs, acc, (int)(p.ij & 0xffff), (int)(p.ij >> 16), p.ir, ke * p.eps, kq * p.qq, diel, ev, ee);
-      // without per-term energies a pair's two parts are added in FP32 first (one rounding,
-      // as small as the parts' own), then to the lane's FP64 sum
-      if (PT) {
-        ev_acc += ev;
-        ee_acc += ee;
-      } else {
-        ev_acc += (double)(ev + ee);
+    if (t < t1) {
+      const int u = t * 64 + lane;
+      if ((mask & 16u) && u < m.ntor) {
+        const uint2 ix = V.tor_idx[u];
+        const float4 p = V.tor_p[u];
+        add(4, t_torsion<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
+                                 (int)(ix.y >> 16), p.x, p.y, p.z));
       }
-    };
-    unsigned u = threadIdx.x;
-    Pair pa = load(u), pb = load(u + NT);
-    for (unsigned left = (np - 1) / (2 * NT); left > 0; left--) {
-      const Pair na = load(u + 2 * NT), nb = load(u + 3 * NT);
-      term(pa);
-      term(pb);
-      pa = na;
-      pb = nb;
-      u += 2 * NT;
-    }
-    if (u < np) term(pa);
-    if (u + NT < np) term(pb);
-    e += ev_acc + ee_acc;
-    if (PT) {
-      et[5] += ev_acc;
-      et[6] += ee_acc;
+    } else if (t < t2) {
+      const int u = (t - t1) * 64 + lane;
+      if ((mask & 4u) && u < m.nsb) {
+        const uint2 ix = V.sb_idx[u];
+        const float4 p = V.sb_p[u];
+        add(2, t_strbend<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)ix.y, p.x, p.y, p.z, p.w,
+                                 V.sb_t0[u]));
+      }
+    } else if (t < t3) {
+      const int u = (t - t2) * 64 + lane;
+      if ((mask & 2u) && u < m.na) {
+        const uint2 ix = V.ang_idx[u];
+        const float2 p = V.ang_p[u];
+        add(1, t_angle<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff), p.x, p.y,
+                               (ix.y >> 16) != 0));
+      }
+    } else if (t < t4) {
+      const int u = (t - t3) * 64 + lane;
+      if ((mask & 8u) && u < m.noop) {
+        const uint2 ix = V.oop_idx[u];
+        add(3, t_oop<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
+                             (int)(ix.y >> 16), V.oop_k[u]));
+      }
+    } else if (t < t5) {
+      const int u = (t - t4) * 64 + lane;
+      if ((mask & 1u) && u < m.nb) {
+        const uint32_t ij = V.bond_ij[u];
+        const float2 p = V.bond_p[u];
+        add(0, t_bond<FAM, G>(xs, acc, (int)(ij & 0xffff), (int)(ij >> 16), p.x, p.y));
+      }
     }
   }
-  return e;
+  return e + eval_pairs<FAM, G, PT, NT, true>(V, m, xs, acc, diel, mask, et);
 }
 
 // ------------------------------------------------------------------------------------
@@ -585,9 +659,9 @@ __global__ void __launch_bounds__(NT) k_energy_grad(KBatch B, const float* __res
   double et[7] = {0, 0, 0, 0, 0, 0, 0};
   double e;
   if (g_out)
-    e = eval_terms<FAM, true, true, NT>(global_view(B, m), m, xs, gacc, diel, mask, et);
+    e = eval_tasks<FAM, true, true, NT>(global_view(B, m), m, xs, gacc, diel, mask, et);
   else
-    e = eval_terms<FAM, false, true, NT>(global_view(B, m), m, xs, gacc, diel, mask, et);
+    e = eval_tasks<FAM, false, true, NT>(global_view(B, m), m, xs, gacc, diel, mask, et);
   e = R.sum(e);  // includes the barrier that completes the gradient atomics
   if (e_terms) {
     double v4[4] = {et[0], et[1], et[2], et[3]};
@@ -1540,7 +1614,7 @@ __global__ void __launch_bounds__(NT) k_bb_fused(KBatch B, const float* __restri
   for (int it = 0; it < max_it; it++) {
     for (int i = tid; i < n; i += NT) gacc[i] = 0ull;
     __syncthreads();
-    E = R.sum(eval_terms<FAM_MEGA, true, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu, nullptr));
+    E = R.sum(eval_tasks<FAM_MEGA, true, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu, nullptr));
     if (it > 0 && E > E_prev + 1.0) {  // energy guard :1031-1038
       for (int i = tid; i < n; i += NT) xs[i] = pp[i];
       alpha = fmaxf(alpha * 0.5f, 1e-7f);
@@ -1606,7 +1680,7 @@ __device__ void mm_eval(const KBatch& B, const MolDesc& m, float* xs, unsigned l
                         double& E, int n) {
   for (int i = threadIdx.x; i < n; i += NT) gacc[i] = 0ull;
   __syncthreads();
-  E = R.sum(eval_terms<FAM_MEGA, true, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu, nullptr));
+  E = R.sum(eval_tasks<FAM_MEGA, true, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu, nullptr));
 }
 
 // mode 0: initial (x = x_in), mode 1: polish restart (x = best_x); both compute E+G, scale g,
@@ -1645,32 +1719,70 @@ __global__ void __launch_bounds__(NT) k_mm_init(KBatch B, MMState S, const float
   }
 }
 
-template <int NT>
-__global__ void __launch_bounds__(NT) k_mm_chunk(KBatch B, MMState S, int steps, int it_end, int do_sync,
-                                                 int phase, const int32_t* prev_flag, int32_t* my_flag, int M,
-                                                 float max_step, float gsc, float tol) {
+// K dot products over a conformer's n coordinates: f(i, p) adds coordinate i's products to p
+template <int NT, int K, class F>
+__device__ __forceinline__ void block_dots(Reducer<NT>& R, int n, double (&p)[K], F f) {
+#pragma unroll
+  for (int k = 0; k < K; k++) p[k] = 0.0;
+  for (int i = threadIdx.x; i < n; i += NT) f(i, p);
+  R.template run<K, 0>(p);
+}
+
+// LDS of k_mm_chunk: reduction buffer, gradient accumulators, x, g, q, x_new and alpha, and the
+// (s, y, rho) history when hl
+size_t mm_lds(int mx, int m, bool hl) {
+  return 16 * 4 * 8 + (size_t)mx * (8 + 16) + 8 * (size_t)m + (hl ? 8 * (size_t)m * (mx + 1) : 0) + 32;
+}
+
+// HL: the (s, y) history is worked on in LDS for the launch's iterations (and written through to
+// the workspace, which the next launch reads); from memory, each of an iteration's 2 len + 1
+// dependent passes waited for its loads. Each lane meets only its own coordinates of it, so it
+// needs no barrier. 128 registers put four workgroups on a CU. 1,000 conformers of 69 atoms on
+// average, 200 + 50 iterations: 7.4 ms; 9.1 ms with three workgroups per CU, 10.5 ms with the
+// history in memory too. Measured and dropped: the recursion in one wave while the others wait
+// (the same sums without barriers: 7.6 ms, and 3.53 against 2.75 ms for 60 conformers), and one
+// 64-thread workgroup per conformer (12.1 ms).
+template <bool HL>
+__global__ void __launch_bounds__(256, 4) k_mm_chunk(KBatch B, MMState S, int steps, int it_end, int do_sync,
+                                                     int phase, const int32_t* prev_flag, int32_t* my_flag, int M,
+                                                     float max_step, float gsc, float tol) {
   extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int NW = NT / 64;
+  constexpr int NT = 256, NW = NT / 64;
   const int c = blockIdx.x;
   if (c >= B.n_confs) return;
   if (prev_flag && *prev_flag == 0) return;  // every conformer converged at the last sync
   const int tid = threadIdx.x;
   const int mx = 3 * B.max_atoms;
   double* red = (double*)smem;
-  unsigned long long* gacc = (unsigned long long*)(red + 16 * NW);
+  double* alf = red + 16 * NW;  // [M]
+  double* lrho = alf + M;       // [M] when HL
+  unsigned long long* gacc = (unsigned long long*)(HL ? lrho + M : lrho);
   float* xs = (float*)(gacc + mx);
   float* gs = xs + mx;
   float* q = gs + mx;
   float* xn = q + mx;
-  double* alf = (double*)(xn + mx);  // [M]
   const MolDesc m = load_desc(B.mol_desc + 16 * B.conf_mol[c]);
   const int n = 3 * m.n_atoms, off = B.conf_off[c];
-  const size_t T = S.total;
+  const size_t T = S.total, HT = HL ? (size_t)mx : T;
+  float* gS = S.S + off;
+  float* gY = S.Y + off;
+  float* hS = HL ? xn + mx : gS;  // slot h's coordinate i at [h * HT + i]
+  float* hY = HL ? hS + (size_t)M * mx : gY;
+  int len = S.ring[2 * c], head = S.ring[2 * c + 1];
   for (int i = tid; i < n; i += NT) {
     xs[i] = S.x[off + i];
     gs[i] = S.g[off + i];
   }
-  int len = S.ring[2 * c], head = S.ring[2 * c + 1];
+  auto rho = [&](int k) { return HL ? lrho[k] : S.rho[(size_t)k * B.n_confs + c]; };
+  if (HL) {
+    // the ring fills slots 0 .. len - 1 first
+    for (int k = tid; k < len; k += NT) lrho[k] = S.rho[(size_t)k * B.n_confs + c];
+    for (int k = 0; k < len; k++)
+      for (int i = tid; i < n; i += NT) {
+        hS[k * HT + i] = gS[k * T + i];
+        hY[k * HT + i] = gY[k * T + i];
+      }
+  }
   Reducer<NT> R{red, 0};
   double E = S.e_new[c];
   __syncthreads();
@@ -1679,62 +1791,61 @@ __global__ void __launch_bounds__(NT) k_mm_chunk(KBatch B, MMState S, int steps,
     // axpy fused into the next dot product's pass, gamma's dots into the first pass and the
     // gamma scaling into the first loop's last axpy: the same FP32 updates of q and FP64 dot
     // products as running the passes one by one (bit-identical), in 2 len + 1 passes.
-    for (int i = tid; i < n; i += NT) q[i] = gs[i];
     if (len > 0) {
-      int sl = (head + len - 1) % M;  // newest entry
-      double v3[3] = {0.0, 0.0, 0.0};
-      for (int i = tid; i < n; i += NT) {
-        const double s = S.S[sl * T + off + i], y = S.Y[sl * T + off + i];
-        v3[0] += s * q[i];
-        v3[1] += s * y;
-        v3[2] += y * y;
-      }
-      R.template run<3, 0>(v3);
+      int sl = head + len - 1;  // newest entry
+      if (sl >= M) sl -= M;
+      double v3[3];
+      block_dots<NT, 3>(R, n, v3, [&](int i, double (&p)[3]) {
+        const float qv = gs[i];
+        q[i] = qv;
+        const double s = hS[sl * HT + i], y = hY[sl * HT + i];
+        p[0] += s * qv;
+        p[1] += s * y;
+        p[2] += y * y;
+      });
       const float gf = (float)(v3[1] / (v3[2] + 1e-30));
-      double a = S.rho[(size_t)sl * B.n_confs + c] * v3[0];
+      double a = rho(sl) * v3[0];
       if (tid == 0) alf[len - 1] = a;
       for (int h = len - 1; h >= 1; h--) {  // q -= alpha_h y_h, then s_{h-1}.q
-        const int sn = (head + h - 1) % M;
+        const int sn = sl == 0 ? M - 1 : sl - 1;
         const float af = (float)a;
-        double sq = 0.0;
-        for (int i = tid; i < n; i += NT) {
-          const float qv = q[i] - af * S.Y[sl * T + off + i];
+        double sq[1];
+        block_dots<NT, 1>(R, n, sq, [&](int i, double (&p)[1]) {
+          const float qv = q[i] - af * hY[sl * HT + i];
           q[i] = qv;
-          sq += (double)S.S[sn * T + off + i] * qv;
-        }
-        sq = R.sum(sq);
-        a = S.rho[(size_t)sn * B.n_confs + c] * sq;
+          p[0] += (double)hS[sn * HT + i] * qv;
+        });
+        a = rho(sn) * sq[0];
         if (tid == 0) alf[h - 1] = a;
         sl = sn;
       }
-      double yr = 0.0;  // q -= alpha_0 y_0, q *= gamma, then y_0.q
+      double yr[1];  // q -= alpha_0 y_0, q *= gamma, then y_0.q
       {
         const float af = (float)a;
-        for (int i = tid; i < n; i += NT) {
-          const float y = S.Y[sl * T + off + i];
+        block_dots<NT, 1>(R, n, yr, [&](int i, double (&p)[1]) {
+          const float y = hY[sl * HT + i];
           float qv = q[i] - af * y;
           qv *= gf;
           q[i] = qv;
-          yr += (double)y * qv;
-        }
+          p[0] += (double)y * qv;
+        });  // its barrier also makes alf visible
       }
-      yr = R.sum(yr);  // its barrier also makes alf visible
       for (int h = 0; h < len; h++) {  // q += (alpha_h - beta_h) s_h, then y_{h+1}.q
-        const float cf = (float)(alf[h] - S.rho[(size_t)sl * B.n_confs + c] * yr);
-        const int sn = (head + h + 1) % M;
+        const float cf = (float)(alf[h] - rho(sl) * yr[0]);
+        const int sn = sl + 1 == M ? 0 : sl + 1;
         if (h + 1 < len) {
-          double y2 = 0.0;
-          for (int i = tid; i < n; i += NT) {
-            const float r = q[i] + cf * S.S[sl * T + off + i];
+          block_dots<NT, 1>(R, n, yr, [&](int i, double (&p)[1]) {
+            const float r = q[i] + cf * hS[sl * HT + i];
             q[i] = r;
-            y2 += (double)S.Y[sn * T + off + i] * r;
-          }
-          yr = R.sum(y2);
+            p[0] += (double)hY[sn * HT + i] * r;
+          });
         } else {
-          for (int i = tid; i < n; i += NT) q[i] += cf * S.S[sl * T + off + i];
+          for (int i = tid; i < n; i += NT) q[i] += cf * hS[sl * HT + i];
         }
         sl = sn;
       }
+    } else {
+      for (int i = tid; i < n; i += NT) q[i] = gs[i];
     }
     __syncthreads();
     // d = -q with the per-atom cap of max_step (:365-373); x_new = x + d
@@ -1752,23 +1863,30 @@ __global__ void __launch_bounds__(NT) k_mm_chunk(KBatch B, MMState S, int steps,
     int sl;
     if (len >= M) {
       sl = head;
-      head = (head + 1) % M;
+      head = head + 1 == M ? 0 : head + 1;
     } else {
-      sl = (head + len) % M;
+      sl = head + len >= M ? head + len - M : head + len;
       len++;
     }
-    double sy = 0.0;
-    for (int i = tid; i < n; i += NT) {
+    double sy[1];
+    block_dots<NT, 1>(R, n, sy, [&](int i, double (&p)[1]) {
       const float gn = from_fx(gacc[i]) * gsc;
       const float s = xn[i] - xs[i], y = gn - gs[i];
-      S.S[sl * T + off + i] = s;
-      S.Y[sl * T + off + i] = y;
-      sy += (double)s * y;
+      hS[sl * HT + i] = s;
+      hY[sl * HT + i] = y;
+      if (HL) {
+        gS[sl * T + i] = s;
+        gY[sl * T + i] = y;
+      }
+      p[0] += (double)s * y;
       xs[i] = xn[i];
       gs[i] = gn;
+    });
+    if (tid == 0) {
+      const double r = sy[0] > 1e-10 ? 1.0 / (sy[0] + 1e-30) : 0.0;
+      if (HL) lrho[sl] = r;
+      S.rho[(size_t)sl * B.n_confs + c] = r;
     }
-    sy = R.sum(sy);
-    if (tid == 0) S.rho[(size_t)sl * B.n_confs + c] = sy > 1e-10 ? 1.0 / (sy + 1e-30) : 0.0;
     __syncthreads();
   }
   if (do_sync) {
@@ -1826,7 +1944,7 @@ __global__ void __launch_bounds__(NT) k_mm_final(KBatch B, MMState S, float* x_b
   for (int i = threadIdx.x; i < n; i += NT) xs[i] = S.bx[off + i];
   __syncthreads();
   Reducer<NT> R{red, 0};
-  double E = R.sum(eval_terms<FAM_MEGA, false, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu, nullptr));
+  double E = R.sum(eval_tasks<FAM_MEGA, false, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu, nullptr));
   double gmax = 0.0;
   if (l2_norm) {
     for (int i = threadIdx.x; i < n; i += NT) gmax += (double)S.g[off + i] * S.g[off + i];
@@ -1912,6 +2030,18 @@ int launch_eg(const KBatch& kb, const float* x, double* e, double* et, float* g,
   hipLaunchKernelGGL((k_energy_grad<FAM, 256>), dim3(kb.n_confs), dim3(256), lds, s, kb, x, e, et, g, mask, diel);
   HIP_TRY(hipGetLastError());
   return MMFFHIP_OK;
+}
+
+// The launch of k_mm_chunk: with the history in LDS when that leaves three workgroups per CU, or
+// when there is at most one per CU anyway.
+struct MMChunk {
+  void (*kernel)(KBatch, MMState, int, int, int, int, const int32_t*, int32_t*, int, float, float, float);
+  size_t lds;
+};
+MMChunk mm_chunk_plan(int n_confs, int mx, int m, const DevInfo& di) {
+  const size_t hl = mm_lds(mx, m, true);
+  if (hl <= (size_t)di.lds / 3 || (n_confs <= di.n_cu && hl <= (size_t)di.lds)) return {k_mm_chunk<true>, hl};
+  return {k_mm_chunk<false>, mm_lds(mx, m, false)};
 }
 
 int round4(int v) { return (v + 3) & ~3; }
@@ -2328,11 +2458,11 @@ int mmffhip_multimol_run_ex(const mmffhip_batch* b, const float* x_in, float* x_
   constexpr int NT = 256;
   const int mx = 3 * b->max_atoms;
   const size_t lds_init = 16 * (NT / 64) * 8 + (size_t)mx * (8 + 4) + 16;
-  const size_t lds_chunk = 16 * (NT / 64) * 8 + (size_t)mx * (8 + 16) + 8 * (size_t)lbfgs_m + 32;
-  if ((int)lds_chunk > dev_info().lds) return fail(MMFFHIP_ERR_SIZE, "molecule too large for one workgroup");
-  const int nfl = n_main + n_pol;
+  const DevInfo di = dev_info();
+  const MMChunk ck = mm_chunk_plan(b->n_confs, mx, lbfgs_m, di);
+  if (ck.lds > (size_t)di.lds) return fail(MMFFHIP_ERR_SIZE, "molecule too large for one workgroup");
   allow_lds((const void*)&k_mm_init<NT>, lds_init);
-  allow_lds((const void*)&k_mm_chunk<NT>, lds_chunk);
+  allow_lds((const void*)ck.kernel, ck.lds);
   allow_lds((const void*)&k_mm_final<NT>, lds_init);
   hipLaunchKernelGGL(k_fill_i32, dim3((4096 + 255) / 256), dim3(256), 0, s, S.flags, 4096, 0);
   hipLaunchKernelGGL((k_mm_init<NT>), dim3(b->n_confs), dim3(NT), lds_init, s, kb, S, x_in, grad_scale, 0,
@@ -2345,7 +2475,7 @@ int mmffhip_multimol_run_ex(const mmffhip_batch* b, const float* x_in, float* x_
     const bool sync = (it % eval_freq) == 0;
     // the batch form has no convergence exit: no conformer ever passes the test (tolerance
     // -1) and no launch reads the previous sync point's count
-    hipLaunchKernelGGL((k_mm_chunk<NT>), dim3(b->n_confs), dim3(NT), lds_chunk, s, kb, S, steps, it, sync ? 1 : 0,
+    hipLaunchKernelGGL(ck.kernel, dim3(b->n_confs), dim3(NT), ck.lds, s, kb, S, steps, it, sync ? 1 : 0,
                        0, (k > 0 && !batch) ? S.flags + (k - 1) : (const int32_t*)nullptr, S.flags + k,
                        (int)lbfgs_m, max_step_per_atom, grad_scale, batch ? -1.0f : grad_tol);
     if (sync) k++;
@@ -2360,13 +2490,12 @@ int mmffhip_multimol_run_ex(const mmffhip_batch* b, const float* x_in, float* x_
     int steps = std::min(eval_freq, polish - it);
     it += steps;
     const bool sync = (it % eval_freq) == 0;
-    hipLaunchKernelGGL((k_mm_chunk<NT>), dim3(b->n_confs), dim3(NT), lds_chunk, s, kb, S, steps, it, sync ? 1 : 0,
+    hipLaunchKernelGGL(ck.kernel, dim3(b->n_confs), dim3(NT), ck.lds, s, kb, S, steps, it, sync ? 1 : 0,
                        1, kp > n_main ? S.flags + (kp - 1) : (const int32_t*)nullptr, S.flags + kp, (int)lbfgs_m,
                        max_step_per_atom, grad_scale, grad_tol);
     if (sync) kp++;
   }
   HIP_TRY(hipGetLastError());
-  (void)nfl;
   hipLaunchKernelGGL((k_mm_final<NT>), dim3(b->n_confs), dim3(NT), lds_init, s, kb, S, x_best, e_final, grad_norm,
                      per_conf_iters, converged, iters_used, batch ? 0 : (int)(max_iters / eval_freq),
                      (int)eval_freq, (int)max_iters, batch ? 1 : 0);

@@ -207,7 +207,10 @@ __device__ __forceinline__ float t_oop(const float* x, Acc& acc, int i, int j, i
     float iK = rsqrtf(fmaxf(dot(v, v), 1e-16f));
     float iL = rsqrtf(fmaxf(dot(w, w), 1e-16f));
     f3 dI = iI * u, dK = iK * v, dL = iL * w;
-    f3 n = cross(-dI, dK);
+    // without the gradient the rounded product of each component is written out; with it the
+    // normal is the gradient's t3, and the compiler forms the two alike
+    f3 n = G ? cross(-dI, dK)
+             : mk(fmaf(-dK.z, dI.y, dK.y * dI.z), fmaf(-dK.x, dI.z, dK.z * dI.x), fmaf(-dK.y, dI.x, dK.x * dI.y));
     float inl = rsqrtf(fmaxf(dot(n, n), 1e-16f));
     n = inl * n;
     float sc = clampf(dot(dL, n), -1.0f, 1.0f);

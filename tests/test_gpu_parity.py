@@ -363,3 +363,21 @@ def test_autotuned_buckets_cover_batch_and_agree(medium_wl):
     ea, eb = a.energy.cpu().numpy(), b.energy.cpu().numpy()
     assert np.median(np.abs(ea - eb)) < 1e-3
     assert (a.status.cpu().numpy() == 0).mean() >= 0.9
+
+
+@pytest.mark.parametrize("fill", [1, 300])
+def test_multimol_history_placement_does_not_change_results(fill):
+    """The lock-step engine keeps its (s, y) history in LDS for small batches and small molecules
+    and in memory beside a large molecule (``fill`` conformers of a chain): the same iterates,
+    bit for bit, of a small molecule's conformers (no convergence exit: grad_tol 0)."""
+    from mlxmolkit_archive_amd import engine, workloads
+    small = workloads.build("small", n_mols=2, n_confs=3)
+    chain = workloads.build("chain", n_mols=1, n_confs=1)
+    x = np.concatenate([small.x, np.tile(chain.x, fill)])
+    kw = dict(max_iters=25, grad_tol=0.0)
+    alone = engine.multimol(engine.device_batch(small.params, small.conf_counts), torch.from_numpy(small.x).cuda(), **kw)
+    both = engine.multimol(engine.device_batch(small.params + chain.params, small.conf_counts + [fill]),
+                           torch.from_numpy(x).cuda(), **kw)
+    torch.cuda.synchronize()
+    assert torch.equal(alone["x"], both["x"][:len(small.x)])
+    assert torch.equal(alone["energy"], both["energy"][:6]) and torch.equal(alone["grad_norm"], both["grad_norm"][:6])
