@@ -1207,59 +1207,25 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
           const bool flush = npend == NPM;
           const float4* gq = (const float4*)gv;
           float4* H4 = (float4*)H;
-          for (int kk = 0; kk < steps; kk++) {
-            if (j < Jw && L < nq) {
-              const int s = w + j * NW;
-              const int M = L + s < nq ? L + s : L + s - nq;
-              if (!((nq & 1) == 0 && s == D - 1 && s != 0 && L >= (nq >> 1))) {
-                float4* bp = H4 + (size_t)(4 * s) * nq + L;
-                float4 b0 = bp[0], b1 = bp[nq], b2 = bp[2 * nq], b3 = bp[3 * nq];
-                if (flush) {
-#pragma unroll
-                  for (int k = 0; k < NPM; k++) {
-                    const float4 sv = ((const float4*)up_plane(k, 0))[L], hv = ((const float4*)up_plane(k, 1))[L];
-                    const float4 av = ((const float4*)up_plane(k, 2))[M], bv = ((const float4*)up_plane(k, 3))[M];
-                    const float ux[4] = {av.x, av.y, av.z, av.w}, uy[4] = {bv.x, bv.y, bv.z, bv.w};
-                    hquad_upd(b0, make_float2(sv.x, hv.x), ux, uy);
-                    hquad_upd(b1, make_float2(sv.y, hv.y), ux, uy);
-                    hquad_upd(b2, make_float2(sv.z, hv.z), ux, uy);
-                    hquad_upd(b3, make_float2(sv.w, hv.w), ux, uy);
-                  }
-                  bp[0] = b0;
-                  bp[nq] = b1;
-                  bp[2 * nq] = b2;
-                  bp[3 * nq] = b3;
-                }
-                // rows 4L.. gain B v_M; then, off the diagonal, rows 4M.. gain B^T v_L. Another
-                // lane of this wave may touch quad M in the first update or quad L in the second,
-                // so the compiler barriers keep each read behind the previous write (the
-                // hardware keeps a wave's LDS operations in order). (Keeping the first update in
-                // registers while a lane's L stays fixed measured no faster: 119.9 against
-                // 118.9 ms on the medium workload; loading the next block's rows while this one
-                // is used spilled 76-244 bytes per lane and measured 125.1 against 119.5 ms.)
-                const float4 vm = gq[M];
-                float4* a4 = (float4*)(acc + cp * n4);
-                {
-                  float4 v = a4[L];
-                  v.x += fmaf(b0.w, vm.w, fmaf(b0.z, vm.z, fmaf(b0.y, vm.y, b0.x * vm.x)));
-                  v.y += fmaf(b1.w, vm.w, fmaf(b1.z, vm.z, fmaf(b1.y, vm.y, b1.x * vm.x)));
-                  v.z += fmaf(b2.w, vm.w, fmaf(b2.z, vm.z, fmaf(b2.y, vm.y, b2.x * vm.x)));
-                  v.w += fmaf(b3.w, vm.w, fmaf(b3.z, vm.z, fmaf(b3.y, vm.y, b3.x * vm.x)));
-                  a4[L] = v;
-                }
-                asm volatile("" ::: "memory");
-                if (s != 0) {
-                  const float4 vl = gq[L];
-                  float4 v = a4[M];
-                  v.x += fmaf(b3.x, vl.w, fmaf(b2.x, vl.z, fmaf(b1.x, vl.y, b0.x * vl.x)));
-                  v.y += fmaf(b3.y, vl.w, fmaf(b2.y, vl.z, fmaf(b1.y, vl.y, b0.y * vl.x)));
-                  v.z += fmaf(b3.z, vl.w, fmaf(b2.z, vl.z, fmaf(b1.z, vl.y, b0.z * vl.x)));
-                  v.w += fmaf(b3.w, vl.w, fmaf(b2.w, vl.z, fmaf(b1.w, vl.y, b0.w * vl.x)));
-                  a4[M] = v;
-                }
-                asm volatile("" ::: "memory");
-              }
-            }
+          // The next block's four rows are loaded while this one is used: a step is one load
+          // latency long otherwise, with three waves per SIMD to cover it. 100,000 ragged
+          // conformers 1,134 -> 1,095 ms. (The 16 registers for it came free with the uniform
+          // reduction results and the shorter pair loop; before them it spilled 76-244 bytes per
+          // lane and lost 5%.)
+          //
+          // one block of a lane's walk: its quads, whether it is kept, and its first row
+          struct Item {
+            int L, M, s;
+            bool on;
+            float4* bp;
+          };
+          auto item = [&]() {
+            Item it;
+            it.L = L;
+            it.s = w + j * NW;
+            it.M = L + it.s < nq ? L + it.s : L + it.s - nq;
+            it.on = j < Jw && L < nq && !((nq & 1) == 0 && it.s == D - 1 && it.s != 0 && L >= (nq >> 1));
+            it.bp = H4 + (it.on ? 4 * it.s * nq + L : 0);
             if (nq <= 64) {
               j += G;
             } else if (nq < 64 + NW) {
@@ -1276,6 +1242,66 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
                 j++;
               }
             }
+            return it;
+          };
+          auto load = [&](const Item& it, float4 (&b)[4]) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) b[r] = it.bp[r * nq];
+          };
+          // rows 4L.. gain B v_M; then, off the diagonal, rows 4M.. gain B^T v_L. Another lane of
+          // this wave may touch quad M in the first update or quad L in the second, so the
+          // compiler barriers keep each read behind the previous write (the hardware keeps a
+          // wave's LDS operations in order).
+          auto use = [&](const Item& it, float4 (&b)[4]) {
+            if (it.on) {
+              const int L = it.L, M = it.M;
+              if (flush) {
+#pragma unroll
+                for (int k = 0; k < NPM; k++) {
+                  const float4 sv = ((const float4*)up_plane(k, 0))[L], hv = ((const float4*)up_plane(k, 1))[L];
+                  const float4 av = ((const float4*)up_plane(k, 2))[M], bv = ((const float4*)up_plane(k, 3))[M];
+                  const float ux[4] = {av.x, av.y, av.z, av.w}, uy[4] = {bv.x, bv.y, bv.z, bv.w};
+                  hquad_upd(b[0], make_float2(sv.x, hv.x), ux, uy);
+                  hquad_upd(b[1], make_float2(sv.y, hv.y), ux, uy);
+                  hquad_upd(b[2], make_float2(sv.z, hv.z), ux, uy);
+                  hquad_upd(b[3], make_float2(sv.w, hv.w), ux, uy);
+                }
+#pragma unroll
+                for (int r = 0; r < 4; r++) it.bp[r * nq] = b[r];
+              }
+              const float4 vm = gq[M];
+              float4* a4 = (float4*)(acc + cp * n4);
+              {
+                float4 v = a4[L];
+                v.x += fmaf(b[0].w, vm.w, fmaf(b[0].z, vm.z, fmaf(b[0].y, vm.y, b[0].x * vm.x)));
+                v.y += fmaf(b[1].w, vm.w, fmaf(b[1].z, vm.z, fmaf(b[1].y, vm.y, b[1].x * vm.x)));
+                v.z += fmaf(b[2].w, vm.w, fmaf(b[2].z, vm.z, fmaf(b[2].y, vm.y, b[2].x * vm.x)));
+                v.w += fmaf(b[3].w, vm.w, fmaf(b[3].z, vm.z, fmaf(b[3].y, vm.y, b[3].x * vm.x)));
+                a4[L] = v;
+              }
+              asm volatile("" ::: "memory");
+              if (it.s != 0) {
+                const float4 vl = gq[L];
+                float4 v = a4[M];
+                v.x += fmaf(b[3].x, vl.w, fmaf(b[2].x, vl.z, fmaf(b[1].x, vl.y, b[0].x * vl.x)));
+                v.y += fmaf(b[3].y, vl.w, fmaf(b[2].y, vl.z, fmaf(b[1].y, vl.y, b[0].y * vl.x)));
+                v.z += fmaf(b[3].z, vl.w, fmaf(b[2].z, vl.z, fmaf(b[1].z, vl.y, b[0].z * vl.x)));
+                v.w += fmaf(b[3].w, vl.w, fmaf(b[2].w, vl.z, fmaf(b[1].w, vl.y, b[0].w * vl.x)));
+                a4[M] = v;
+              }
+              asm volatile("" ::: "memory");
+            }
+          };
+          Item ia = item();
+          float4 ba[4], bb[4];
+          load(ia, ba);
+          for (int kk = 0; kk < steps; kk += 2) {
+            const Item ib = item();
+            load(ib, bb);
+            use(ia, ba);
+            ia = item();
+            load(ia, ba);
+            use(ib, bb);
           }
           // the pending updates' part of H g when they were not added element by element:
           // y_t += alpha_t (s.g) + beta_t (h.g), with the dot products reduced in FP64
