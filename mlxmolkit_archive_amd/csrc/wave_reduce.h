@@ -70,6 +70,16 @@ __device__ __forceinline__ double red_rows(double v) {
   const double r2 = __hiloint2double((int)h23[0], (int)l23[0]), r3 = __hiloint2double((int)h23[1], (int)l23[1]);
   return MAX ? fmax(fmax(r0, r1), fmax(r2, r3)) : ((r0 + r1) + r2) + r3;
 }
+// One value: its rows' results by readlane, which is shorter than the swaps when there is nothing
+// to share them with
+template <bool MAX>
+__device__ __forceinline__ double wave_red1(double v) {
+  v = red_op<MAX>(v, row_xor<1>(v));
+  v = red_op<MAX>(v, row_xor<2>(v));
+  v = red_op<MAX>(v, dpp_d<DPP_ROW_HALF_MIRROR>(v));
+  v = red_op<MAX>(v, row_xor<8>(v));
+  return red_op<MAX>(red_op<MAX>(red_op<MAX>(lane_d(v, 0), lane_d(v, 16)), lane_d(v, 32)), lane_d(v, 48));
+}
 // value q of v over the wave, in the lanes with (lane & 7) == q (K > 4), (lane & 3) == q (K > 2), ...
 template <int K, bool MAX>
 __device__ __forceinline__ double wave_red(const double (&v)[K], int lane) {
@@ -81,7 +91,9 @@ __device__ __forceinline__ double wave_red(const double (&v)[K], int lane) {
 }
 
 // SLOT: LDS words per wave, a power of two that covers the values of one reduction
-template <int NT, int SLOT = 8>
+// EXTRA: the workgroup has more waves than NT / 64; they take part in the barriers and read the
+// totals, and add nothing
+template <int NT, int SLOT = 8, bool EXTRA = false>
 struct Reducer {
   static constexpr int NW = NT / 64;
   double* buf;  // 2 phases * NW * SLOT doubles
@@ -94,6 +106,23 @@ struct Reducer {
     constexpr int KT = K + KM;
     static_assert(KT <= SLOT, "at most SLOT values per reduction");
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if constexpr (KT == 1) {
+      constexpr bool MAX = KM == 1;
+      double a = wave_red1<MAX>(v[0]);
+      if constexpr (NW > 1) {
+        double* b = buf + phase * (NW * SLOT);
+        if (lane == 0 && (!EXTRA || w < NW)) b[w * SLOT] = a;
+        __syncthreads();
+        a = b[0];
+#pragma unroll
+        for (int ww = 1; ww < NW; ww++) a = red_op<MAX>(a, b[ww * SLOT]);
+        phase ^= 1;
+      } else {
+        __syncthreads();
+      }
+      v[0] = a;
+      return;
+    }
     double s = 0.0, x = 0.0;
     if constexpr (K > 0) {
       double t[K];
@@ -112,8 +141,8 @@ struct Reducer {
     } else {
       // sums in the words 0..K-1 of a wave's slot, maxima in K..KT-1
       double* b = buf + phase * (NW * SLOT);
-      if (K > 0 && lane < K) b[w * SLOT + lane] = s;
-      if (KM > 0 && lane < KM) b[w * SLOT + K + lane] = x;
+      if (K > 0 && lane < K && (!EXTRA || w < NW)) b[w * SLOT + lane] = s;
+      if (KM > 0 && lane < KM && (!EXTRA || w < NW)) b[w * SLOT + K + lane] = x;
       __syncthreads();
       if constexpr (K > 0) {
         const int q = lane & (SLOT - 1);
