@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "mmff_hip.h"
 #include "mmff_terms.h"
@@ -515,6 +516,135 @@ __device__ __forceinline__ double eval_tasks(const TView& V, const MolDesc& m, c
   return e + eval_pairs<FAM, G, PT, NT, true>(V, m, xs, acc, diel, mask, et);
 }
 
+// eval_terms with HELP times as many threads as the NT lanes whose energy sums it forms. Every
+// thread evaluates terms (bonded ones as in eval_tasks, pairs in steps of NT); their FP32 energies
+// go through LDS to the lanes that eval_terms would have evaluated them on, which add them up in
+// eval_terms' order, so the energy has the same bits as with NT threads (gradient sums are exact
+// in any order). eb holds the bonded energies (eb_n floats), ring two rounds of pair energies.
+// Returns the lane's energy partial; zero for the threads past NT.
+constexpr int HELP_STEPS = 2;  // pairs per thread and round
+template <int NT>
+constexpr size_t help_ring_floats(int help) {
+  return 2 * (size_t)HELP_STEPS * help * NT;
+}
+template <int FAM, bool G, bool EV, int NT, int HELP>
+__device__ __forceinline__ double eval_help(const TView& V, const MolDesc& m, const float* xs,
+                                            unsigned long long* gacc, int diel, float* eb, int eb_n, float* ring) {
+  constexpr int NR = NT * HELP, NW = NR / 64, K = HELP_STEPS * HELP;
+  LdsAcc<G> acc{gacc};
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // eval_terms' numbering: bonds, angles, stretch-bends, out-of-planes, torsions
+  const int c1 = m.nb, c2 = c1 + m.na, c3 = c2 + m.nsb, c4 = c3 + m.noop, c5 = c4 + m.ntor;
+  const bool ordered = c5 <= eb_n;  // (a caller that understated its tables: each thread keeps its own)
+  double own = 0.0;
+  auto put = [&](int t, float v) {
+    if (!EV) return;
+    if (ordered)
+      eb[t] = v;
+    else
+      own += v;
+  };
+  const int t1 = (m.ntor + 63) >> 6, t2 = t1 + ((m.nsb + 63) >> 6), t3 = t2 + ((m.na + 63) >> 6),
+            t4 = t3 + ((m.noop + 63) >> 6), t5 = t4 + ((m.nb + 63) >> 6);
+  for (int k = 0; k * NW < t5; k++) {
+    const int t = (k & 1) ? (k + 1) * NW - 1 - w : k * NW + w;
+    if (t < t1) {
+      const int u = t * 64 + lane;
+      if (u < m.ntor) {
+        const uint2 ix = V.tor_idx[u];
+        const float4 p = V.tor_p[u];
+        put(c4 + u, t_torsion<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
+                                      (int)(ix.y >> 16), p.x, p.y, p.z));
+      }
+    } else if (t < t2) {
+      const int u = (t - t1) * 64 + lane;
+      if (u < m.nsb) {
+        const uint2 ix = V.sb_idx[u];
+        const float4 p = V.sb_p[u];
+        put(c2 + u, t_strbend<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)ix.y, p.x, p.y, p.z,
+                                      p.w, V.sb_t0[u]));
+      }
+    } else if (t < t3) {
+      const int u = (t - t2) * 64 + lane;
+      if (u < m.na) {
+        const uint2 ix = V.ang_idx[u];
+        const float2 p = V.ang_p[u];
+        put(c1 + u, t_angle<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff), p.x, p.y,
+                                    (ix.y >> 16) != 0));
+      }
+    } else if (t < t4) {
+      const int u = (t - t3) * 64 + lane;
+      if (u < m.noop) {
+        const uint2 ix = V.oop_idx[u];
+        put(c3 + u, t_oop<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
+                                  (int)(ix.y >> 16), V.oop_k[u]));
+      }
+    } else if (t < t5) {
+      const int u = (t - t4) * 64 + lane;
+      if (u < m.nb) {
+        const uint32_t ij = V.bond_ij[u];
+        const float2 p = V.bond_p[u];
+        put(u, t_bond<FAM, G>(xs, acc, (int)(ij & 0xffff), (int)(ij >> 16), p.x, p.y));
+      }
+    }
+  }
+  // pairs: in round r thread (h, t) takes pairs (K r + HELP_STEPS h + j) NT + t
+  const int np = m.npair, last = np - 1;
+  const int t = threadIdx.x & (NT - 1), h = threadIdx.x / NT;
+  const int rounds = np > 0 ? (np - 1) / (K * NT) + 1 : 0;
+  double pairs = 0.0;
+  uint32_t ij[HELP_STEPS];
+  float4 pp[HELP_STEPS];
+  const int u0 = HELP_STEPS * h * NT + t;
+  if (rounds > 0) {
+#pragma unroll
+    for (int j = 0; j < HELP_STEPS; j++) {
+      const unsigned u = (unsigned)min(u0 + j * NT, last);
+      ij[j] = V.pair_ij[u];
+      pp[j] = V.pair_p[u];
+    }
+  }
+  if (EV && rounds == 0) __syncthreads();  // the bonded energies
+  for (int r = 0; r < rounds; r++) {
+    uint32_t nij[HELP_STEPS];
+    float4 npp[HELP_STEPS];
+    const int u1 = u0 + r * K * NT;
+#pragma unroll
+    for (int j = 0; j < HELP_STEPS; j++) {
+      const unsigned u = (unsigned)min(u1 + (K + j) * NT, last);
+      nij[j] = V.pair_ij[u];
+      npp[j] = V.pair_p[u];
+    }
+    float* row = ring + (r & 1) * K * NT;
+#pragma unroll
+    for (int j = 0; j < HELP_STEPS; j++) {
+      if (u1 + j * NT < np) {
+        float ev = 0.f, ee = 0.f;
+        t_pair<FAM, G, EV>(xs, acc, (int)(ij[j] & 0xffff), (int)(ij[j] >> 16), pp[j].w, pp[j].y, pp[j].z, diel, ev, ee);
+        if (EV) row[(HELP_STEPS * h + j) * NT + t] = ev + ee;
+      }
+      ij[j] = nij[j];
+      pp[j] = npp[j];
+    }
+    if (EV) {
+      __syncthreads();  // this round's energies; the other half is free, its readers are past it
+      if (h == 0) {
+#pragma unroll
+        for (int k = 0; k < K; k++)
+          if ((r * K + k) * NT + t < np) pairs += (double)row[k * NT + t];
+      }
+    }
+  }
+  if (!EV) return 0.0;
+  if (!ordered) return own + (pairs + 0.0);
+  double e = 0.0;
+  if (h == 0) {
+    for (int k = t; k < c5; k += NT) e += eb[k];
+    if (np > 0) e += pairs + 0.0;
+  }
+  return e;
+}
+
 // ------------------------------------------------------------------------------------
 // four consecutive elements (t, j..j+3) of a symmetric matrix in padded packed storage
 // (column c at pcol(c), cb = pcol(t), pj = pcol(j)), with the matching gradient entries
@@ -716,7 +846,8 @@ struct NkParams {
   int m;
   int max_n;          // 3 * max_atoms rounded up to a multiple of 4
   int ls_grad;
-  int tbytes;         // LDS bytes reserved for staged term tables (TL kernels)
+  int tbytes;         // LDS bytes reserved for staged term tables (TL kernels), else 0
+  int eb_floats;      // LDS floats for bonded energies (HELP kernels)
   int xcd_on;         // order is split into 8 per-XCD queues at xcd_off
   int32_t xcd_off[9];
 };
@@ -750,14 +881,16 @@ __host__ __device__ inline int sym_acc_floats(int max_n) { return max_n > 256 ? 
 // hm: Hessian placement (0 packed LDS, 1 full HBM, 2 packed HBM, 3 symmetric blocked HBM);
 // only the full and symmetric HBM BFGS kernels keep the extra pending-update slots, and the
 // symmetric one adds its per-wave accumulators
-__host__ __device__ inline size_t nk_lds_bytes(int algo, int hm, int nt, int max_n, int m, size_t tbytes = 0) {
+// help > 1: two rounds of pair energies and eb_floats of bonded energies
+__host__ __device__ inline size_t nk_lds_bytes(int algo, int hm, int nt, int max_n, int m, size_t tbytes = 0,
+                                               int help = 1, int eb_floats = 0) {
   const bool hlds = hm == 0;
   size_t nw = (size_t)nt / 64;
   size_t b = 16 * nw * sizeof(double) + 64 + 2 * (size_t)LBFGS_MAX_M * sizeof(double);
   b += (size_t)max_n * 8;  // gradient accumulators
   b += (size_t)max_n * 4 * 4;   // xs, d, xo, hd
   b += (size_t)max_n * 8;       // g, dg
-  b += (size_t)max_n * 16;      // a pending update: s, h, alpha, beta
+  if (algo == MMFFHIP_BFGS || help == 1) b += (size_t)max_n * 16;  // a pending update: s, h, alpha, beta
   if (algo == MMFFHIP_BFGS && (hm == 1 || hm == 3)) b += (size_t)(hpend_for(nt) - 1) * max_n * 16;  // more pending updates
   if (algo == MMFFHIP_BFGS && hm == 3) b += nw * (size_t)sym_acc_floats(max_n) * 4;
   if (algo == MMFFHIP_LBFGS) {
@@ -766,6 +899,7 @@ __host__ __device__ inline size_t nk_lds_bytes(int algo, int hm, int nt, int max
     b += ((packed_floats(max_n) * 4) + 15) & ~(size_t)15;
   }
   b += (tbytes + 15) & ~(size_t)15;
+  if (help > 1) b += 4 * (help_ring_floats<1>(help) * nt + (size_t)eb_floats);
   return b;
 }
 
@@ -789,14 +923,20 @@ __device__ __forceinline__ float h_init(const float* pc, float psc, int i, int j
 // for three waves per SIMD (at most 168 VGPRs), so three workgroups share a CU: their LDS
 // use is small, and the extra resident conformers hide memory latency better than the
 // registers the compiler would otherwise use (medium workload: 172.6 against 178.5 ms).
-template <int ALGO, int HM, int TL, int NT>
-__global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 1) k_minimize_nk(KBatch B, NkParams P) {
+// HELP: a conformer's workgroup has HELP * NT threads, of which the first NT do all that NT threads
+// do and the others share the term evaluation (eval_help): same results, shorter iterations.
+// For batches of at most one conformer per CU, whose time is the longest conformer's chain of
+// iterations. Three times 256 threads keep three waves per SIMD and their 168 registers.
+template <int ALGO, int HM, int TL, int NT, int HELP = 1>
+__global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256) ? (HELP > 1 ? 1 : 3) : 1)
+    k_minimize_nk(KBatch B, NkParams P) {
   constexpr bool HLDS = HM == 0;    // LDS-resident (also selects the LDS L-BFGS history)
   constexpr bool PACKED = HM == 0 || HM == 2;  // packed upper triangle, select read + column-pair write-back
   constexpr bool SYM = HM == 3 && ALGO == MMFFHIP_BFGS;  // symmetric 4x4 blocks in HBM
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int NW = NT / 64;
-  const int tid = threadIdx.x;
+  // a helper's index lies past every loop's end
+  const int tid = HELP == 1 || threadIdx.x < NT ? (int)threadIdx.x : 1 << 30;
   const int mn = P.max_n;
   double* red = (double*)smem;
   int* s_int = (int*)(red + 16 * NW);
@@ -822,7 +962,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
   auto up_plane = [&](int k, int c) { return UP + (size_t)(4 * k + c) * mn; };  // c: s, h, alpha, beta
   auto sh_slot = [&](int k) { return (float2*)up_plane(k, 0); };
   auto ab_slot = [&](int k) { return (float2*)up_plane(k, 2); };
-  float* big = UP + (size_t)NPM * 4 * mn;
+  float* big = ALGO == MMFFHIP_BFGS || HELP == 1 ? UP + (size_t)NPM * 4 * mn : UP;
   float* H = HLDS ? big : P.hglob + (size_t)blockIdx.x * P.slot_floats;
   size_t big_floats = 0;
   if (HLDS) big_floats = ALGO == MMFFHIP_BFGS ? packed_floats(mn) : 2 * (size_t)P.m * mn;
@@ -833,13 +973,15 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
     for (int i = tid; i < NW * sacc_w; i += NT) big[i] = 0.f;
   }
   unsigned char* tstage = (unsigned char*)(big + big_floats);
+  float* ring = (float*)(tstage + P.tbytes);  // HELP: pair energies, then bonded energies
+  float* eb = ring + help_ring_floats<NT>(HELP);
   const int M = P.m;
   float* S = H;
   float* Y = H + (size_t)M * mn;
   double* rho = lb_sc;
   double* alf = lb_sc + LBFGS_MAX_M;
 
-  Reducer<NT> R{red, 0};
+  Reducer<NT, 8, (HELP > 1)> R{red, 0};
 
   for (;;) {
     if (tid == 0) {
@@ -938,9 +1080,18 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
     };
     __syncthreads();
 
+    auto evaluate = [&](auto grad, auto energy) {
+      constexpr bool G = decltype(grad)::value, EV = decltype(energy)::value;
+      if constexpr (HELP > 1)
+        return eval_help<FAM_TG, G, EV, NT, HELP>(TV, m, xs, gacc, P.diel, eb, P.eb_floats, ring);
+      else
+        return eval_terms<FAM_TG, G, false, NT, TL == 0, EV>(TV, m, xs, gacc, P.diel, 0x7fu, nullptr);
+    };
+    const std::true_type yes;
+    const std::false_type no;
     int n_grads = 1, n_evals = 0, iters = 0;
     // initial energy + gradient (mmff_bfgs_source_tg.metal:115-135)
-    double E = R.sum(eval_terms<FAM_TG, true, false, NT, TL == 0>(TV, m, xs, gacc, P.diel, 0x7fu, nullptr));
+    double E = R.sum(evaluate(yes, yes));
     float gscale = GRAD_SCALE_INIT;
     {
       double mxg = 0.0;
@@ -1017,9 +1168,9 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
         __syncthreads();
         double te;
         if (P.ls_grad)
-          te = R.sum(eval_terms<FAM_TG, true, false, NT, TL == 0>(TV, m, xs, gacc, P.diel, 0x7fu, nullptr));
+          te = R.sum(evaluate(yes, yes));
         else
-          te = R.sum(eval_terms<FAM_TG, false, false, NT, TL == 0>(TV, m, xs, gacc, P.diel, 0x7fu, nullptr));
+          te = R.sum(evaluate(no, yes));
         n_evals++;
         if (te - E_old <= FUNCTOL * lam * slope) {
           E = te;
@@ -1087,7 +1238,7 @@ __global__ void __launch_bounds__(NT, ((HM == 1 || HM == 3) && NT <= 256) ? 3 : 
       if (!have_grad) {
         for (int i = tid; i < n; i += NT) gacc[i] = 0ull;
         __syncthreads();
-        eval_terms<FAM_TG, true, false, NT, TL == 0, false>(TV, m, xs, gacc, P.diel, 0x7fu, nullptr);
+        evaluate(yes, no);
         __syncthreads();
       }
       n_grads++;
@@ -2077,16 +2228,23 @@ struct NkPlan {
   int hm = 0;  // Hessian placement of k_minimize_nk (0 packed LDS, 1 full HBM, 2 packed HBM, 3 symmetric HBM)
   int tl = 0;  // term tables: 0 global, 1 all staged in LDS, 2 bonded staged
   int tbytes = 0;
+  int help = 1;       // threads per lane (k_minimize_nk's HELP)
+  int eb_floats = 0;
   size_t lds = 0;
   int grid = 0;
   size_t slot_floats = 0;
   int max_n = 0;
 };
 
-template <int ALGO, int HM, int TL, int NT>
+template <int ALGO, int HM, int TL, int NT, int HELP = 1>
 const void* nk_kernel_ptr() {
-  return (const void*)&k_minimize_nk<ALGO, HM, TL, NT>;
+  return (const void*)&k_minimize_nk<ALGO, HM, TL, NT, HELP>;
 }
+
+// kernels with NK_HELP threads per lane of 256
+constexpr int NK_HELP = 3;
+#define NK_HELP_EACH(X) \
+  X(0, 3, 2, 256) X(0, 3, 0, 256) X(1, 0, 2, 256) X(1, 0, 0, 256) X(1, 1, 2, 256) X(1, 1, 0, 256)
 
 #define NK_FOR_EACH(X)                                                                                   \
   X(0, 0, 1, 64) X(0, 0, 1, 128) X(0, 0, 1, 192) X(0, 0, 1, 256) X(0, 0, 1, 384) X(0, 0, 1, 512)        \
@@ -2102,11 +2260,15 @@ const void* nk_kernel_ptr() {
   X(1, 0, 0, 128) X(1, 0, 0, 256) X(1, 0, 0, 512)                                                      \
   X(1, 1, 0, 128) X(1, 1, 0, 192) X(1, 1, 0, 256) X(1, 1, 0, 512) X(1, 1, 2, 256)
 
-const void* nk_kernel(int algo, int hm, int tl, int nt) {
+const void* nk_kernel(int algo, int hm, int tl, int nt, int help = 1) {
 #define NKSEL(A, H, TL, T) \
-  if (algo == A && hm == H && tl == TL && nt == T) return nk_kernel_ptr<A, H, TL, T>();
+  if (algo == A && hm == H && tl == TL && nt == T && help == 1) return nk_kernel_ptr<A, H, TL, T>();
+#define NKSELH(A, H, TL, T) \
+  if (algo == A && hm == H && tl == TL && nt == T && help == NK_HELP) return nk_kernel_ptr<A, H, TL, T, NK_HELP>();
   NK_FOR_EACH(NKSEL)
+  NK_HELP_EACH(NKSELH)
 #undef NKSEL
+#undef NKSELH
   return nullptr;
 }
 
@@ -2164,11 +2326,36 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
       pl.lds = with;
     }
   }
-  const void* kp = nk_kernel(o->algo, pl.hm, pl.tl, pl.nt);
+  // At most one conformer per CU: the time is the longest conformer's, so its workgroup gets
+  // helper threads, and L-BFGS its history in LDS where that fits (both leave the results as
+  // they are). The bonded terms' energies take a word each; a bonded term has at least 12 table
+  // bytes, so table_lds_bytes bounds their number. Ten conformers of 48 atoms, BFGS,
+  // host work included: 4.28 -> 3.99 ms; 221 chains of 199-329 atoms, L-BFGS: 180 -> 127 ms (151 with
+  // the history in LDS alone).
+  if (b->n_confs <= di.n_cu && o->table_lds_bytes > 0) {
+    const int eb = (o->table_lds_bytes / 12 + 64) & ~63;
+    const struct {
+      int hm, tl;
+    } tries[] = {{0, 2}, {0, 0}, {pl.hm, 2}, {pl.hm, 0}};
+    for (const auto& t : tries) {
+      if (t.hm == 0 && o->algo != MMFFHIP_LBFGS) continue;
+      const int tb = t.tl ? ((o->table_lds_bytes + 15) / 16) * 16 : 0;
+      const size_t lds = nk_lds_bytes(o->algo, t.hm, pl.nt, pl.max_n, m, (size_t)tb, NK_HELP, eb);
+      if (!nk_kernel(o->algo, t.hm, t.tl, pl.nt, NK_HELP) || lds > (size_t)di.lds) continue;
+      pl.hm = t.hm;
+      pl.tl = t.tl;
+      pl.tbytes = tb;
+      pl.help = NK_HELP;
+      pl.eb_floats = eb;
+      pl.lds = lds;
+      break;
+    }
+  }
+  const void* kp = nk_kernel(o->algo, pl.hm, pl.tl, pl.nt, pl.help);
   if (!kp) return fail(MMFFHIP_ERR_ARG, "no kernel instantiated for this (algo, placement, block) combination");
   allow_lds(kp, pl.lds);
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kp, pl.nt, pl.lds) != hipSuccess || per_cu < 1)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kp, pl.nt * pl.help, pl.lds) != hipSuccess || per_cu < 1)
     per_cu = 1;
   pl.grid = std::max(1, std::min(b->n_confs, di.n_cu * per_cu));
   pl.slot_floats = 0;
@@ -2184,19 +2371,26 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
 
 size_t nk_ws_bytes(const NkPlan& pl) { return 256 + (size_t)pl.grid * pl.slot_floats * 4; }
 
-template <int ALGO, int HM, int TL, int NT>
+template <int ALGO, int HM, int TL, int NT, int HELP = 1>
 void launch_nk_t(const KBatch& kb, const NkParams& P, const NkPlan& pl, hipStream_t s) {
-  hipLaunchKernelGGL((k_minimize_nk<ALGO, HM, TL, NT>), dim3(pl.grid), dim3(NT), pl.lds, s, kb, P);
+  hipLaunchKernelGGL((k_minimize_nk<ALGO, HM, TL, NT, HELP>), dim3(pl.grid), dim3(NT * HELP), pl.lds, s, kb, P);
 }
 
 void launch_nk(int algo, const KBatch& kb, const NkParams& P, const NkPlan& pl, hipStream_t s) {
 #define NKL(A, H, TL, T)                                          \
-  if (algo == A && pl.hm == H && pl.tl == TL && pl.nt == T) {     \
-    launch_nk_t<A, H, TL, T>(kb, P, pl, s);                       \
-    return;                                                       \
+  if (algo == A && pl.hm == H && pl.tl == TL && pl.nt == T && pl.help == 1) { \
+    launch_nk_t<A, H, TL, T>(kb, P, pl, s);                                   \
+    return;                                                                   \
+  }
+#define NKLH(A, H, TL, T)                                                           \
+  if (algo == A && pl.hm == H && pl.tl == TL && pl.nt == T && pl.help == NK_HELP) { \
+    launch_nk_t<A, H, TL, T, NK_HELP>(kb, P, pl, s);                                \
+    return;                                                                         \
   }
   NK_FOR_EACH(NKL)
+  NK_HELP_EACH(NKLH)
 #undef NKL
+#undef NKLH
 }
 
 // Clear the work queue at the front of `workspace` with a fill kernel (graph-capture safe)
@@ -2224,7 +2418,8 @@ int run_nk(const mmffhip_batch* b, const mmffhip_nk_opts* o, const NkPlan& pl, c
   P.m = o->algo == MMFFHIP_LBFGS ? o->lbfgs_m : 1;
   P.max_n = pl.max_n;
   P.ls_grad = o->ls_grad;
-  P.tbytes = pl.tbytes;
+  P.tbytes = pl.tl ? pl.tbytes : 0;
+  P.eb_floats = pl.eb_floats;
   P.xcd_on = 0;
   for (int x = 0; x < 9; x++) P.xcd_off[x] = 0;
   if (o->xcd_offsets) {

@@ -17,6 +17,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+import conftest
 import oracle
 from golden_io import load_small
 
@@ -381,3 +382,28 @@ def test_multimol_history_placement_does_not_change_results(fill):
     torch.cuda.synchronize()
     assert torch.equal(alone["x"], both["x"][:len(small.x)])
     assert torch.equal(alone["energy"], both["energy"][:6]) and torch.equal(alone["grad_norm"], both["grad_norm"][:6])
+
+
+@pytest.mark.parametrize("use_lbfgs", [False, True])
+@pytest.mark.parametrize("ls_grad", [False, True])
+@pytest.mark.parametrize("family", ["small", "ragged", "chain"])
+def test_helper_threads_do_not_change_results(family, use_lbfgs, ls_grad):
+    """A batch of at most one conformer per CU gives each conformer helper threads for its term
+    evaluation (and L-BFGS its history in LDS): bit for bit the results that the same conformers
+    have inside a batch too large for that, among them a molecule of two atoms and no bonded terms
+    but one. Statuses and counters too."""
+    from mlxmolkit_archive_amd import engine, workloads
+    wl = workloads.build(family, n_mols=1 if family == "chain" else 3, n_confs=2)
+    p2 = conftest.mol_params("[H][H]", seed=4, k=1)
+    params, counts = wl.params + [p2[1]], list(wl.conf_counts) + [1]
+    x = np.concatenate([wl.x, p2[2]])
+    n = len(x)
+    kw = dict(max_iters=25, grad_tol=1e-4, use_lbfgs=use_lbfgs, ls_grad=ls_grad, lbfgs_m=8)
+    few = engine.NkRunner(engine.device_batch(params, counts), **kw).run(torch.from_numpy(x).cuda())
+    fill = workloads.build("small", n_mols=1, n_confs=600)
+    many = engine.NkRunner(engine.device_batch(params + fill.params, counts + [600]), **kw).run(
+        torch.from_numpy(np.concatenate([x, fill.x])).cuda())
+    torch.cuda.synchronize()
+    c = sum(counts)
+    assert torch.equal(few.x, many.x[:n]) and torch.equal(few.energy, many.energy[:c])
+    assert torch.equal(few.status, many.status[:c]) and torch.equal(few.counters, many.counters[:c])
