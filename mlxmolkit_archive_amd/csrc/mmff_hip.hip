@@ -516,12 +516,126 @@ __device__ __forceinline__ double eval_tasks(const TView& V, const MolDesc& m, c
   return e + eval_pairs<FAM, G, PT, NT, true>(V, m, xs, acc, diel, mask, et);
 }
 
-// eval_terms with HELP times as many threads as the NT lanes whose energy sums it forms. Every
-// thread evaluates terms (bonded ones as in eval_tasks, pairs in steps of NT); their FP32 energies
-// go through LDS to the lanes that eval_terms would have evaluated them on, which add them up in
-// eval_terms' order, so the energy has the same bits as with NT threads (gradient sums are exact
-// in any order). eb holds the bonded energies (eb_n floats), ring two rounds of pair energies.
-// Returns the lane's energy partial; zero for the threads past NT.
+// The bonded terms of eval_tasks for the minimizers that compare energies trial by trial, with
+// the energy bits of eval_terms' generic loop over NT lanes: every task writes its terms' FP32
+// energies to eb (eb_n >= 64 floats of LDS) under eval_terms' numbering, and lane t < NT adds up
+// numbers t, t + NT, ... in order. Gradient sums are exact in any order, so a task is free to take
+// every T-th term of its type (T tasks): terms follow their central atoms in the tables, and 64
+// consecutive ones send up to 27 lanes' atomics to one LDS word. With the generic loop the bonded
+// terms took 49% of the n <= 96 launch of a 100,000-conformer ragged batch (pairs 14%), 39% for
+// n <= 192, 29% for n <= 354 and 15% above; tasks of consecutive terms changed the batch from
+// 1,095 to 1,084 ms, tasks of spread terms to 999 ms, and 8% of the n <= 96 launch (3% for
+// n <= 354) is left to conflicts.
+// Terms that eb cannot hold at once go in several windows of consecutive terms. The last window's
+// sums are left to the caller, after a barrier of its own: ordered_sum with the returned bounds.
+struct Window {
+  int s, end;
+};
+template <int NT>
+__device__ __forceinline__ void ordered_sum(double& e, const float* eb, Window w, int t) {
+  if (t < NT)
+    for (int k = w.s + ((t - w.s) % NT + NT) % NT; k < w.end; k += NT) e += eb[k - w.s];
+}
+template <int FAM, bool G, bool EV, int NT, int NR>
+__device__ __forceinline__ Window bonded_tasks(const TView& V, const MolDesc& m, const float* xs, LdsAcc<G>& acc,
+                                               float* eb, int eb_n, double& e) {
+  constexpr int NW = NR / 64;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // eval_terms' numbering: bonds, angles, stretch-bends, out-of-planes, torsions
+  const int c1 = m.nb, c2 = c1 + m.na, c3 = c2 + m.nsb, c4 = c3 + m.noop, c5 = c4 + m.ntor;
+  const int t1 = (m.ntor + 63) >> 6, t2 = t1 + ((m.nsb + 63) >> 6), t3 = t2 + ((m.na + 63) >> 6),
+            t4 = t3 + ((m.noop + 63) >> 6), t5 = t4 + ((m.nb + 63) >> 6);
+  Window win{0, c5};
+  const bool one = !EV || c5 <= eb_n;
+  for (;;) {
+    if (EV && c5 - win.s > eb_n) {
+      // up to the last task that fits
+      const int base[6] = {0, c1, c2, c3, c4, c5}, lim = win.s + eb_n;
+      win.end = win.s;
+#pragma unroll
+      for (int k = 0; k < 5; k++)
+        if (lim > base[k] && win.s < base[k + 1])
+          win.end = lim >= base[k + 1] ? base[k + 1] : base[k] + ((lim - base[k]) & ~63);
+    } else {
+      win.end = c5;
+    }
+    for (int k = 0; k * NW < t5; k++) {
+      const int t = (k & 1) ? (k + 1) * NW - 1 - w : k * NW + w;
+      auto mine = [&](int first, int end, int base, int n, int& u) {
+        if (one) {
+          u = lane * (end - first) + (t - first);
+          return u < n;
+        }
+        u = (t - first) * 64;
+        const bool in = base + u >= win.s && base + u < win.end;
+        u += lane;
+        return in && u < n;
+      };
+      auto put = [&](int i, float v) {
+        if (EV) eb[i - win.s] = v;
+      };
+      int u;
+      if (t < t1) {
+        if (mine(0, t1, c4, m.ntor, u)) {
+          const uint2 ix = V.tor_idx[u];
+          const float4 p = V.tor_p[u];
+          put(c4 + u, t_torsion<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
+                                        (int)(ix.y >> 16), p.x, p.y, p.z));
+        }
+      } else if (t < t2) {
+        if (mine(t1, t2, c2, m.nsb, u)) {
+          const uint2 ix = V.sb_idx[u];
+          const float4 p = V.sb_p[u];
+          put(c2 + u, t_strbend<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)ix.y, p.x, p.y, p.z,
+                                        p.w, V.sb_t0[u]));
+        }
+      } else if (t < t3) {
+        if (mine(t2, t3, c1, m.na, u)) {
+          const uint2 ix = V.ang_idx[u];
+          const float2 p = V.ang_p[u];
+          put(c1 + u, t_angle<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff), p.x,
+                                      p.y, (ix.y >> 16) != 0));
+        }
+      } else if (t < t4) {
+        if (mine(t3, t4, c3, m.noop, u)) {
+          const uint2 ix = V.oop_idx[u];
+          put(c3 + u, t_oop<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
+                                    (int)(ix.y >> 16), V.oop_k[u]));
+        }
+      } else if (t < t5) {
+        if (mine(t4, t5, 0, m.nb, u)) {
+          const uint32_t ij = V.bond_ij[u];
+          const float2 p = V.bond_p[u];
+          put(u, t_bond<FAM, G>(xs, acc, (int)(ij & 0xffff), (int)(ij >> 16), p.x, p.y));
+        }
+      }
+    }
+    if (win.end >= c5) return win;
+    __syncthreads();
+    ordered_sum<NT>(e, eb, win, (int)threadIdx.x);
+    __syncthreads();
+    win.s = win.end;
+  }
+}
+
+// eval_terms with the bonded terms as bonded_tasks: the same results
+template <int FAM, bool G, bool EV, int NT>
+__device__ __forceinline__ double eval_ordered(const TView& V, const MolDesc& m, const float* xs,
+                                               unsigned long long* gacc, int diel, float* eb, int eb_n) {
+  LdsAcc<G> acc{gacc};
+  double e = 0.0;
+  const Window win = bonded_tasks<FAM, G, EV, NT, NT>(V, m, xs, acc, eb, eb_n, e);
+  const double pairs = eval_pairs<FAM, G, false, NT, EV>(V, m, xs, acc, diel, 0x7fu, nullptr);
+  if (!EV) return 0.0;
+  __syncthreads();
+  ordered_sum<NT>(e, eb, win, (int)threadIdx.x);
+  return e + pairs;
+}
+
+// eval_ordered with HELP times as many threads as the NT lanes whose energy sums it forms: every
+// thread evaluates bonded terms and pairs (in steps of NT), and the pairs' FP32 energies go
+// through LDS too, two rounds of them in ring. Returns the lane's energy partial; zero for the
+// threads past NT.
 constexpr int HELP_STEPS = 2;  // pairs per thread and round
 template <int NT>
 constexpr size_t help_ring_floats(int help) {
@@ -530,64 +644,10 @@ constexpr size_t help_ring_floats(int help) {
 template <int FAM, bool G, bool EV, int NT, int HELP>
 __device__ __forceinline__ double eval_help(const TView& V, const MolDesc& m, const float* xs,
                                             unsigned long long* gacc, int diel, float* eb, int eb_n, float* ring) {
-  constexpr int NR = NT * HELP, NW = NR / 64, K = HELP_STEPS * HELP;
+  constexpr int NR = NT * HELP, K = HELP_STEPS * HELP;
   LdsAcc<G> acc{gacc};
-  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // eval_terms' numbering: bonds, angles, stretch-bends, out-of-planes, torsions
-  const int c1 = m.nb, c2 = c1 + m.na, c3 = c2 + m.nsb, c4 = c3 + m.noop, c5 = c4 + m.ntor;
-  const bool ordered = c5 <= eb_n;  // (a caller that understated its tables: each thread keeps its own)
-  double own = 0.0;
-  auto put = [&](int t, float v) {
-    if (!EV) return;
-    if (ordered)
-      eb[t] = v;
-    else
-      own += v;
-  };
-  const int t1 = (m.ntor + 63) >> 6, t2 = t1 + ((m.nsb + 63) >> 6), t3 = t2 + ((m.na + 63) >> 6),
-            t4 = t3 + ((m.noop + 63) >> 6), t5 = t4 + ((m.nb + 63) >> 6);
-  for (int k = 0; k * NW < t5; k++) {
-    const int t = (k & 1) ? (k + 1) * NW - 1 - w : k * NW + w;
-    if (t < t1) {
-      const int u = t * 64 + lane;
-      if (u < m.ntor) {
-        const uint2 ix = V.tor_idx[u];
-        const float4 p = V.tor_p[u];
-        put(c4 + u, t_torsion<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
-                                      (int)(ix.y >> 16), p.x, p.y, p.z));
-      }
-    } else if (t < t2) {
-      const int u = (t - t1) * 64 + lane;
-      if (u < m.nsb) {
-        const uint2 ix = V.sb_idx[u];
-        const float4 p = V.sb_p[u];
-        put(c2 + u, t_strbend<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)ix.y, p.x, p.y, p.z,
-                                      p.w, V.sb_t0[u]));
-      }
-    } else if (t < t3) {
-      const int u = (t - t2) * 64 + lane;
-      if (u < m.na) {
-        const uint2 ix = V.ang_idx[u];
-        const float2 p = V.ang_p[u];
-        put(c1 + u, t_angle<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff), p.x, p.y,
-                                    (ix.y >> 16) != 0));
-      }
-    } else if (t < t4) {
-      const int u = (t - t3) * 64 + lane;
-      if (u < m.noop) {
-        const uint2 ix = V.oop_idx[u];
-        put(c3 + u, t_oop<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
-                                  (int)(ix.y >> 16), V.oop_k[u]));
-      }
-    } else if (t < t5) {
-      const int u = (t - t4) * 64 + lane;
-      if (u < m.nb) {
-        const uint32_t ij = V.bond_ij[u];
-        const float2 p = V.bond_p[u];
-        put(u, t_bond<FAM, G>(xs, acc, (int)(ij & 0xffff), (int)(ij >> 16), p.x, p.y));
-      }
-    }
-  }
+  double e = 0.0;
+  const Window win = bonded_tasks<FAM, G, EV, NT, NR>(V, m, xs, acc, eb, eb_n, e);
   // pairs: in round r thread (h, t) takes pairs (K r + HELP_STEPS h + j) NT + t
   const int np = m.npair, last = np - 1;
   const int t = threadIdx.x & (NT - 1), h = threadIdx.x / NT;
@@ -636,13 +696,8 @@ __device__ __forceinline__ double eval_help(const TView& V, const MolDesc& m, co
     }
   }
   if (!EV) return 0.0;
-  if (!ordered) return own + (pairs + 0.0);
-  double e = 0.0;
-  if (h == 0) {
-    for (int k = t; k < c5; k += NT) e += eb[k];
-    if (np > 0) e += pairs + 0.0;
-  }
-  return e;
+  ordered_sum<NT>(e, eb, win, (int)threadIdx.x);
+  return e + pairs;
 }
 
 // ------------------------------------------------------------------------------------
@@ -943,11 +998,9 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
   double* lb_sc = (double*)(s_int + 16);  // rho[16], alpha[16]
   unsigned long long* gacc = (unsigned long long*)(lb_sc + 2 * LBFGS_MAX_M);
   float* gv = (float*)(gacc + mn);  // scaled gradient g
-  float* dgv = gv + mn;             // its last change dg
-  float* xs = dgv + mn;
+  float* xs = gv + mn;
   float* d = xs + mn;   // direction (also y2 = H g scratch)
   float* xo = d + mn;   // previous x, then xi = x - x_old
-  float* hd = xo + mn;  // H dg (BFGS) / two-loop q (L-BFGS)
   // A rank-2 update U(t, j) = alpha_t s_j + beta_t h_j (s = x - x_old, h = H dg) takes a slot of
   // 4 mn floats. Global-Hessian BFGS keeps up to NPM pending updates and writes H back once
   // every NPM iterations; the others apply theirs at once. The symmetric pass reads whole quads
@@ -958,20 +1011,25 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
   // The other placements read an update row by row and keep the pairs.
   constexpr bool LAZY = (HM == 1 || HM == 3) && ALGO == MMFFHIP_BFGS;
   constexpr int NPM = LAZY ? hpend_for(NT) : 1;
-  float* UP = hd + mn;
+  float* UP = xo + mn;
   auto up_plane = [&](int k, int c) { return UP + (size_t)(4 * k + c) * mn; };  // c: s, h, alpha, beta
   auto sh_slot = [&](int k) { return (float2*)up_plane(k, 0); };
   auto ab_slot = [&](int k) { return (float2*)up_plane(k, 2); };
-  float* big = ALGO == MMFFHIP_BFGS || HELP == 1 ? UP + (size_t)NPM * 4 * mn : UP;
+  float* dgv = ALGO == MMFFHIP_BFGS || HELP == 1 ? UP + (size_t)NPM * 4 * mn : UP;  // last change of g
+  float* hd = dgv + mn;  // H dg (BFGS) / two-loop q (L-BFGS)
+  float* big = hd + mn;
   float* H = HLDS ? big : P.hglob + (size_t)blockIdx.x * P.slot_floats;
   size_t big_floats = 0;
   if (HLDS) big_floats = ALGO == MMFFHIP_BFGS ? packed_floats(mn) : 2 * (size_t)P.m * mn;
-  // symmetric storage: per-wave H v accumulators (kept zero between passes)
+  // symmetric storage: per-wave H v accumulators, cleared before each pass
   const int sacc_w = sym_acc_floats(mn);
-  if (SYM) {
-    big_floats = (size_t)NW * sacc_w;
-    for (int i = tid; i < NW * sacc_w; i += NT) big[i] = 0.f;
-  }
+  if (SYM) big_floats = (size_t)NW * sacc_w;
+  // During an evaluation the bonded terms' energies lie in dgv, hd and the accumulators (at least
+  // 12 floats per atom, which hold all but a cage molecule's at once), none of which is live then;
+  // L-BFGS has that room where BFGS keeps its update.
+  constexpr bool ORDERED = HELP == 1 && (SYM || ALGO == MMFFHIP_LBFGS);
+  float* ebuf = SYM ? dgv : UP;
+  const int ebuf_n = SYM ? 2 * mn + NW * sacc_w : 4 * mn;
   unsigned char* tstage = (unsigned char*)(big + big_floats);
   float* ring = (float*)(tstage + P.tbytes);  // HELP: pair energies, then bonded energies
   float* eb = ring + help_ring_floats<NT>(HELP);
@@ -1084,6 +1142,8 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
       constexpr bool G = decltype(grad)::value, EV = decltype(energy)::value;
       if constexpr (HELP > 1)
         return eval_help<FAM_TG, G, EV, NT, HELP>(TV, m, xs, gacc, P.diel, eb, P.eb_floats, ring);
+      else if constexpr (ORDERED)
+        return eval_ordered<FAM_TG, G, EV, NT>(TV, m, xs, gacc, P.diel, ebuf, ebuf_n);
       else
         return eval_terms<FAM_TG, G, false, NT, TL == 0, EV>(TV, m, xs, gacc, P.diel, 0x7fu, nullptr);
     };
@@ -1259,6 +1319,8 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
         dgv[i] = gn - gv[i];
         gv[i] = gn;
       }
+      if (SYM)
+        for (int i = tid; i < NW * sacc_w; i += NT) big[i] = 0.f;
       if (v2[1] / fmax(E * (double)gscale, 1.0) < (double)P.grad_tol) {  // :300-316
         status = 0;
         break;
@@ -1497,15 +1559,13 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
           } else {
             __syncthreads();  // every wave's accumulators are complete
           }
-          // sum the waves' accumulators in a fixed order and clear them for the next pass
+          // sum the waves' accumulators in a fixed order
           for (int t = tid; t < n4; t += NT) {
             const int idx = t;
             float y = 0.f;
             for (int ww = 0; ww < NW; ww++)
               for (int c = 0; c < G; c++) {
-                float* a = big + (size_t)ww * sacc_w + c * n4 + idx;
-                y += *a;
-                *a = 0.f;
+                y += big[(size_t)ww * sacc_w + c * n4 + idx];
               }
             if (t < n) {
               if (fact) {
@@ -2357,6 +2417,10 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
   int per_cu = 0;
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kp, pl.nt * pl.help, pl.lds) != hipSuccess || per_cu < 1)
     per_cu = 1;
+  // Twelve waves per CU at most, whatever registers a kernel leaves free: the resident Hessians
+  // stay in the Infinity Cache, a fourth wave per SIMD gains 1% at best (100,000 ragged conformers
+  // 1,084 -> 1,075 ms, 2,500 small ones 13.6 -> 15.0), and callers size their buckets by this grid.
+  per_cu = std::min(per_cu, std::max(1, 12 / (pl.nt * pl.help / 64)));
   pl.grid = std::max(1, std::min(b->n_confs, di.n_cu * per_cu));
   pl.slot_floats = 0;
   if (pl.hm != 0) {

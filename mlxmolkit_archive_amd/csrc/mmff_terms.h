@@ -273,11 +273,10 @@ __device__ __forceinline__ float t_torsion(const float* x, Acc& acc, int i1, int
     float e = 0.0f;
     if (comb >= 1e-16f) {
       float cp = clampf(dot(c1, c2) * rsqrtf(comb), -1.0f, 1.0f);
-      float cos2 = 2.0f * cp * cp - 1.0f, cos3 = cp * (4.0f * cp * cp - 3.0f);
-      // the rounding is written out for the energy alone (which of the first two products is
-      // rounded before the sum would otherwise follow the code that loads V1 and V2)
-      e = G ? 0.5f * (V1 * (1.0f + cp) + V2 * (1.0f - cos2) + V3 * (1.0f + cos3))
-            : 0.5f * fmaf(V3, fmaf(cp, fmaf(cp, 4.0f * cp, -3.0f), 1.0f), fmaf(V1, 1.0f + cp, V2 * (1.0f - cos2)));
+      float cos2 = fmaf(cp, 2.0f * cp, -1.0f);
+      // the rounding is written out: which of the first two products is rounded before the sum
+      // would otherwise follow the code that loads V1 and V2
+      e = 0.5f * fmaf(V3, fmaf(cp, fmaf(cp, 4.0f * cp, -3.0f), 1.0f), fmaf(V1, 1.0f + cp, V2 * (1.0f - cos2)));
     }
     if (G) {
       if (n1 >= 1e-30f && n2 >= 1e-30f) {

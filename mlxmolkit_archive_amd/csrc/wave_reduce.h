@@ -54,7 +54,7 @@ __device__ __forceinline__ void red_step(const double (&v)[K], double (&r)[(K + 
     const double keep = up ? v[2 * k + 1] : v[2 * k], send = up ? v[2 * k] : v[2 * k + 1];
     r[k] = red_op<MAX>(keep, row_xor<X>(send));
   }
-  if (K & 1) r[K / 2] = red_op<MAX>(v[K - 1], row_xor<X>(v[K - 1]));
+  if constexpr (K & 1) r[K / 2] = red_op<MAX>(v[K - 1], row_xor<X>(v[K - 1]));
 }
 // ((row 0 + row 1) + row 2) + row 3 of lane l's column, in every row
 template <bool MAX>
