@@ -452,11 +452,12 @@ __device__ __forceinline__ double eval_terms(const TView& TV, const MolDesc& m, 
 // eval_terms for kernels whose results do not hang on the order of the energy sum (single points;
 // the descents, where the energy only guards): the bonded terms go to the waves in tasks of 64
 // terms of one type, the heaviest types first and the waves taken back and forth, so no wave runs
-// several types' code for parts of its lanes and the waves finish together. The minimizers that
-// compare energies trial by trial keep eval_terms' fixed order. With the generic bonded loop,
-// which also held the next term's parameters in registers (83 now against 103 for the MEGA
-// kernel): 12,139 ragged MEGA energies and gradients 143 -> 123 us, 2,500 TG energies with terms
-// 14.9 -> 13.0 us, the Barzilai-Borwein descent of 1,000 conformers 6.08 -> 4.65 ms.
+// several types' code for parts of its lanes and the waves finish together. A task takes every
+// T-th term of its type (T tasks), because neighbouring terms share atoms and their lanes' atomics
+// would queue for the same LDS words. The minimizers that compare energies trial by trial use
+// bonded_tasks below. 12,139 ragged MEGA energies and gradients: generic loop 143 us, tasks of
+// consecutive terms 123, of spread terms 103; the Barzilai-Borwein descent of 1,000 conformers:
+// 6.08, 4.59, 4.00 ms; the lock-step L-BFGS: 7.00 and 6.28 ms.
 template <int FAM, bool G, bool PT, int NT>
 __device__ __forceinline__ double eval_tasks(const TView& V, const MolDesc& m, const float* xs,
                                              unsigned long long* gacc, int diel, uint32_t mask, double* et) {
@@ -474,7 +475,7 @@ __device__ __forceinline__ double eval_tasks(const TView& V, const MolDesc& m, c
       if (PT) et[kind] += v;
     };
     if (t < t1) {
-      const int u = t * 64 + lane;
+      const int u = lane * t1 + t;
       if ((mask & 16u) && u < m.ntor) {
         const uint2 ix = V.tor_idx[u];
         const float4 p = V.tor_p[u];
@@ -482,7 +483,7 @@ __device__ __forceinline__ double eval_tasks(const TView& V, const MolDesc& m, c
                                  (int)(ix.y >> 16), p.x, p.y, p.z));
       }
     } else if (t < t2) {
-      const int u = (t - t1) * 64 + lane;
+      const int u = lane * (t2 - t1) + (t - t1);
       if ((mask & 4u) && u < m.nsb) {
         const uint2 ix = V.sb_idx[u];
         const float4 p = V.sb_p[u];
@@ -490,7 +491,7 @@ __device__ __forceinline__ double eval_tasks(const TView& V, const MolDesc& m, c
                                  V.sb_t0[u]));
       }
     } else if (t < t3) {
-      const int u = (t - t2) * 64 + lane;
+      const int u = lane * (t3 - t2) + (t - t2);
       if ((mask & 2u) && u < m.na) {
         const uint2 ix = V.ang_idx[u];
         const float2 p = V.ang_p[u];
@@ -498,14 +499,14 @@ __device__ __forceinline__ double eval_tasks(const TView& V, const MolDesc& m, c
                                (ix.y >> 16) != 0));
       }
     } else if (t < t4) {
-      const int u = (t - t3) * 64 + lane;
+      const int u = lane * (t4 - t3) + (t - t3);
       if ((mask & 8u) && u < m.noop) {
         const uint2 ix = V.oop_idx[u];
         add(3, t_oop<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
                              (int)(ix.y >> 16), V.oop_k[u]));
       }
     } else if (t < t5) {
-      const int u = (t - t4) * 64 + lane;
+      const int u = lane * (t5 - t4) + (t - t4);
       if ((mask & 1u) && u < m.nb) {
         const uint32_t ij = V.bond_ij[u];
         const float2 p = V.bond_p[u];
