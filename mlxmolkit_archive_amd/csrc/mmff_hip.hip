@@ -2259,15 +2259,27 @@ size_t eg_lds(int nt, int max_atoms) {
   return 16 * (nt / 64) * 8 + (size_t)3 * max_atoms * (8 + 4) + 16;
 }
 
+// At most one conformer per CU: sixteen waves per conformer, whose latency is the call's; four
+// otherwise. One conformer of a 245-atom chain 50 -> 24 us, 180 conformers of three chains (energies
+// alone) 34.5 -> 19.1 us; molecules of 60 atoms are bound by the host's 10 us per call either way.
+template <int FAM, int NT>
+int launch_eg_nt(const KBatch& kb, const float* x, double* e, double* et, float* g, uint32_t mask, int diel,
+                 hipStream_t s) {
+  const size_t lds = eg_lds(NT, kb.max_atoms);
+  allow_lds((const void*)&k_energy_grad<FAM, NT>, lds);
+  hipLaunchKernelGGL((k_energy_grad<FAM, NT>), dim3(kb.n_confs), dim3(NT), lds, s, kb, x, e, et, g, mask, diel);
+  HIP_TRY(hipGetLastError());
+  return MMFFHIP_OK;
+}
 template <int FAM>
 int launch_eg(const KBatch& kb, const float* x, double* e, double* et, float* g, uint32_t mask, int diel,
               hipStream_t s) {
-  const size_t lds = eg_lds(256, kb.max_atoms);
-  if ((int)lds > dev_info().lds) return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
-  allow_lds((const void*)&k_energy_grad<FAM, 256>, lds);
-  hipLaunchKernelGGL((k_energy_grad<FAM, 256>), dim3(kb.n_confs), dim3(256), lds, s, kb, x, e, et, g, mask, diel);
-  HIP_TRY(hipGetLastError());
-  return MMFFHIP_OK;
+  const DevInfo di = dev_info();
+  if ((int)eg_lds(256, kb.max_atoms) > di.lds)
+    return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
+  if (kb.n_confs <= di.n_cu && (int)eg_lds(1024, kb.max_atoms) <= di.lds)
+    return launch_eg_nt<FAM, 1024>(kb, x, e, et, g, mask, diel, s);
+  return launch_eg_nt<FAM, 256>(kb, x, e, et, g, mask, diel, s);
 }
 
 // The launch of k_mm_chunk: with the history in LDS when that leaves three workgroups per CU, or
