@@ -1913,9 +1913,9 @@ struct MMState {
   size_t total;
 };
 
-template <int NT>
-__device__ void mm_eval(const KBatch& B, const MolDesc& m, float* xs, unsigned long long* gacc, Reducer<NT>& R,
-                        double& E, int n) {
+template <int NT, class Red>
+__device__ void mm_eval(const KBatch& B, const MolDesc& m, float* xs, unsigned long long* gacc, Red& R, double& E,
+                        int n) {
   for (int i = threadIdx.x; i < n; i += NT) gacc[i] = 0ull;
   __syncthreads();
   E = R.sum(eval_tasks<FAM_MEGA, true, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu, nullptr));
@@ -1958,18 +1958,18 @@ __global__ void __launch_bounds__(NT) k_mm_init(KBatch B, MMState S, const float
 }
 
 // K dot products over a conformer's n coordinates: f(i, p) adds coordinate i's products to p
-template <int NT, int K, class F>
-__device__ __forceinline__ void block_dots(Reducer<NT>& R, int n, double (&p)[K], F f) {
+template <int NT, int K, class Red, class F>
+__device__ __forceinline__ void block_dots(Red& R, int tid, int n, double (&p)[K], F f) {
 #pragma unroll
   for (int k = 0; k < K; k++) p[k] = 0.0;
-  for (int i = threadIdx.x; i < n; i += NT) f(i, p);
+  for (int i = tid; i < n; i += NT) f(i, p);
   R.template run<K, 0>(p);
 }
 
 // LDS of k_mm_chunk: reduction buffer, gradient accumulators, x, g, q, x_new and alpha, and the
 // (s, y, rho) history when hl
-size_t mm_lds(int mx, int m, bool hl) {
-  return 16 * 4 * 8 + (size_t)mx * (8 + 16) + 8 * (size_t)m + (hl ? 8 * (size_t)m * (mx + 1) : 0) + 32;
+size_t mm_lds(int nr, int mx, int m, bool hl) {
+  return 16 * (size_t)(nr > 256 ? 2 * (nr / 64) : 4) * 8 + (size_t)mx * (8 + 16) + 8 * (size_t)m + (hl ? 8 * (size_t)m * (mx + 1) : 0) + 32;
 }
 
 // HL: the (s, y) history is worked on in LDS for the launch's iterations (and written through to
@@ -1980,19 +1980,22 @@ size_t mm_lds(int mx, int m, bool hl) {
 // history in memory too. Measured and dropped: the recursion in one wave while the others wait
 // (the same sums without barriers: 7.6 ms, and 3.53 against 2.75 ms for 60 conformers), and one
 // 64-thread workgroup per conformer (12.1 ms).
-template <bool HL>
-__global__ void __launch_bounds__(256, 4) k_mm_chunk(KBatch B, MMState S, int steps, int it_end, int do_sync,
+// NR: threads of the workgroup. The first 256 do everything but the evaluation, which all share
+// (1,024 for batches of at most one conformer per CU; 60 ragged conformers, 100 + 25 iterations:
+// 2.59 -> 2.16 ms).
+template <bool HL, int NR>
+__global__ void __launch_bounds__(NR, NR > 256 ? 1 : 4) k_mm_chunk(KBatch B, MMState S, int steps, int it_end, int do_sync,
                                                      int phase, const int32_t* prev_flag, int32_t* my_flag, int M,
                                                      float max_step, float gsc, float tol) {
   extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int NT = 256, NW = NT / 64;
+  constexpr int NT = 256, NW = NR / 64;
   const int c = blockIdx.x;
   if (c >= B.n_confs) return;
   if (prev_flag && *prev_flag == 0) return;  // every conformer converged at the last sync
-  const int tid = threadIdx.x;
+  const int tid = NR == NT || threadIdx.x < NT ? (int)threadIdx.x : 1 << 30;
   const int mx = 3 * B.max_atoms;
   double* red = (double*)smem;
-  double* alf = red + 16 * NW;  // [M]
+  double* alf = red + 16 * NW + (NR > NT ? 16 * NW : 0);  // [M]
   double* lrho = alf + M;       // [M] when HL
   unsigned long long* gacc = (unsigned long long*)(HL ? lrho + M : lrho);
   float* xs = (float*)(gacc + mx);
@@ -2021,7 +2024,8 @@ __global__ void __launch_bounds__(256, 4) k_mm_chunk(KBatch B, MMState S, int st
         hY[k * HT + i] = gY[k * T + i];
       }
   }
-  Reducer<NT> R{red, 0};
+  Reducer<NT, 8, (NR > NT)> R{red, 0};
+  Reducer<NR> RE{NR > NT ? red + 16 * NW : red, 0};
   double E = S.e_new[c];
   __syncthreads();
   for (int st = 0; st < steps; st++) {
@@ -2033,7 +2037,7 @@ __global__ void __launch_bounds__(256, 4) k_mm_chunk(KBatch B, MMState S, int st
       int sl = head + len - 1;  // newest entry
       if (sl >= M) sl -= M;
       double v3[3];
-      block_dots<NT, 3>(R, n, v3, [&](int i, double (&p)[3]) {
+      block_dots<NT, 3>(R, tid, n, v3, [&](int i, double (&p)[3]) {
         const float qv = gs[i];
         q[i] = qv;
         const double s = hS[sl * HT + i], y = hY[sl * HT + i];
@@ -2048,7 +2052,7 @@ __global__ void __launch_bounds__(256, 4) k_mm_chunk(KBatch B, MMState S, int st
         const int sn = sl == 0 ? M - 1 : sl - 1;
         const float af = (float)a;
         double sq[1];
-        block_dots<NT, 1>(R, n, sq, [&](int i, double (&p)[1]) {
+        block_dots<NT, 1>(R, tid, n, sq, [&](int i, double (&p)[1]) {
           const float qv = q[i] - af * hY[sl * HT + i];
           q[i] = qv;
           p[0] += (double)hS[sn * HT + i] * qv;
@@ -2060,7 +2064,7 @@ __global__ void __launch_bounds__(256, 4) k_mm_chunk(KBatch B, MMState S, int st
       double yr[1];  // q -= alpha_0 y_0, q *= gamma, then y_0.q
       {
         const float af = (float)a;
-        block_dots<NT, 1>(R, n, yr, [&](int i, double (&p)[1]) {
+        block_dots<NT, 1>(R, tid, n, yr, [&](int i, double (&p)[1]) {
           const float y = hY[sl * HT + i];
           float qv = q[i] - af * y;
           qv *= gf;
@@ -2072,7 +2076,7 @@ __global__ void __launch_bounds__(256, 4) k_mm_chunk(KBatch B, MMState S, int st
         const float cf = (float)(alf[h] - rho(sl) * yr[0]);
         const int sn = sl + 1 == M ? 0 : sl + 1;
         if (h + 1 < len) {
-          block_dots<NT, 1>(R, n, yr, [&](int i, double (&p)[1]) {
+          block_dots<NT, 1>(R, tid, n, yr, [&](int i, double (&p)[1]) {
             const float r = q[i] + cf * hS[sl * HT + i];
             q[i] = r;
             p[0] += (double)hY[sn * HT + i] * r;
@@ -2096,7 +2100,10 @@ __global__ void __launch_bounds__(256, 4) k_mm_chunk(KBatch B, MMState S, int st
       xn[3 * a + 2] = xs[3 * a + 2] + dz * f;
     }
     __syncthreads();
-    mm_eval<NT>(B, m, xn, gacc, R, E, n);
+    if constexpr (NR == NT)
+      mm_eval<NT>(B, m, xn, gacc, R, E, n);
+    else
+      mm_eval<NR>(B, m, xn, gacc, RE, E, n);
     // push (s, y, rho) into the ring (:385-399); rho = 0 on bad curvature
     int sl;
     if (len >= M) {
@@ -2107,7 +2114,7 @@ __global__ void __launch_bounds__(256, 4) k_mm_chunk(KBatch B, MMState S, int st
       len++;
     }
     double sy[1];
-    block_dots<NT, 1>(R, n, sy, [&](int i, double (&p)[1]) {
+    block_dots<NT, 1>(R, tid, n, sy, [&](int i, double (&p)[1]) {
       const float gn = from_fx(gacc[i]) * gsc;
       const float s = xn[i] - xs[i], y = gn - gs[i];
       hS[sl * HT + i] = s;
@@ -2282,16 +2289,22 @@ int launch_eg(const KBatch& kb, const float* x, double* e, double* et, float* g,
   return launch_eg_nt<FAM, 256>(kb, x, e, et, g, mask, diel, s);
 }
 
-// The launch of k_mm_chunk: with the history in LDS when that leaves three workgroups per CU, or
-// when there is at most one per CU anyway.
+// The launch of k_mm_chunk: wide workgroups when there is at most one conformer per CU; the history
+// in LDS when it fits there, or leaves three workgroups per CU.
 struct MMChunk {
   void (*kernel)(KBatch, MMState, int, int, int, int, const int32_t*, int32_t*, int, float, float, float);
+  int nr;
   size_t lds;
 };
 MMChunk mm_chunk_plan(int n_confs, int mx, int m, const DevInfo& di) {
-  const size_t hl = mm_lds(mx, m, true);
-  if (hl <= (size_t)di.lds / 3 || (n_confs <= di.n_cu && hl <= (size_t)di.lds)) return {k_mm_chunk<true>, hl};
-  return {k_mm_chunk<false>, mm_lds(mx, m, false)};
+  if (n_confs <= di.n_cu) {
+    const size_t hl = mm_lds(1024, mx, m, true), g = mm_lds(1024, mx, m, false);
+    if (hl <= (size_t)di.lds) return {k_mm_chunk<true, 1024>, 1024, hl};
+    if (g <= (size_t)di.lds) return {k_mm_chunk<false, 1024>, 1024, g};
+  }
+  const size_t hl = mm_lds(256, mx, m, true);
+  if (hl <= (size_t)di.lds / 3) return {k_mm_chunk<true, 256>, 256, hl};
+  return {k_mm_chunk<false, 256>, 256, mm_lds(256, mx, m, false)};
 }
 
 int round4(int v) { return (v + 3) & ~3; }
@@ -2779,7 +2792,7 @@ int mmffhip_multimol_run_ex(const mmffhip_batch* b, const float* x_in, float* x_
     const bool sync = (it % eval_freq) == 0;
     // the batch form has no convergence exit: no conformer ever passes the test (tolerance
     // -1) and no launch reads the previous sync point's count
-    hipLaunchKernelGGL(ck.kernel, dim3(b->n_confs), dim3(NT), ck.lds, s, kb, S, steps, it, sync ? 1 : 0,
+    hipLaunchKernelGGL(ck.kernel, dim3(b->n_confs), dim3(ck.nr), ck.lds, s, kb, S, steps, it, sync ? 1 : 0,
                        0, (k > 0 && !batch) ? S.flags + (k - 1) : (const int32_t*)nullptr, S.flags + k,
                        (int)lbfgs_m, max_step_per_atom, grad_scale, batch ? -1.0f : grad_tol);
     if (sync) k++;
@@ -2794,7 +2807,7 @@ int mmffhip_multimol_run_ex(const mmffhip_batch* b, const float* x_in, float* x_
     int steps = std::min(eval_freq, polish - it);
     it += steps;
     const bool sync = (it % eval_freq) == 0;
-    hipLaunchKernelGGL(ck.kernel, dim3(b->n_confs), dim3(NT), ck.lds, s, kb, S, steps, it, sync ? 1 : 0,
+    hipLaunchKernelGGL(ck.kernel, dim3(b->n_confs), dim3(ck.nr), ck.lds, s, kb, S, steps, it, sync ? 1 : 0,
                        1, kp > n_main ? S.flags + (kp - 1) : (const int32_t*)nullptr, S.flags + kp, (int)lbfgs_m,
                        max_step_per_atom, grad_scale, grad_tol);
     if (sync) kp++;
