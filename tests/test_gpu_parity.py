@@ -407,3 +407,21 @@ def test_helper_threads_do_not_change_results(family, use_lbfgs, ls_grad):
     c = sum(counts)
     assert torch.equal(few.x, many.x[:n]) and torch.equal(few.energy, many.energy[:c])
     assert torch.equal(few.status, many.status[:c]) and torch.equal(few.counters, many.counters[:c])
+
+
+@pytest.mark.parametrize("use_lbfgs", [False, True])
+def test_cage_molecule_energies_in_windows(use_lbfgs):
+    """Cubane has 14 bonded terms per atom, more than the LDS words that hold their energies
+    during an L-BFGS evaluation (12 per atom of the launch's largest molecule), so they pass in
+    windows: bit for bit the results of a batch small enough for helper threads, which hold them
+    all; and BFGS, which has room for them, likewise."""
+    from mlxmolkit_archive_amd import engine
+    _, p, x = conftest.mol_params("C12C3C4C1C5C2C3C45", seed=5, k=2)
+    n_terms = sum(len(a) for a in (p.bond_idx1, p.angle_idx1, p.strbend_idx1, p.oop_idx1, p.torsion_idx1))
+    assert p.n_atoms == 16 and n_terms > 12 * p.n_atoms
+    kw = dict(max_iters=40, grad_tol=1e-4, use_lbfgs=use_lbfgs, ls_grad=True, lbfgs_m=8)
+    few = engine.NkRunner(engine.device_batch([p], [2]), **kw).run(torch.from_numpy(x).cuda())
+    many = engine.NkRunner(engine.device_batch([p], [600]), **kw).run(torch.from_numpy(np.tile(x, 300)).cuda())
+    torch.cuda.synchronize()
+    assert torch.equal(few.x.repeat(300), many.x) and torch.equal(few.energy.repeat(300), many.energy)
+    assert torch.equal(few.counters.repeat(300, 1), many.counters)
