@@ -44,7 +44,8 @@ enum mmffhip_algo { MMFFHIP_BFGS = 0, MMFFHIP_LBFGS = 1 };
  * upper triangle in LDS; GLOBAL = full matrix in HBM; GLOBAL_PACKED
  * = packed upper triangle in HBM (dense BFGS; L-BFGS treats it as GLOBAL); GLOBAL_SYM = one
  * 4x4 block per pair of row quads in HBM, half the bytes of GLOBAL (dense BFGS; L-BFGS treats
- * it as GLOBAL) */
+ * it as GLOBAL). A batch of at most one conformer per compute unit keeps its L-BFGS history in
+ * LDS where it fits, also when GLOBAL is asked for: results are the same */
 enum mmffhip_hess_place {
   MMFFHIP_HESS_AUTO = 0,
   MMFFHIP_HESS_LDS = 1,
@@ -97,7 +98,10 @@ typedef struct {
   int32_t lbfgs_m;     /* history length for MMFFHIP_LBFGS (reference nk kernel uses 8) */
   int32_t hess_place;  /* mmffhip_hess_place */
   int32_t block;       /* threads per workgroup, a multiple of 64 up to 1024 with an instantiated
-                          kernel for (algo, placement, staging); 0 = plan default */
+                          kernel for (algo, placement, staging); 0 = plan default. With
+                          table_lds_bytes > 0, a batch of at most one conformer per compute unit
+                          may be launched with three times as many (the rest help evaluate;
+                          same results) */
   int32_t ls_grad;     /* 1: evaluate E+G at every line-search trial (saves the separate
                           gradient pass when the first trial is accepted) */
   const float *precond;  /* optional per-atom 3x3 initial inverse-Hessian blocks, 9 floats per

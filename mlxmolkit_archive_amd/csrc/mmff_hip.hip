@@ -1976,10 +1976,13 @@ size_t mm_lds(int nr, int mx, int m, bool hl) {
 // the workspace, which the next launch reads); from memory, each of an iteration's 2 len + 1
 // dependent passes waited for its loads. Each lane meets only its own coordinates of it, so it
 // needs no barrier. 128 registers put four workgroups on a CU. 1,000 conformers of 69 atoms on
-// average, 200 + 50 iterations: 7.4 ms; 9.1 ms with three workgroups per CU, 10.5 ms with the
-// history in memory too. Measured and dropped: the recursion in one wave while the others wait
-// (the same sums without barriers: 7.6 ms, and 3.53 against 2.75 ms for 60 conformers), and one
-// 64-thread workgroup per conformer (12.1 ms).
+// average, 200 + 50 iterations: 6.28 ms, 10.7 ms with the history read from memory and one loop
+// over all term types. Of that, measured before the reductions by readlane and the spread terms:
+// 7.4 ms; 9.1 ms with three workgroups per CU, 10.5 ms with the history in memory. Dropped: the
+// recursion in one wave while the others wait (the same sums without barriers: 7.6 against 7.4 ms,
+// and 3.53 against 2.75 ms for 60 conformers), and one 64-thread workgroup per conformer (12.1 ms).
+// What bounds it: the 2 len + 1 passes of an iteration, each a block reduction (a barrier and a
+// wave's latency), then the evaluation's vector instructions.
 // NR: threads of the workgroup. The first 256 do everything but the evaluation, which all share
 // (1,024 for batches of at most one conformer per CU; 60 ragged conformers, 100 + 25 iterations:
 // 2.59 -> 2.16 ms).
@@ -2417,7 +2420,8 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
   // they are). The bonded terms' energies take a word each; a bonded term has at least 12 table
   // bytes, so table_lds_bytes bounds their number. Ten conformers of 48 atoms, BFGS,
   // host work included: 4.28 -> 3.99 ms; 221 chains of 199-329 atoms, L-BFGS: 180 -> 127 ms (151 with
-  // the history in LDS alone).
+  // the history in LDS alone); with the bonded tasks' spread terms 3.95 and 116 ms. Above one
+  // conformer per CU the waves of other conformers fill the CU and helpers would only displace them.
   if (b->n_confs <= di.n_cu && o->table_lds_bytes > 0) {
     const int eb = (o->table_lds_bytes / 12 + 64) & ~63;
     const struct {

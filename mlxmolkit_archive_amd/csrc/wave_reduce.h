@@ -30,10 +30,10 @@ __device__ __forceinline__ float dpp_f(float v) {
 // Sums (or maxima) of K values per lane over a wave at once. At each butterfly step a lane keeps
 // one of two values and sends the other to its partner, so the values left halve from step to
 // step instead of each going through all steps: 69 instructions for K = 8, against 248 for
-// eight separate wsum (of 16-28 per value, a third of them DPP moves). Lane bits 0-2 end up
-// selecting the value: value q is in lanes l with (l & (KP - 1)) == q. Each value's additions
-// pair the same lanes in the same order as wsum's (IEEE addition commutes), so the result has
-// the same bits.
+// eight separate butterflies (of 16-28 per value, a third of them DPP moves). Lane bits 0-2 end
+// up selecting the value: value q is in lanes l with (l & (KP - 1)) == q. Each value's additions
+// pair the same lanes in the same order as in a butterfly of its own (IEEE addition commutes), so
+// the result has the same bits.
 template <bool MAX>
 __device__ __forceinline__ double red_op(double a, double b) {
   return MAX ? fmax(a, b) : a + b;
