@@ -30,14 +30,6 @@ constexpr int MLP_OUT = 6;
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-__device__ __forceinline__ short to_bf16(float f) {
-  // round to nearest even
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7f800000u) == 0x7f800000u) return (short)(u >> 16);  // inf / nan
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (short)(u >> 16);
-}
-
 __device__ __forceinline__ float softplus_eps(float v) {
   return (v > 20.f ? v : log1pf(expf(v))) + 1e-3f;
 }
@@ -69,8 +61,11 @@ struct MlpW {
 // strides of 58 and 34 words put the 32 rows of an 8-byte operand read in 32 different bank pairs.
 // v_mfma_f32_32x32x8_bf16 operand layout (wave64): lane l supplies A[l%32][4*(l/32)+0..3]
 // and B[4*(l/32)+0..3][l%32]; it receives D[8*(r/4) + 4*(l/32) + r%4][l%32], r = 0..15.
-// 500,003 atoms: 69 us (3.3 TB/s of features and blocks); 326 us with 4-byte feature loads and
-// units in lanes, 134 us with 16-byte loads and units in lanes.
+// The weights and the first tile are loaded all at once before anything waits: 32 atoms take 5.9 us
+// from one launch to the next, 12.6 us with the weights laid out a word at a time.
+// 500,003 atoms, launches back to back: 51 us (4.4 TB/s of features and blocks; a copy reaches 4.8),
+// 62 us with the weights a word at a time. One call: 326 us with 4-byte feature loads and units in
+// lanes, 134 us with 16-byte loads and units in lanes, 69 us with the weights a word at a time, 50 us now.
 constexpr int INF_WAVES = 4;
 constexpr int INF_LDX = 116, INF_LDH = 68;  // row strides (bf16) of features and hidden units
 constexpr int INF_WAVE_SHORTS = 32 * INF_LDX + 32 * INF_LDH + 2 * 32 * 9;  // features, hidden, blocks (f32)
@@ -129,16 +124,52 @@ __global__ void __launch_bounds__(64 * INF_WAVES, 2)
   short* s3 = s2 + 64 * INF_LDH;             // W3 [32][INF_LDH], rows 6..31 zero
   float* bias = (float*)(s3 + 32 * INF_LDH); // b1, b2, b3 padded to 32
   short* tiles = (short*)(bias + 160);
+  const int n_tiles = (n_atoms + 31) / 32, step = gridDim.x * INF_WAVES;
+  int t = blockIdx.x * INF_WAVES + wv;
+  float4 f[INF_VEC];
+  // Lanes past the last atom read the last word again: a row only reaches its own atom's outputs,
+  // and those past n_atoms are not stored. (A load under a condition of its own is waited for.)
+  auto fetch = [&](int tile) {
+    const int last = min(32, n_atoms - tile * 32) * (MLP_IN / 4) - 1;
+    const float4* src = (const float4*)feat + (size_t)tile * (32 * MLP_IN / 4);
+#pragma unroll
+    for (int v = 0; v < INF_VEC; v++) {
+      const int i = min(v * 64 + lane, last);
+      if (VEC) {
+        f[v] = src[i];
+      } else {
+        const float* p = (const float*)src + 4 * i;
+        f[v] = make_float4(p[0], p[1], p[2], p[3]);
+      }
+    }
+  };
+  if (t < n_tiles) fetch(t);  // in flight while the weights are laid out
   bf16x4 w1a[MLP_KPAD / 8], w1b[MLP_KPAD / 8];
   {
     short* s1 = tiles;
-    for (int i = tid; i < 64 * MLP_KPAD; i += blockDim.x) {
-      const int o = i / MLP_KPAD, k = i % MLP_KPAD;
-      s1[o * INF_LDX + k] = to_bf16(k < MLP_IN ? W.w1[o * MLP_IN + k] : 0.f);
+    // all loads first: one latency instead of one per few words (the launch's fixed cost)
+    constexpr int N1 = 64 * MLP_IN / 4, V1 = (N1 + 64 * INF_WAVES - 1) / (64 * INF_WAVES), V2 = 64 * 64 / 4 / (64 * INF_WAVES);
+    auto word = [](const float* w, int i) { return make_float4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]); };
+    auto put = [](short* d, float4 v) { *(uint2*)d = make_uint2(pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)); };
+    float4 u1[V1], u2[V2];
+#pragma unroll
+    for (int v = 0; v < V1; v++) u1[v] = word(W.w1, min(v * 64 * INF_WAVES + tid, N1 - 1));
+#pragma unroll
+    for (int v = 0; v < V2; v++) u2[v] = word(W.w2, v * 64 * INF_WAVES + tid);
+    const float4 u3 = word(W.w3, min(tid, MLP_OUT * 16 - 1));
+#pragma unroll
+    for (int v = 0; v < V1; v++) {
+      const int i = min(v * 64 * INF_WAVES + tid, N1 - 1), o = i / (MLP_IN / 4);
+      put(s1 + o * INF_LDX + 4 * (i - o * (MLP_IN / 4)), u1[v]);
     }
-    for (int i = tid; i < 64 * 64; i += blockDim.x) s2[(i >> 6) * INF_LDH + (i & 63)] = to_bf16(W.w2[i]);
-    for (int i = tid; i < 32 * 64; i += blockDim.x)
-      s3[(i >> 6) * INF_LDH + (i & 63)] = to_bf16(i < MLP_OUT * 64 ? W.w3[i] : 0.f);
+    if (tid < 128) put(s1 + (tid >> 1) * INF_LDX + MLP_IN + 4 * (tid & 1), make_float4(0.f, 0.f, 0.f, 0.f));
+#pragma unroll
+    for (int v = 0; v < V2; v++) {
+      const int i = v * 64 * INF_WAVES + tid;
+      put(s2 + (i >> 4) * INF_LDH + 4 * (i & 15), u2[v]);
+    }
+    for (int i = tid; i < 32 * 16; i += 64 * INF_WAVES)
+      put(s3 + (i >> 4) * INF_LDH + 4 * (i & 15), i < MLP_OUT * 16 ? u3 : make_float4(0.f, 0.f, 0.f, 0.f));
     if (tid < 160) bias[tid] = tid < 64 ? W.b1[tid] : tid < 128 ? W.b2[tid - 64] : tid < 128 + MLP_OUT ? W.b3[tid - 128] : 0.f;
     __syncthreads();
     const short* p = s1 + c32 * INF_LDX + (lane >> 5) * 4;
@@ -161,27 +192,9 @@ __global__ void __launch_bounds__(64 * INF_WAVES, 2)
   float* blk = (float*)(hid + 32 * INF_LDH);  // outputs [32][8], then blocks [32][9]
   for (int i = lane; i < 32 * (MLP_KPAD - MLP_IN); i += 64)
     act[(i >> 3) * INF_LDX + MLP_IN + (i & 7)] = 0;  // the padding columns of the first layer
-  const int n_tiles = (n_atoms + 31) / 32, step = gridDim.x * INF_WAVES;
-  int t = blockIdx.x * INF_WAVES + wv;
-  float4 f[INF_VEC];
-  auto fetch = [&](int tile) {
-    const size_t left = ((size_t)n_atoms - (size_t)tile * 32) * (MLP_IN / 4);  // 16-byte words to the end
-    const float4* src = (const float4*)feat + (size_t)tile * (32 * MLP_IN / 4);
-#pragma unroll
-    for (int v = 0; v < INF_VEC; v++) {
-      const int i = v * 64 + lane;
-      if (VEC) {
-        f[v] = (size_t)i < left ? src[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-      } else {
-        const float* p = (const float*)src + 4 * i;
-        f[v] = (size_t)i < left ? make_float4(p[0], p[1], p[2], p[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-    }
-  };
-  if (t < n_tiles) fetch(t);
   for (; t < n_tiles; t += step) {
     const int a0 = t * 32;
-    // features of 32 atoms -> bf16 tile (rows past n_atoms are zero)
+    // features of 32 atoms -> bf16 tile
 #pragma unroll
     for (int v = 0; v < INF_VEC; v++) {
       const int i = v * 64 + lane, r = i / (MLP_IN / 4), k = 4 * (i - r * (MLP_IN / 4));
