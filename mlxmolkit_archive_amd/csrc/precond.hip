@@ -257,7 +257,9 @@ __global__ void __launch_bounds__(64 * INF_WAVES, 2)
 // is deterministic. Row strides are 4 x odd words, so the operand reads (16 rows x 4 columns)
 // touch 64 different banks.
 //
-// Measured at 8,192 atoms: 38 us a step, launches and allocations included, against 2.90 ms with
+// Measured at 8,192 atoms: 32 us a step, launches and allocations included (38 us with the weights
+// and features brought into LDS a word at a time: most workgroups take one tile, so that latency is
+// theirs in full), against 2.90 ms with
 // one lane per atom in the layers and one lane per parameter in the weight gradients (2.53 ms
 // of it a serial walk over the atoms on 44 of 256 CUs). 64-atom tiles put the 8,192-atom
 // mini-batch on 128 CUs; 32-atom ones would use all 256 but double the partial sums (11 MB).
@@ -322,22 +324,55 @@ __global__ void __launch_bounds__(TR_NT) k_mlp_train(MlpW W, const float* __rest
   float* w2 = w1 + 64 * LDX;
   float* w3 = w2 + 64 * LDH;            // rows 6..15 zero
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  for (int i = tid; i < NP_W1; i += TR_NT) w1[(i / MLP_IN) * LDX + i % MLP_IN] = W.w1[i];
-  for (int i = tid; i < NP_W2; i += TR_NT) w2[(i >> 6) * LDH + (i & 63)] = W.w2[i];
-  for (int i = tid; i < 16 * 64; i += TR_NT) w3[(i >> 6) * LDH + (i & 63)] = i < NP_W3 ? W.w3[i] : 0.f;
+  const int tiles = (n_atoms + TR_ATOMS - 1) / TR_ATOMS;
+  // All of a thread's weight and feature words are loaded before the first is stored: one latency
+  // instead of one per few words. Features past the last atom read its last word again and become
+  // zeros on the way into LDS.
+  auto word = [](const float* p, int i) { return make_float4(p[4 * i], p[4 * i + 1], p[4 * i + 2], p[4 * i + 3]); };
+  constexpr int NX = TR_ATOMS * MLP_IN / 4, VX = (NX + TR_NT - 1) / TR_NT;  // words of a tile's features (and of W1)
+  static_assert(TR_ATOMS == 64 && NP_W1 == TR_ATOMS * MLP_IN && NP_W2 == 8 * TR_NT, "word counts");
+  float4 fx[VX];
+  auto fetch = [&](int t) {
+    const int last = min(TR_ATOMS, n_atoms - t * TR_ATOMS) * (MLP_IN / 4) - 1;
+    const float* src = feat + (size_t)t * TR_ATOMS * MLP_IN;
+#pragma unroll
+    for (int v = 0; v < VX; v++) fx[v] = word(src, min(v * TR_NT + tid, last));
+  };
+  {
+    float4 u1[VX], u2[2], u3;
+#pragma unroll
+    for (int v = 0; v < VX; v++) u1[v] = word(W.w1, min(v * TR_NT + tid, NX - 1));
+#pragma unroll
+    for (int v = 0; v < 2; v++) u2[v] = word(W.w2, v * TR_NT + tid);
+    u3 = word(W.w3, min(tid, NP_W3 / 4 - 1));
+    if (blockIdx.x < tiles) fetch(blockIdx.x);
+#pragma unroll
+    for (int v = 0; v < VX; v++) {
+      const int i = min(v * TR_NT + tid, NX - 1), o = i / (MLP_IN / 4);
+      *(float4*)(w1 + o * LDX + 4 * (i - o * (MLP_IN / 4))) = u1[v];
+    }
+#pragma unroll
+    for (int v = 0; v < 2; v++) {
+      const int i = v * TR_NT + tid;
+      *(float4*)(w2 + (i >> 4) * LDH + 4 * (i & 15)) = u2[v];
+    }
+    if (tid < 16 * 16) *(float4*)(w3 + (tid >> 4) * LDH + 4 * (tid & 15)) = tid < NP_W3 / 4 ? u3 : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
   const int rt = wv & 3, half = wv >> 2;      // 16-atom row tile and column half of a layer
   const int row = rt * 16, c16 = lane & 15, q = lane >> 4;
   f64x4 g[6];                                 // weight-gradient tiles of this wave
 #pragma unroll
   for (int i = 0; i < 6; i++) g[i] = f64x4{0.0, 0.0, 0.0, 0.0};
   double gb = 0.0;                            // bias gradient of thread tid (b1, b2, b3)
-  const int tiles = (n_atoms + TR_ATOMS - 1) / TR_ATOMS;
   for (int t = blockIdx.x; t < tiles; t += gridDim.x) {
     const int a0 = t * TR_ATOMS, na = min(TR_ATOMS, n_atoms - a0);
-    for (int i = tid; i < TR_ATOMS * MLP_IN; i += TR_NT) {
-      const int r = i / MLP_IN;
-      xs[r * LDX + i - r * MLP_IN] = r < na ? feat[(size_t)a0 * MLP_IN + i] : 0.f;
+#pragma unroll
+    for (int v = 0; v < VX; v++) {
+      const int i = v * TR_NT + tid, r = i / (MLP_IN / 4);
+      if (i < NX)
+        *(float4*)(xs + r * LDX + 4 * (i - r * (MLP_IN / 4))) = r < na ? fx[v] : make_float4(0.f, 0.f, 0.f, 0.f);
     }
+    if (t + gridDim.x < tiles) fetch(t + gridDim.x);
     __syncthreads();
     // forward; a layer's output tile has its biases as the start of the sums
     auto layer_out = [&](f32x4 acc, float* z, int ld, int n0) {
