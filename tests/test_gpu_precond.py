@@ -115,6 +115,23 @@ def test_mlp_inference_tiles_and_alignment(n):
     assert np.median(err) < 1e-2 and err.max() < 5e-2, (n, np.median(err), err.max())
 
 
+@pytest.mark.parametrize("n", [1, 65, 16385])
+def test_mlp_parameters_and_features_off_a_16_byte_boundary(n):
+    """Weights and features are read four words at a time: parameters and features one float past
+    a 16-byte boundary give the same bits in training and inference."""
+    m = _model(11)
+    f, g = torch.from_numpy(_feat(n, 200 + n)).cuda(), np.random.default_rng(n)
+    t = torch.from_numpy(g.normal(0, 0.5, (n, 9)).astype(np.float32)).cuda()
+    want = (*m.loss_grad(f, t), m.blocks(f))
+    f_off = torch.empty(n * mo.N_IN + 1, dtype=torch.float32, device="cuda")[1:].view(n, mo.N_IN)
+    p_off = torch.empty(m.params.numel() + 1, dtype=torch.float32, device="cuda")[1:]
+    m.params = p_off.copy_(m.params)
+    got = (*m.loss_grad(f_off.copy_(f), t), m.blocks(f_off))
+    torch.cuda.synchronize()
+    assert f_off.data_ptr() % 16 == 4 and p_off.data_ptr() % 16 == 4
+    assert all(torch.equal(a, b) for a, b in zip(want, got))
+
+
 def test_hessian_blocks_match_oracle_finite_differences(small_wl):
     from mlxmolkit_archive_amd import engine
     from mlxmolkit_archive_amd.precond import hessian_diag_blocks
