@@ -22,6 +22,7 @@
 #include <string>
 #include <type_traits>
 
+#include "bonded_windows.h"
 #include "mmff_hip.h"
 #include "mmff_terms.h"
 #include "wave_reduce.h"
@@ -519,7 +520,7 @@ __device__ __forceinline__ double eval_tasks(const TView& V, const MolDesc& m, c
 
 // The bonded terms of eval_tasks for the minimizers that compare energies trial by trial, with
 // the energy bits of eval_terms' generic loop over NT lanes: every task writes its terms' FP32
-// energies to eb (eb_n >= 64 floats of LDS) under eval_terms' numbering, and lane t < NT adds up
+// energies to eb (eb_n >= BONDED_WINDOW_MIN floats of LDS) under eval_terms' numbering, and lane t < NT adds up
 // numbers t, t + NT, ... in order. Gradient sums are exact in any order, so a task is free to take
 // every T-th term of its type (T tasks): terms follow their central atoms in the tables, and 64
 // consecutive ones send up to 27 lanes' atomics to one LDS word. With the generic loop the bonded
@@ -549,17 +550,7 @@ __device__ __forceinline__ Window bonded_tasks(const TView& V, const MolDesc& m,
   Window win{0, c5};
   const bool one = !EV || c5 <= eb_n;
   for (;;) {
-    if (EV && c5 - win.s > eb_n) {
-      // up to the last task that fits
-      const int base[6] = {0, c1, c2, c3, c4, c5}, lim = win.s + eb_n;
-      win.end = win.s;
-#pragma unroll
-      for (int k = 0; k < 5; k++)
-        if (lim > base[k] && win.s < base[k + 1])
-          win.end = lim >= base[k + 1] ? base[k + 1] : base[k] + ((lim - base[k]) & ~63);
-    } else {
-      win.end = c5;
-    }
+    win.end = EV ? bonded_window_end({0, c1, c2, c3, c4, c5}, win.s, eb_n) : c5;
     for (int k = 0; k * NW < t5; k++) {
       const int t = (k & 1) ? (k + 1) * NW - 1 - w : k * NW + w;
       auto mine = [&](int first, int end, int base, int n, int& u) {
@@ -946,7 +937,10 @@ __host__ __device__ inline size_t nk_lds_bytes(int algo, int hm, int nt, int max
   b += (size_t)max_n * 8;  // gradient accumulators
   b += (size_t)max_n * 4 * 4;   // xs, d, xo, hd
   b += (size_t)max_n * 8;       // g, dg
-  if (algo == MMFFHIP_BFGS || help == 1) b += (size_t)max_n * 16;  // a pending update: s, h, alpha, beta
+  if (algo == MMFFHIP_BFGS)
+    b += (size_t)max_n * 16;  // a pending update: s, h, alpha, beta
+  else if (help == 1)
+    b += (size_t)lbfgs_eb_floats(max_n) * 4;  // bonded energies
   if (algo == MMFFHIP_BFGS && (hm == 1 || hm == 3)) b += (size_t)(hpend_for(nt) - 1) * max_n * 16;  // more pending updates
   if (algo == MMFFHIP_BFGS && hm == 3) b += nw * (size_t)sym_acc_floats(max_n) * 4;
   if (algo == MMFFHIP_LBFGS) {
@@ -1016,7 +1010,7 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
   auto up_plane = [&](int k, int c) { return UP + (size_t)(4 * k + c) * mn; };  // c: s, h, alpha, beta
   auto sh_slot = [&](int k) { return (float2*)up_plane(k, 0); };
   auto ab_slot = [&](int k) { return (float2*)up_plane(k, 2); };
-  float* dgv = ALGO == MMFFHIP_BFGS || HELP == 1 ? UP + (size_t)NPM * 4 * mn : UP;  // last change of g
+  float* dgv = UP + (ALGO == MMFFHIP_BFGS ? NPM * 4 * mn : HELP == 1 ? lbfgs_eb_floats(mn) : 0);  // last change of g
   float* hd = dgv + mn;  // H dg (BFGS) / two-loop q (L-BFGS)
   float* big = hd + mn;
   float* H = HLDS ? big : P.hglob + (size_t)blockIdx.x * P.slot_floats;
@@ -1026,11 +1020,11 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
   const int sacc_w = sym_acc_floats(mn);
   if (SYM) big_floats = (size_t)NW * sacc_w;
   // During an evaluation the bonded terms' energies lie in dgv, hd and the accumulators (at least
-  // 12 floats per atom, which hold all but a cage molecule's at once), none of which is live then;
-  // L-BFGS has that room where BFGS keeps its update.
+  // 12 floats per atom, which hold all but a cage molecule's at once, and never less than a task's
+  // 64), none of which is live then; L-BFGS has that room where BFGS keeps its update.
   constexpr bool ORDERED = HELP == 1 && (SYM || ALGO == MMFFHIP_LBFGS);
   float* ebuf = SYM ? dgv : UP;
-  const int ebuf_n = SYM ? 2 * mn + NW * sacc_w : 4 * mn;
+  const int ebuf_n = SYM ? 2 * mn + NW * sacc_w : lbfgs_eb_floats(mn);
   unsigned char* tstage = (unsigned char*)(big + big_floats);
   float* ring = (float*)(tstage + P.tbytes);  // HELP: pair energies, then bonded energies
   float* eb = ring + help_ring_floats<NT>(HELP);

@@ -425,3 +425,20 @@ def test_cage_molecule_energies_in_windows(use_lbfgs):
     torch.cuda.synchronize()
     assert torch.equal(few.x.repeat(300), many.x) and torch.equal(few.energy.repeat(300), many.energy)
     assert torch.equal(few.counters.repeat(300, 1), many.counters)
+
+
+def test_bonded_windows_of_the_smallest_molecules():
+    """A two-atom molecule whose bond is listed 100 times: more terms of one type than the LDS
+    words that 12 per atom would give an L-BFGS launch, whose energies then pass in windows of
+    64. Bit for bit the results of a batch small enough for helper threads, which hold them all."""
+    from mlxmolkit_archive_amd import engine
+    _, p, x = conftest.mol_params("[H][H]", seed=4, k=2)
+    for f in ("bond_idx1", "bond_idx2", "bond_kb", "bond_r0"):
+        setattr(p, f, np.repeat(getattr(p, f), 100))
+    assert p.n_atoms == 2 and len(p.bond_idx1) == 100
+    kw = dict(max_iters=20, grad_tol=1e-4, use_lbfgs=True, ls_grad=True, lbfgs_m=8)
+    few = engine.NkRunner(engine.device_batch([p], [2]), **kw).run(torch.from_numpy(x).cuda())
+    many = engine.NkRunner(engine.device_batch([p], [600]), **kw).run(torch.from_numpy(np.tile(x, 300)).cuda())
+    torch.cuda.synchronize()
+    assert torch.equal(few.x.repeat(300), many.x) and torch.equal(few.energy.repeat(300), many.energy)
+    assert torch.equal(few.counters.repeat(300, 1), many.counters)
