@@ -218,7 +218,8 @@ int mmffhip_mlp_dims(int32_t *n_in, int32_t *n_hidden, int32_t *n_out, int32_t *
 int mmffhip_mlp_infer(const float *params, const float *feat, int32_t n_atoms, float *blocks, void *stream);
 /* Training: FP32 forward and backward of sum_a weight_a * ||block_a - target_a||_F^2.
  * loss (optional): per-atom unweighted loss; grad (optional): n_params floats, the gradient
- * summed over atoms in a fixed order (deterministic); weight may be NULL (all ones). */
+ * summed over atoms in a fixed order (deterministic); weight may be NULL (all ones). The workspace
+ * of n_atoms serves every smaller batch too. */
 int mmffhip_mlp_workspace(int32_t n_atoms, size_t *bytes);
 int mmffhip_mlp_forward_backward(const float *params, const float *feat, int32_t n_atoms, const float *target,
                                  const float *weight, float *blocks, float *loss, float *grad, void *workspace,

@@ -276,12 +276,15 @@ constexpr size_t TR_LDS = (size_t)TR_LDS_FLOATS * 4;
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
+inline int train_tiles(int n_atoms) { return n_atoms / TR_ATOMS + (n_atoms % TR_ATOMS > 0); }
 // Workgroups of the training kernel: at most one per CU's worth, with tiles shared out evenly.
 inline int train_grid(int n_atoms) {
-  const int tiles = (n_atoms + TR_ATOMS - 1) / TR_ATOMS;
+  const int tiles = train_tiles(n_atoms);
   const int rounds = (tiles + TR_MAX_GRID - 1) / TR_MAX_GRID;
   return rounds > 0 ? (tiles + rounds - 1) / rounds : 0;
 }
+// Their partial sums, with room to start them at a 256-byte boundary
+inline size_t train_ws_bytes(int workgroups) { return (size_t)workgroups * MLP_NPARAM * sizeof(double) + 256; }
 
 // One 16 x 16 tile of A (rows of `a`, stride lda) times the transpose of B (rows of `b`, stride
 // ldb) over K columns, added to acc. v_mfma_f32_16x16x4: lane l supplies A[l%16][l/16] and
@@ -578,7 +581,10 @@ int mmffhip_mlp_infer(const float* params, const float* feat, int32_t n_atoms, f
 
 int mmffhip_mlp_workspace(int32_t n_atoms, size_t* bytes) {
   if (!bytes || n_atoms < 0) return perr(MMFFHIP_ERR_ARG, "bad arguments");
-  *bytes = (size_t)train_grid(n_atoms) * MLP_NPARAM * sizeof(double) + 256;
+  // The tiles are shared out evenly, so more atoms can take fewer workgroups (16,384: 256, 16,385:
+  // 129). The size asked for does not follow: room for n_atoms is room for every smaller batch.
+  const int tiles = train_tiles(n_atoms);
+  *bytes = train_ws_bytes(tiles < TR_MAX_GRID ? tiles : TR_MAX_GRID);
   return MMFFHIP_OK;
 }
 
@@ -587,17 +593,14 @@ int mmffhip_mlp_forward_backward(const float* params, const float* feat, int32_t
                                  size_t workspace_bytes, void* stream) {
   if (n_atoms <= 0) return perr(MMFFHIP_ERR_ARG, "n_atoms must be positive");
   if (!params || !feat || !target || !workspace) return perr(MMFFHIP_ERR_ARG, "params, feat, target, workspace required");
-  size_t need = 0;
-  mmffhip_mlp_workspace(n_atoms, &need);
-  if (workspace_bytes < need) return perr(MMFFHIP_ERR_SIZE, "workspace too small");
+  const int grid = train_grid(n_atoms);
+  if (workspace_bytes < train_ws_bytes(grid)) return perr(MMFFHIP_ERR_SIZE, "workspace too small");
   if (hipFuncSetAttribute((const void*)&k_mlp_train, hipFuncAttributeMaxDynamicSharedMemorySize, (int)TR_LDS) !=
       hipSuccess)
     return perr(MMFFHIP_ERR_HIP, "hipFuncSetAttribute failed");
   const MlpW W = mlp_weights(params);
-  // the partial sums start at the first 256-byte boundary (the queried size has room for that)
   double* part = grad ? (double*)(((uintptr_t)workspace + 255) & ~(uintptr_t)255) : nullptr;
   hipStream_t s = (hipStream_t)stream;
-  const int grid = train_grid(n_atoms);
   hipLaunchKernelGGL(k_mlp_train, dim3(grid), dim3(TR_NT), TR_LDS, s, W, feat, n_atoms, target, weight, blocks, loss,
                      part);
   if (grad)

@@ -37,3 +37,18 @@ def test_oracle_is_not_linked_by_the_product():
     """The product library must not depend on the oracle in any form."""
     data = lib_path("libmmff_hip.so").read_bytes()
     assert b"oracle" not in data
+
+
+def test_training_workspace_grows_with_the_batch():
+    """A workspace allocated for the largest batch serves the smaller ones: the size never falls as
+    atoms are added, also where the tiles spread over fewer workgroups (16,384 -> 16,385 atoms)."""
+    L = _lib.load()
+    sizes = []
+    for n in [*range(0, 70), *range(63, 40000, 64), *range(64, 40000, 64), *range(65, 40000, 64), 2**31 - 1]:
+        b = ctypes.c_size_t()
+        assert L.mmffhip_mlp_workspace(n, ctypes.byref(b)) == 0
+        sizes.append((n, b.value))
+    sizes.sort()
+    assert all(a[1] <= b[1] for a, b in zip(sizes, sizes[1:]))
+    at = dict(sizes)
+    assert at[1] > at[0] and at[16384] == at[16385] and at[32768] == at[32769]
