@@ -129,7 +129,8 @@ int mmffhip_device_info(int32_t *n_cu, int32_t *n_xcd, int32_t *lds_bytes);
 
 /* Single-point energies and gradients. e_out: n_confs doubles. e_terms (optional):
  * 7 doubles per conformer {bond, angle, strbend, oop, torsion, vdw, ele}. g_out (optional):
- * float gradient in the coordinate layout. term_mask selects terms (bit k = term k). */
+ * float gradient in the coordinate layout. term_mask selects terms (bit k = term k).
+ * A conformer's results do not depend on the batch it is in. */
 int mmffhip_energy_grad(const mmffhip_batch *b, int family, int diel, const float *x, double *e_out,
                         double *e_terms, float *g_out, uint32_t term_mask, void *stream);
 

@@ -180,7 +180,7 @@ struct LdsAcc {
 // Term tables are read from global memory (L2-resident: shared by the molecule's
 // conformers); each lane prefetches its next term's indices and parameters before it
 // evaluates the current one, so table latency overlaps the term arithmetic.
-// Returns this lane's FP64 energy partial; per-term partials in et[7] when PT.
+// Returns this lane's FP64 energy partial.
 struct TermData {
   uint32_t a, b;  // packed atom indices
   float4 p;       // parameters
@@ -335,67 +335,56 @@ __device__ __forceinline__ TermData load_term(const TView& V, int t, int c1, int
   return d;
 }
 
+// One row of the pair table (its unused first parameter left out); 32-bit offsets from the
+// (uniform) table bases
+struct Pair {
+  uint32_t ij;
+  float eps, qq, ir;
+};
+__device__ __forceinline__ Pair load_pair(const TView& V, unsigned u) {
+  const float* q = (const float*)((const char*)V.pair_p + 16u * u);
+  return Pair{*(const uint32_t*)((const char*)V.pair_ij + 4u * u), q[1], q[2], q[3]};
+}
+
 // non-bonded pairs: two pairs per lane per step (independent dependency chains), the
 // next two loaded while the current two are computed. The loads are unconditional (index
 // clamped to the last pair; such duplicates are never used), so the wait before the
 // current pairs' use leaves the next pairs' loads in flight. Every step but the last is full
 // for all lanes, so the loop counts in scalar registers and masks nothing.
-template <int FAM, bool G, bool PT, int NT, bool EV>
-__device__ __forceinline__ double eval_pairs(const TView& TV, const MolDesc& m, const float* xs, LdsAcc<G>& acc,
-                                             int diel, uint32_t mask, double* et) {
-  if ((mask & 96u) && m.npair > 0) {
-    const float ke = (mask & 32u) ? 1.0f : 0.0f, kq = (mask & 64u) ? 1.0f : 0.0f;
-    const unsigned np = (unsigned)m.npair, last = np - 1;
-    struct Pair {
-      uint32_t ij;
-      float eps, qq, ir;
-    };
-    // 32-bit offsets from the (uniform) table bases
-    auto load = [&](unsigned u) {
-      u = min(u, last);
-      const float* q = (const float*)((const char*)TV.pair_p + 16u * u);
-      return Pair{*(const uint32_t*)((const char*)TV.pair_ij + 4u * u), q[1], q[2], q[3]};
-    };
-    double ev_acc = 0.0, ee_acc = 0.0;
-    auto term = [&](const Pair& p) {
-      float ev = 0.f, ee = 0.f;
-      t_pair<FAM, G, EV>(xs, acc, (int)(p.ij & 0xffff), (int)(p.ij >> 16), p.ir, ke * p.eps, kq * p.qq, diel, ev, ee);
-      // without per-term energies a pair's two parts are added in FP32 first (one rounding,
-      // as small as the parts' own), then to the lane's FP64 sum
-      if (PT) {
-        ev_acc += ev;
-        ee_acc += ee;
-      } else {
-        ev_acc += (double)(ev + ee);
-      }
-    };
-    unsigned u = threadIdx.x;
-    Pair pa = load(u), pb = load(u + NT);
-    for (unsigned left = (np - 1) / (2 * NT); left > 0; left--) {
-      const Pair na = load(u + 2 * NT), nb = load(u + 3 * NT);
-      term(pa);
-      term(pb);
-      pa = na;
-      pb = nb;
-      u += 2 * NT;
-    }
-    if (u < np) term(pa);
-    if (u + NT < np) term(pb);
-    if (PT) {
-      et[5] += ev_acc;
-      et[6] += ee_acc;
-    }
-    return ev_acc + ee_acc;
+template <int FAM, bool G, int NT, bool EV>
+__device__ __forceinline__ double eval_pairs(const TView& V, const MolDesc& m, const float* xs, LdsAcc<G>& acc,
+                                             int diel) {
+  if (m.npair <= 0) return 0.0;
+  const unsigned np = (unsigned)m.npair, last = np - 1;
+  double e = 0.0;
+  // a pair's two parts are added in FP32 first (one rounding, as small as the parts' own), then
+  // to the lane's FP64 sum
+  auto term = [&](const Pair& p) {
+    float ev = 0.f, ee = 0.f;
+    t_pair<FAM, G, EV>(xs, acc, (int)(p.ij & 0xffff), (int)(p.ij >> 16), p.ir, p.eps, p.qq, diel, ev, ee);
+    e += (double)(ev + ee);
+  };
+  unsigned u = threadIdx.x;
+  Pair pa = load_pair(V, min(u, last)), pb = load_pair(V, min(u + NT, last));
+  for (unsigned left = last / (2 * NT); left > 0; left--) {
+    const Pair na = load_pair(V, min(u + 2 * NT, last)), nb = load_pair(V, min(u + 3 * NT, last));
+    term(pa);
+    term(pb);
+    pa = na;
+    pb = nb;
+    u += 2 * NT;
   }
-  return 0.0;
+  if (u < np) term(pa);
+  if (u + NT < np) term(pb);
+  return e;
 }
 
 // PREF: load each bonded term's tables one step ahead (tables in global memory); with the
 // tables in LDS the loads are short and the prefetch only holds registers.
 // EV: the energies are used (otherwise only the gradient is).
-template <int FAM, bool G, bool PT, int NT, bool PREF = true, bool EV = true>
+template <int FAM, bool G, int NT, bool PREF, bool EV>
 __device__ __forceinline__ double eval_terms(const TView& TV, const MolDesc& m, const float* xs,
-                                             unsigned long long* gacc, int diel, uint32_t mask, double* et) {
+                                             unsigned long long* gacc, int diel) {
   LdsAcc<G> acc{gacc};
   double e = 0.0;
   // bonded terms (one generic loop, next term prefetched when PREF)
@@ -413,109 +402,216 @@ __device__ __forceinline__ double eval_terms(const TView& TV, const MolDesc& m, 
     const int i0 = (int)(cur.a & 0xffff), i1 = (int)(cur.a >> 16);
     const int i2 = (int)(cur.b & 0xffff), i3 = (int)(cur.b >> 16);
     if (t < c1) {
-      if (mask & 1u) {
-        const float v = t_bond<FAM, G>(xs, acc, i0, i1, cur.p.x, cur.p.y);
-        e += v;
-        if (PT) et[0] += v;
-      }
+      e += t_bond<FAM, G>(xs, acc, i0, i1, cur.p.x, cur.p.y);
     } else if (t < c2) {
-      if (mask & 2u) {
-        const float v = t_angle<FAM, G>(xs, acc, i0, i1, i2, cur.p.x, cur.p.y, i3 != 0);
-        e += v;
-        if (PT) et[1] += v;
-      }
+      e += t_angle<FAM, G>(xs, acc, i0, i1, i2, cur.p.x, cur.p.y, i3 != 0);
     } else if (t < c3) {
-      if (mask & 4u) {
-        const float v = t_strbend<FAM, G>(xs, acc, i0, i1, (int)cur.b, cur.p.x, cur.p.y, cur.p.z, cur.p.w, cur.q);
-        e += v;
-        if (PT) et[2] += v;
-      }
+      e += t_strbend<FAM, G>(xs, acc, i0, i1, (int)cur.b, cur.p.x, cur.p.y, cur.p.z, cur.p.w, cur.q);
     } else if (t < c4) {
-      if (mask & 8u) {
-        const float v = t_oop<FAM, G>(xs, acc, i0, i1, i2, i3, cur.p.x);
-        e += v;
-        if (PT) et[3] += v;
-      }
+      e += t_oop<FAM, G>(xs, acc, i0, i1, i2, i3, cur.p.x);
     } else {
-      if (mask & 16u) {
-        const float v = t_torsion<FAM, G>(xs, acc, i0, i1, i2, i3, cur.p.x, cur.p.y, cur.p.z);
-        e += v;
-        if (PT) et[4] += v;
-      }
+      e += t_torsion<FAM, G>(xs, acc, i0, i1, i2, i3, cur.p.x, cur.p.y, cur.p.z);
     }
     if (PREF) cur = nxt;
     t = tn;
   }
-  e += eval_pairs<FAM, G, PT, NT, EV>(TV, m, xs, acc, diel, mask, et);
-  return e;
+  return e + eval_pairs<FAM, G, NT, EV>(TV, m, xs, acc, diel);
 }
 
-// eval_terms for kernels whose results do not hang on the order of the energy sum (single points;
-// the descents, where the energy only guards): the bonded terms go to the waves in tasks of 64
-// terms of one type, the heaviest types first and the waves taken back and forth, so no wave runs
-// several types' code for parts of its lanes and the waves finish together. A task takes every
-// T-th term of its type (T tasks), because neighbouring terms share atoms and their lanes' atomics
-// would queue for the same LDS words. The minimizers that compare energies trial by trial use
-// bonded_tasks below. 12,139 ragged MEGA energies and gradients: generic loop 143 us, tasks of
-// consecutive terms 123, of spread terms 103; the Barzilai-Borwein descent of 1,000 conformers:
-// 6.08, 4.59, 4.00 ms; the lock-step L-BFGS: 7.00 and 6.28 ms.
-template <int FAM, bool G, bool PT, int NT>
-__device__ __forceinline__ double eval_tasks(const TView& V, const MolDesc& m, const float* xs,
-                                             unsigned long long* gacc, int diel, uint32_t mask, double* et) {
-  constexpr int NW = NT / 64;
+// The evaluation of the single points, the descent and the lock-step engine. Their workgroups have
+// 256 threads, or 1,024 for batches of at most one conformer per CU, and a conformer's results do
+// not depend on which: an energy is the sum over SUM_GROUPS groups of 256 lanes, each with a share
+// of the terms of its own. A workgroup of 256 threads does one group after another and adds up a
+// lane's four sums as it goes; one of 1,024 does the four at once and adds them in the same order
+// in LDS (combine_groups). (Gradient sums are exact in any order.)
+//
+// Bonded terms go to the groups' 16 waves in tasks of 64 terms of one type, the heaviest types
+// first and the waves taken back and forth, so no wave runs several types' code for parts of its
+// lanes and the waves finish together. A task takes every T-th term of its type (T tasks), because
+// neighbouring terms share atoms and their lanes' atomics would queue for the same LDS words. The
+// minimizers that compare energies trial by trial use bonded_tasks below. A group's pairs are a
+// quarter of the list, so one group after another is one walk over it.
+// 12,139 ragged MEGA energies and gradients: generic loop 143 us, tasks of consecutive terms 123, of
+// spread terms 103, without the sums of kinds 97.5; the Barzilai-Borwein descent of 1,000
+// conformers: 6.08, 4.59, 4.00 ms, with the sums by groups 4.07; the lock-step L-BFGS: 7.00, 6.28,
+// 6.37 ms.
+constexpr int SUM_LANES = 256, SUM_GROUPS = 4;
+
+// A lane's energy sums: bonded terms, pairs, and each kind of term when PT
+template <bool PT>
+struct LaneSums {
+  double b = 0.0, p = 0.0, kind[PT ? 7 : 1] = {};
+};
+
+// SEP: a pair's two parts go to FP64 sums of their own; otherwise they are added in FP32 first, as in
+// eval_pairs
+template <int FAM, bool G, bool SEP, bool PT, int NT>
+__device__ __forceinline__ LaneSums<PT> eval_tasks(const TView& V, const MolDesc& m, const float* xs,
+                                                   unsigned long long* gacc, int diel, uint32_t mask) {
+  static_assert(NT == SUM_LANES || NT == SUM_LANES * SUM_GROUPS, "one group after another, or all at once");
+  static_assert(SEP || !PT, "kinds are summed apart");
+  constexpr bool ALL = NT == SUM_LANES;
+  constexpr int GW = SUM_LANES / 64, NW = GW * SUM_GROUPS;
   LdsAcc<G> acc{gacc};
-  double e = 0.0;
+  LaneSums<PT> sum;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h0 = ALL ? 0 : w / GW, h1 = ALL ? SUM_GROUPS : h0 + 1, wg = w % GW;
   // first task of each type after the torsions
   const int t1 = (m.ntor + 63) >> 6, t2 = t1 + ((m.nsb + 63) >> 6), t3 = t2 + ((m.na + 63) >> 6),
             t4 = t3 + ((m.noop + 63) >> 6), t5 = t4 + ((m.nb + 63) >> 6);
-  for (int k = 0; k * NW < t5; k++) {
-    const int t = (k & 1) ? (k + 1) * NW - 1 - w : k * NW + w;
-    auto add = [&](int kind, float v) {
-      e += v;
-      if (PT) et[kind] += v;
+  auto tor = [&](int u) {
+    const uint2 ix = V.tor_idx[u];
+    const float4 p = V.tor_p[u];
+    return t_torsion<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff), (int)(ix.y >> 16),
+                             p.x, p.y, p.z);
+  };
+  auto sb = [&](int u) {
+    const uint2 ix = V.sb_idx[u];
+    const float4 p = V.sb_p[u];
+    return t_strbend<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)ix.y, p.x, p.y, p.z, p.w, V.sb_t0[u]);
+  };
+  auto ang = [&](int u) {
+    const uint2 ix = V.ang_idx[u];
+    const float2 p = V.ang_p[u];
+    return t_angle<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff), p.x, p.y,
+                           (ix.y >> 16) != 0);
+  };
+  auto oop = [&](int u) {
+    const uint2 ix = V.oop_idx[u];
+    return t_oop<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff), (int)(ix.y >> 16),
+                         V.oop_k[u]);
+  };
+  auto bond = [&](int u) {
+    const uint32_t ij = V.bond_ij[u];
+    const float2 p = V.bond_p[u];
+    return t_bond<FAM, G>(xs, acc, (int)(ij & 0xffff), (int)(ij >> 16), p.x, p.y);
+  };
+#pragma unroll 1
+  for (int h = h0; h < h1 && GW * h < t5; h++) {
+    int t = GW * h + ((h & 1) ? GW - 1 - wg : wg);  // a wave's tasks in this group: every NW-th from here
+    double e = 0.0;
+    // task t of kind c, whose tasks are first .. end - 1 and whose terms are n
+    auto one = [&](int c, int first, int end, int n, auto term, double& k) {
+      const int u = lane * (end - first) + (t - first);
+      if ((mask >> c & 1u) && u < n) {
+        const float v = term(u);
+        e += v;
+        if (PT) k += v;
+      }
     };
-    if (t < t1) {
-      const int u = lane * t1 + t;
-      if ((mask & 16u) && u < m.ntor) {
-        const uint2 ix = V.tor_idx[u];
-        const float4 p = V.tor_p[u];
-        add(4, t_torsion<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
-                                 (int)(ix.y >> 16), p.x, p.y, p.z));
-      }
-    } else if (t < t2) {
-      const int u = lane * (t2 - t1) + (t - t1);
-      if ((mask & 4u) && u < m.nsb) {
-        const uint2 ix = V.sb_idx[u];
-        const float4 p = V.sb_p[u];
-        add(2, t_strbend<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)ix.y, p.x, p.y, p.z, p.w,
-                                 V.sb_t0[u]));
-      }
-    } else if (t < t3) {
-      const int u = lane * (t3 - t2) + (t - t2);
-      if ((mask & 2u) && u < m.na) {
-        const uint2 ix = V.ang_idx[u];
-        const float2 p = V.ang_p[u];
-        add(1, t_angle<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff), p.x, p.y,
-                               (ix.y >> 16) != 0));
-      }
-    } else if (t < t4) {
-      const int u = lane * (t4 - t3) + (t - t3);
-      if ((mask & 8u) && u < m.noop) {
-        const uint2 ix = V.oop_idx[u];
-        add(3, t_oop<FAM, G>(xs, acc, (int)(ix.x & 0xffff), (int)(ix.x >> 16), (int)(ix.y & 0xffff),
-                             (int)(ix.y >> 16), V.oop_k[u]));
-      }
-    } else if (t < t5) {
-      const int u = lane * (t5 - t4) + (t - t4);
-      if ((mask & 1u) && u < m.nb) {
-        const uint32_t ij = V.bond_ij[u];
-        const float2 p = V.bond_p[u];
-        add(0, t_bond<FAM, G>(xs, acc, (int)(ij & 0xffff), (int)(ij >> 16), p.x, p.y));
+    if constexpr (PT) {
+      // a loop for each kind, so that one sum of kinds is in the making at a time
+      auto all = [&](int c, int first, int end, int n, auto term) {
+        double k = 0.0;
+        for (; t < end; t += NW) one(c, first, end, n, term, k);
+        sum.kind[c] += k;
+      };
+      all(4, 0, t1, m.ntor, tor);
+      all(2, t1, t2, m.nsb, sb);
+      all(1, t2, t3, m.na, ang);
+      all(3, t3, t4, m.noop, oop);
+      all(0, t4, t5, m.nb, bond);
+    } else {
+      double k;
+      for (; t < t5; t += NW) {
+        if (t < t1) one(4, 0, t1, m.ntor, tor, k);
+        else if (t < t2) one(2, t1, t2, m.nsb, sb, k);
+        else if (t < t3) one(1, t2, t3, m.na, ang, k);
+        else if (t < t4) one(3, t3, t4, m.noop, oop, k);
+        else one(0, t4, t5, m.nb, bond, k);
       }
     }
+    sum.b += e;
   }
-  return e + eval_pairs<FAM, G, PT, NT, true>(V, m, xs, acc, diel, mask, et);
+  if (!(mask & 96u) || m.npair <= 0) return sum;
+  // eval_pairs' walk, two pairs per lane and step
+  constexpr unsigned STEP = 2 * SUM_LANES;
+  const unsigned np = (unsigned)m.npair, last = np - 1;
+  auto row = [&](unsigned u) { return load_pair(V, min(u, last)); };
+  const float ke = (mask & 32u) ? 1.0f : 0.0f, kq = (mask & 64u) ? 1.0f : 0.0f;
+  // group h has the steps h * per .. (h + 1) * per
+  double sv = 0.0, se = 0.0;
+  auto term = [&](const Pair& p) {
+    float ev = 0.f, ee = 0.f;
+    t_pair<FAM, G, true>(xs, acc, (int)(p.ij & 0xffff), (int)(p.ij >> 16), p.ir, ke * p.eps, kq * p.qq, diel, ev, ee);
+    if (SEP) {
+      sv += ev;
+      se += ee;
+    } else {
+      sv += (double)(ev + ee);
+    }
+  };
+  auto close = [&]() {  // a group's sums are complete
+    sum.p += SEP ? sv + se : sv;
+    if (PT) {
+      sum.kind[5] += sv;
+      sum.kind[6] += se;
+    }
+    sv = se = 0.0;
+  };
+  const unsigned steps = last / STEP + 1, per = (steps + SUM_GROUPS - 1) / SUM_GROUPS;
+  unsigned s = min(h0 * per, steps);
+  const unsigned end = min(h1 * per, steps), full = min(end, steps - 1);
+  if (s < end) {
+    unsigned u = s * STEP + (threadIdx.x & (SUM_LANES - 1)), stop = ALL ? per : end;  // this group's end
+    Pair pa = row(u), pb = row(u + SUM_LANES);
+    for (;; stop += per) {
+      for (const unsigned lim = min(stop, full); s < lim; s++) {
+        const Pair na = row(u + STEP), nb = row(u + STEP + SUM_LANES);
+        term(pa);
+        term(pb);
+        pa = na;
+        pb = nb;
+        u += STEP;
+      }
+      if (!ALL || s < stop) break;  // the list's last step, if any is left, is this group's too
+      close();
+    }
+    if (s < end) {
+      if (u < np) term(pa);
+      if (u + SUM_LANES < np) term(pb);
+    }
+    close();
+  }
+  return sum;
+}
+
+// The groups' sums of K values, for the lanes of the first group (the others' are left as they
+// are). buf: LDS for `room` >= 1 values of EX_WORDS doubles at a time; everybody is done with
+// its earlier contents.
+constexpr int EX_WORDS = SUM_LANES * (SUM_GROUPS - 1);
+template <int NT, int K>
+__device__ __forceinline__ void combine_groups(double (&v)[K], double* buf, int room) {
+  if constexpr (NT > SUM_LANES) {
+    const int t = (int)threadIdx.x;
+    for (int k0 = 0; k0 < K; k0 += room) {
+      if (k0 > 0) __syncthreads();
+#pragma unroll
+      for (int k = 0; k < K; k++)
+        if (t >= SUM_LANES && k >= k0 && k < k0 + room) buf[(k - k0) * EX_WORDS + t - SUM_LANES] = v[k];
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < K; k++)
+        if (t < SUM_LANES && k >= k0 && k < k0 + room) {
+          const double* b = buf + (k - k0) * EX_WORDS + t;
+          v[k] = ((v[k] + b[0]) + b[SUM_LANES]) + b[2 * SUM_LANES];
+        }
+    }
+  }
+}
+// The energy, on every lane; includes a barrier behind the evaluation
+template <int NT, bool PT, class Red>
+__device__ __forceinline__ double group_energy(const LaneSums<PT>& s, double* buf, int room, Red& R) {
+  double v[2] = {s.b, s.p};
+  combine_groups<NT>(v, buf, room);
+  return R.sum(v[0] + v[1]);
+}
+// LDS bytes of an area of at least `bytes` that serves as combine_groups' buffer too: K values at
+// once, or one if that does not fit beside `rest` other bytes
+size_t ex_area(int nt, size_t bytes, int K, size_t rest, size_t limit) {
+  if (nt == SUM_LANES) return bytes;
+  const size_t one = EX_WORDS * sizeof(double);
+  return std::max(bytes, rest + std::max(bytes, K * one) <= limit ? K * one : one);
 }
 
 // The bonded terms of eval_tasks for the minimizers that compare energies trial by trial, with
@@ -617,7 +713,7 @@ __device__ __forceinline__ double eval_ordered(const TView& V, const MolDesc& m,
   LdsAcc<G> acc{gacc};
   double e = 0.0;
   const Window win = bonded_tasks<FAM, G, EV, NT, NT>(V, m, xs, acc, eb, eb_n, e);
-  const double pairs = eval_pairs<FAM, G, false, NT, EV>(V, m, xs, acc, diel, 0x7fu, nullptr);
+  const double pairs = eval_pairs<FAM, G, NT, EV>(V, m, xs, acc, diel);
   if (!EV) return 0.0;
   __syncthreads();
   ordered_sum<NT>(e, eb, win, (int)threadIdx.x);
@@ -811,19 +907,24 @@ __device__ __forceinline__ void hcol_update4(float* col, const float2* AB, float
   }
 }
 
+constexpr int RED_WORDS = 2 * (SUM_LANES / 64) * 8;  // doubles of a Reducer<SUM_LANES>
+
 // ------------------------------------------------------------------------------------
 // Kernel: single-point energy / gradient / per-term energies, one workgroup per conformer.
 // Replaces mmff_energy_grad_metal(_mega) (mmff_metal_kernel.py:713-775); the TG family is
 // what the nk kernel evaluates (mmff_bfgs_header.metal).
-template <int FAM, int NT>
-__global__ void __launch_bounds__(NT) k_energy_grad(KBatch B, const float* __restrict__ x, double* e_out,
-                                                    double* e_terms, float* g_out, uint32_t mask, int diel) {
+// xs_bytes: the positions' LDS, where the groups' sums meet once the positions are done with
+// The narrow kernels with kinds are held to 7 and 5 waves per SIMD (TG, MEGA), which they miss by a
+// register or two: 12,139 ragged MEGA energies with kinds 73.7 us, 80.1 at four
+template <int FAM, bool PT, int NT>
+__global__ void __launch_bounds__(NT, NT == 256 ? (FAM == FAM_TG ? 7 : 5) : 4) k_energy_grad(KBatch B, const float* __restrict__ x, double* e_out,
+                                                    double* e_terms, float* g_out, uint32_t mask, int diel,
+                                                    int xs_bytes) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int c = blockIdx.x;
   if (c >= B.n_confs) return;
-  constexpr int NW = NT / 64;
   double* red = (double*)smem;
-  unsigned long long* gacc = (unsigned long long*)(red + 16 * NW);
+  unsigned long long* gacc = (unsigned long long*)(red + RED_WORDS);
   const int mx = 3 * B.max_atoms;
   float* xs = (float*)(gacc + mx);
   const MolDesc m = load_desc(B.mol_desc + 16 * B.conf_mol[c]);
@@ -832,18 +933,21 @@ __global__ void __launch_bounds__(NT) k_energy_grad(KBatch B, const float* __res
   for (int i = threadIdx.x; i < n; i += NT) xs[i] = x[off + i];
   for (int i = threadIdx.x; i < n; i += NT) gacc[i] = 0ull;
   __syncthreads();
-  Reducer<NT> R{red, 0};
-  double et[7] = {0, 0, 0, 0, 0, 0, 0};
-  double e;
+  Reducer<SUM_LANES, 8, (NT > SUM_LANES)> R{red, 0};
+  LaneSums<PT> sum;
   if (g_out)
-    e = eval_tasks<FAM, true, true, NT>(global_view(B, m), m, xs, gacc, diel, mask, et);
+    sum = eval_tasks<FAM, true, true, PT, NT>(global_view(B, m), m, xs, gacc, diel, mask);
   else
-    e = eval_tasks<FAM, false, true, NT>(global_view(B, m), m, xs, gacc, diel, mask, et);
-  e = R.sum(e);  // includes the barrier that completes the gradient atomics
-  if (e_terms) {
-    double v4[4] = {et[0], et[1], et[2], et[3]};
+    sum = eval_tasks<FAM, false, true, PT, NT>(global_view(B, m), m, xs, gacc, diel, mask);
+  double* buf = (double*)xs;
+  const int room = xs_bytes / (EX_WORDS * (int)sizeof(double));
+  if (NT > SUM_LANES) __syncthreads();  // the positions give way to the sums
+  const double e = group_energy<NT>(sum, buf, room, R);
+  if constexpr (PT) {
+    combine_groups<NT>(sum.kind, buf, room);
+    double v4[4] = {sum.kind[0], sum.kind[1], sum.kind[2], sum.kind[3]};
     R.template run<4, 0>(v4);
-    double v3[4] = {et[4], et[5], et[6], 0.0};
+    double v3[4] = {sum.kind[4], sum.kind[5], sum.kind[6], 0.0};
     R.template run<4, 0>(v3);
     if (threadIdx.x == 0) {
       for (int k = 0; k < 4; k++) e_terms[7 * c + k] = v4[k];
@@ -1140,7 +1244,7 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
       else if constexpr (ORDERED)
         return eval_ordered<FAM_TG, G, EV, NT>(TV, m, xs, gacc, P.diel, ebuf, ebuf_n);
       else
-        return eval_terms<FAM_TG, G, false, NT, TL == 0, EV>(TV, m, xs, gacc, P.diel, 0x7fu, nullptr);
+        return eval_terms<FAM_TG, G, NT, TL == 0, EV>(TV, m, xs, gacc, P.diel);
     };
     const std::true_type yes;
     const std::false_type no;
@@ -1817,21 +1921,24 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
 
 // ------------------------------------------------------------------------------------
 // BB fused steepest descent, MEGA family: mmff_metal_kernel.py:845-1075.
-template <int NT>
-__global__ void __launch_bounds__(NT) k_bb_fused(KBatch B, const float* __restrict__ x_in, float* x_out,
-                                                 double* e_out, int max_it, float max_step, float grad_lr) {
+// NR: threads of the workgroup. The first 256 do everything but the evaluation, which all share.
+// g_bytes: the gradient's LDS, where the groups' sums meet during an evaluation.
+template <int NR>
+__global__ void __launch_bounds__(NR) k_bb_fused(KBatch B, const float* __restrict__ x_in, float* x_out,
+                                                 double* e_out, int max_it, float max_step, float grad_lr,
+                                                 int g_bytes) {
   extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int NW = NT / 64;
+  constexpr int NT = SUM_LANES;
   const int c = blockIdx.x;
   if (c >= B.n_confs) return;
-  const int tid = threadIdx.x;
-  const int mx = 3 * B.max_atoms;
+  const int tid = NR == NT || threadIdx.x < NT ? (int)threadIdx.x : 1 << 30;
+  const int mx = 3 * B.max_atoms, room = g_bytes / (EX_WORDS * (int)sizeof(double));
   double* red = (double*)smem;
-  unsigned long long* gacc = (unsigned long long*)(red + 16 * NW);
-  float* xs = (float*)(gacc + mx);
+  unsigned long long* gacc = (unsigned long long*)(red + RED_WORDS);
+  float* g = (float*)(gacc + mx);
+  float* xs = (float*)((char*)g + g_bytes);
   float* pp = xs + mx;
   float* pg = pp + mx;
-  float* g = pg + mx;
   const MolDesc m = load_desc(B.mol_desc + 16 * B.conf_mol[c]);
   const int n = 3 * m.n_atoms;
   const int off = B.conf_off[c];
@@ -1840,13 +1947,14 @@ __global__ void __launch_bounds__(NT) k_bb_fused(KBatch B, const float* __restri
     pp[i] = xs[i];
     pg[i] = 0.f;
   }
-  Reducer<NT> R{red, 0};
+  Reducer<NT, 8, (NR > NT)> R{red, 0};
   float alpha = grad_lr;
   double E_prev = 1e30, E = 0.0;
   for (int it = 0; it < max_it; it++) {
-    for (int i = tid; i < n; i += NT) gacc[i] = 0ull;
+    for (int i = threadIdx.x; i < n; i += NR) gacc[i] = 0ull;
     __syncthreads();
-    E = R.sum(eval_tasks<FAM_MEGA, true, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu, nullptr));
+    E = group_energy<NR>(eval_tasks<FAM_MEGA, true, false, false, NR>(global_view(B, m), m, xs, gacc, 1, 0x7fu), (double*)g,
+                         room, R);
     if (it > 0 && E > E_prev + 1.0) {  // energy guard :1031-1038
       for (int i = tid; i < n; i += NT) xs[i] = pp[i];
       alpha = fmaxf(alpha * 0.5f, 1e-7f);
@@ -1907,12 +2015,12 @@ struct MMState {
   size_t total;
 };
 
-template <int NT, class Red>
+template <int NR, class Red>
 __device__ void mm_eval(const KBatch& B, const MolDesc& m, float* xs, unsigned long long* gacc, Red& R, double& E,
-                        int n) {
-  for (int i = threadIdx.x; i < n; i += NT) gacc[i] = 0ull;
+                        int n, double* buf = nullptr, int room = 0) {
+  for (int i = threadIdx.x; i < n; i += NR) gacc[i] = 0ull;
   __syncthreads();
-  E = R.sum(eval_tasks<FAM_MEGA, true, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu, nullptr));
+  E = group_energy<NR>(eval_tasks<FAM_MEGA, true, false, false, NR>(global_view(B, m), m, xs, gacc, 1, 0x7fu), buf, room, R);
 }
 
 // mode 0: initial (x = x_in), mode 1: polish restart (x = best_x); both compute E+G, scale g,
@@ -1960,10 +2068,12 @@ __device__ __forceinline__ void block_dots(Red& R, int tid, int n, double (&p)[K
   R.template run<K, 0>(p);
 }
 
-// LDS of k_mm_chunk: reduction buffer, gradient accumulators, x, g, q, x_new and alpha, and the
-// (s, y, rho) history when hl
-size_t mm_lds(int nr, int mx, int m, bool hl) {
-  return 16 * (size_t)(nr > 256 ? 2 * (nr / 64) : 4) * 8 + (size_t)mx * (8 + 16) + 8 * (size_t)m + (hl ? 8 * (size_t)m * (mx + 1) : 0) + 32;
+// LDS of k_mm_chunk: reduction buffer, gradient accumulators, x, g, x_new and alpha, the (s, y, rho)
+// history when hl, and q (q_bytes of it; the groups' sums meet there during an evaluation)
+size_t mm_lds(int nr, int mx, int m, bool hl, size_t limit, int& q_bytes) {
+  const size_t rest = RED_WORDS * 8 + (size_t)mx * (8 + 12) + 8 * (size_t)m + (hl ? 8 * (size_t)m * (mx + 1) : 0) + 32;
+  q_bytes = (int)ex_area(nr, (size_t)mx * 4, 2, rest, limit);
+  return rest + q_bytes;
 }
 
 // HL: the (s, y) history is worked on in LDS for the launch's iterations (and written through to
@@ -1983,22 +2093,23 @@ size_t mm_lds(int nr, int mx, int m, bool hl) {
 template <bool HL, int NR>
 __global__ void __launch_bounds__(NR, NR > 256 ? 1 : 4) k_mm_chunk(KBatch B, MMState S, int steps, int it_end, int do_sync,
                                                      int phase, const int32_t* prev_flag, int32_t* my_flag, int M,
-                                                     float max_step, float gsc, float tol) {
+                                                     float max_step, float gsc, float tol, int q_bytes) {
   extern __shared__ __align__(16) unsigned char smem[];
-  constexpr int NT = 256, NW = NR / 64;
+  constexpr int NT = SUM_LANES;
   const int c = blockIdx.x;
   if (c >= B.n_confs) return;
   if (prev_flag && *prev_flag == 0) return;  // every conformer converged at the last sync
   const int tid = NR == NT || threadIdx.x < NT ? (int)threadIdx.x : 1 << 30;
   const int mx = 3 * B.max_atoms;
   double* red = (double*)smem;
-  double* alf = red + 16 * NW + (NR > NT ? 16 * NW : 0);  // [M]
-  double* lrho = alf + M;       // [M] when HL
+  double* alf = red + RED_WORDS;  // [M]
+  double* lrho = alf + M;         // [M] when HL
   unsigned long long* gacc = (unsigned long long*)(HL ? lrho + M : lrho);
-  float* xs = (float*)(gacc + mx);
+  float* q = (float*)(gacc + mx);
+  float* xs = (float*)((char*)q + q_bytes);
   float* gs = xs + mx;
-  float* q = gs + mx;
-  float* xn = q + mx;
+  float* xn = gs + mx;
+  const int room = q_bytes / (EX_WORDS * (int)sizeof(double));
   const MolDesc m = load_desc(B.mol_desc + 16 * B.conf_mol[c]);
   const int n = 3 * m.n_atoms, off = B.conf_off[c];
   const size_t T = S.total, HT = HL ? (size_t)mx : T;
@@ -2022,7 +2133,6 @@ __global__ void __launch_bounds__(NR, NR > 256 ? 1 : 4) k_mm_chunk(KBatch B, MMS
       }
   }
   Reducer<NT, 8, (NR > NT)> R{red, 0};
-  Reducer<NR> RE{NR > NT ? red + 16 * NW : red, 0};
   double E = S.e_new[c];
   __syncthreads();
   for (int st = 0; st < steps; st++) {
@@ -2097,10 +2207,7 @@ __global__ void __launch_bounds__(NR, NR > 256 ? 1 : 4) k_mm_chunk(KBatch B, MMS
       xn[3 * a + 2] = xs[3 * a + 2] + dz * f;
     }
     __syncthreads();
-    if constexpr (NR == NT)
-      mm_eval<NT>(B, m, xn, gacc, R, E, n);
-    else
-      mm_eval<NR>(B, m, xn, gacc, RE, E, n);
+    mm_eval<NR>(B, m, xn, gacc, R, E, n, (double*)q, room);
     // push (s, y, rho) into the ring (:385-399); rho = 0 on bad curvature
     int sl;
     if (len >= M) {
@@ -2186,7 +2293,8 @@ __global__ void __launch_bounds__(NT) k_mm_final(KBatch B, MMState S, float* x_b
   for (int i = threadIdx.x; i < n; i += NT) xs[i] = S.bx[off + i];
   __syncthreads();
   Reducer<NT> R{red, 0};
-  double E = R.sum(eval_tasks<FAM_MEGA, false, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu, nullptr));
+  double E = group_energy<NT>(eval_tasks<FAM_MEGA, false, false, false, NT>(global_view(B, m), m, xs, gacc, 1, 0x7fu), nullptr,
+                              0, R);
   double gmax = 0.0;
   if (l2_norm) {
     for (int i = threadIdx.x; i < n; i += NT) gmax += (double)S.g[off + i] * S.g[off + i];
@@ -2259,49 +2367,63 @@ int check_batch(const mmffhip_batch* b) {
   return MMFFHIP_OK;
 }
 
-size_t eg_lds(int nt, int max_atoms) {
-  return 16 * (nt / 64) * 8 + (size_t)3 * max_atoms * (8 + 4) + 16;
+// LDS of k_energy_grad, of which xs_bytes are the positions' (wide workgroups: the sums' of energy
+// and kinds at once, which always fits where the narrow kernel does)
+size_t eg_lds(int nt, int max_atoms, bool terms, size_t limit, int& xs_bytes) {
+  const size_t rest = RED_WORDS * 8 + (size_t)3 * max_atoms * 8 + 16;
+  xs_bytes = (int)ex_area(nt, (size_t)3 * max_atoms * 4, terms ? 7 : 2, rest, limit);
+  return rest + xs_bytes;
 }
 
 // At most one conformer per CU: sixteen waves per conformer, whose latency is the call's; four
 // otherwise. One conformer of a 245-atom chain 50 -> 24 us, 180 conformers of three chains (energies
 // alone) 34.5 -> 19.1 us; molecules of 60 atoms are bound by the host's 10 us per call either way.
-template <int FAM, int NT>
-int launch_eg_nt(const KBatch& kb, const float* x, double* e, double* et, float* g, uint32_t mask, int diel,
-                 hipStream_t s) {
-  const size_t lds = eg_lds(NT, kb.max_atoms);
-  allow_lds((const void*)&k_energy_grad<FAM, NT>, lds);
-  hipLaunchKernelGGL((k_energy_grad<FAM, NT>), dim3(kb.n_confs), dim3(NT), lds, s, kb, x, e, et, g, mask, diel);
-  HIP_TRY(hipGetLastError());
-  return MMFFHIP_OK;
-}
-template <int FAM>
+template <int FAM, bool PT>
 int launch_eg(const KBatch& kb, const float* x, double* e, double* et, float* g, uint32_t mask, int diel,
               hipStream_t s) {
   const DevInfo di = dev_info();
-  if ((int)eg_lds(256, kb.max_atoms) > di.lds)
-    return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
-  if (kb.n_confs <= di.n_cu && (int)eg_lds(1024, kb.max_atoms) <= di.lds)
-    return launch_eg_nt<FAM, 1024>(kb, x, e, et, g, mask, diel, s);
-  return launch_eg_nt<FAM, 256>(kb, x, e, et, g, mask, diel, s);
+  int xs_bytes = 0;
+  size_t lds = eg_lds(256, kb.max_atoms, PT, di.lds, xs_bytes);
+  if (lds > (size_t)di.lds) return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
+  int nt = 256;
+  auto kernel = k_energy_grad<FAM, PT, 256>;
+  if (kb.n_confs <= di.n_cu) {
+    int wide_xs = 0;
+    const size_t wide = eg_lds(1024, kb.max_atoms, PT, di.lds, wide_xs);
+    if (wide <= (size_t)di.lds) {
+      kernel = k_energy_grad<FAM, PT, 1024>;
+      nt = 1024;
+      lds = wide;
+      xs_bytes = wide_xs;
+    }
+  }
+  allow_lds((const void*)kernel, lds);
+  hipLaunchKernelGGL(kernel, dim3(kb.n_confs), dim3(nt), lds, s, kb, x, e, et, g, mask, diel, xs_bytes);
+  HIP_TRY(hipGetLastError());
+  return MMFFHIP_OK;
 }
 
 // The launch of k_mm_chunk: wide workgroups when there is at most one conformer per CU; the history
 // in LDS when it fits there, or leaves three workgroups per CU.
 struct MMChunk {
-  void (*kernel)(KBatch, MMState, int, int, int, int, const int32_t*, int32_t*, int, float, float, float);
+  void (*kernel)(KBatch, MMState, int, int, int, int, const int32_t*, int32_t*, int, float, float, float, int);
   int nr;
   size_t lds;
+  int q_bytes;
 };
 MMChunk mm_chunk_plan(int n_confs, int mx, int m, const DevInfo& di) {
+  const size_t limit = (size_t)di.lds;
+  int q = 0;
   if (n_confs <= di.n_cu) {
-    const size_t hl = mm_lds(1024, mx, m, true), g = mm_lds(1024, mx, m, false);
-    if (hl <= (size_t)di.lds) return {k_mm_chunk<true, 1024>, 1024, hl};
-    if (g <= (size_t)di.lds) return {k_mm_chunk<false, 1024>, 1024, g};
+    const size_t hl = mm_lds(1024, mx, m, true, limit, q);
+    if (hl <= limit) return {k_mm_chunk<true, 1024>, 1024, hl, q};
+    const size_t g = mm_lds(1024, mx, m, false, limit, q);
+    if (g <= limit) return {k_mm_chunk<false, 1024>, 1024, g, q};
   }
-  const size_t hl = mm_lds(256, mx, m, true);
-  if (hl <= (size_t)di.lds / 3) return {k_mm_chunk<true, 256>, 256, hl};
-  return {k_mm_chunk<false, 256>, 256, mm_lds(256, mx, m, false)};
+  const size_t hl = mm_lds(256, mx, m, true, limit, q);
+  if (hl <= limit / 3) return {k_mm_chunk<true, 256>, 256, hl, q};
+  const size_t g = mm_lds(256, mx, m, false, limit, q);
+  return {k_mm_chunk<false, 256>, 256, g, q};
 }
 
 int round4(int v) { return (v + 3) & ~3; }
@@ -2589,9 +2711,11 @@ int mmffhip_energy_grad(const mmffhip_batch* b, int family, int diel, const floa
     return fail(MMFFHIP_ERR_ARG, "the MEGA family has a constant dielectric only");
   KBatch kb = to_kbatch(b);
   hipStream_t s = (hipStream_t)stream;
-  if (family == MMFFHIP_FAMILY_TG) return launch_eg<FAM_TG>(kb, x, e_out, e_terms, g_out, term_mask, diel, s);
-  if (family == MMFFHIP_FAMILY_MEGA) return launch_eg<FAM_MEGA>(kb, x, e_out, e_terms, g_out, term_mask, 1, s);
-  return fail(MMFFHIP_ERR_ARG, "unknown family");
+  const bool tg = family == MMFFHIP_FAMILY_TG;
+  if (!tg && family != MMFFHIP_FAMILY_MEGA) return fail(MMFFHIP_ERR_ARG, "unknown family");
+  const auto launch = e_terms ? (tg ? launch_eg<FAM_TG, true> : launch_eg<FAM_MEGA, true>)
+                              : (tg ? launch_eg<FAM_TG, false> : launch_eg<FAM_MEGA, false>);
+  return launch(kb, x, e_out, e_terms, g_out, term_mask, tg ? diel : 1, s);
 }
 
 int mmffhip_minimize_nk_workspace(const mmffhip_batch* b, const mmffhip_nk_opts* o, size_t* bytes) {
@@ -2681,18 +2805,23 @@ int mmffhip_bb_fused(const mmffhip_batch* b, const float* x_in, float* x_out, do
   if (b->n_confs == 0) return MMFFHIP_OK;
   if (!x_in || !x_out || !e_out) return fail(MMFFHIP_ERR_ARG, "x_in, x_out and e_out are required");
   if (max_iters < 0) return fail(MMFFHIP_ERR_ARG, "max_iters must be >= 0");
-  auto lds = [&](int nt) { return 16 * (size_t)(nt / 64) * 8 + (size_t)3 * b->max_atoms * (8 + 4 * 4) + 16; };
   const DevInfo di = dev_info();
-  if ((int)lds(256) > di.lds) return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
+  int g_bytes = 0;
+  auto plan = [&](int nt) {
+    const size_t rest = RED_WORDS * 8 + (size_t)3 * b->max_atoms * (8 + 3 * 4) + 16;
+    g_bytes = (int)ex_area(nt, (size_t)3 * b->max_atoms * 4, 2, rest, di.lds);
+    return rest + g_bytes;
+  };
+  if (plan(256) > (size_t)di.lds) return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
   KBatch kb = to_kbatch(b);
   // at most one conformer per CU: sixteen waves each, as in launch_eg. 60 ragged conformers,
   // 200 steps: 2.19 -> 1.50 ms
-  const bool wide = b->n_confs <= di.n_cu && (int)lds(1024) <= di.lds;
-  const int nt = wide ? 1024 : 256;
-  const auto kernel = wide ? k_bb_fused<1024> : k_bb_fused<256>;
-  allow_lds((const void*)kernel, lds(nt));
-  hipLaunchKernelGGL(kernel, dim3(b->n_confs), dim3(nt), lds(nt), (hipStream_t)stream, kb, x_in, x_out, e_out,
-                     (int)max_iters, max_step, grad_lr);
+  const int nt = b->n_confs <= di.n_cu && plan(1024) <= (size_t)di.lds ? 1024 : 256;
+  const size_t lds = plan(nt);
+  const auto kernel = nt == 1024 ? k_bb_fused<1024> : k_bb_fused<256>;
+  allow_lds((const void*)kernel, lds);
+  hipLaunchKernelGGL(kernel, dim3(b->n_confs), dim3(nt), lds, (hipStream_t)stream, kb, x_in, x_out, e_out,
+                     (int)max_iters, max_step, grad_lr, g_bytes);
   HIP_TRY(hipGetLastError());
   return MMFFHIP_OK;
 }
@@ -2792,7 +2921,7 @@ int mmffhip_multimol_run_ex(const mmffhip_batch* b, const float* x_in, float* x_
     // -1) and no launch reads the previous sync point's count
     hipLaunchKernelGGL(ck.kernel, dim3(b->n_confs), dim3(ck.nr), ck.lds, s, kb, S, steps, it, sync ? 1 : 0,
                        0, (k > 0 && !batch) ? S.flags + (k - 1) : (const int32_t*)nullptr, S.flags + k,
-                       (int)lbfgs_m, max_step_per_atom, grad_scale, batch ? -1.0f : grad_tol);
+                       (int)lbfgs_m, max_step_per_atom, grad_scale, batch ? -1.0f : grad_tol, ck.q_bytes);
     if (sync) k++;
   }
   HIP_TRY(hipGetLastError());
@@ -2807,7 +2936,7 @@ int mmffhip_multimol_run_ex(const mmffhip_batch* b, const float* x_in, float* x_
     const bool sync = (it % eval_freq) == 0;
     hipLaunchKernelGGL(ck.kernel, dim3(b->n_confs), dim3(ck.nr), ck.lds, s, kb, S, steps, it, sync ? 1 : 0,
                        1, kp > n_main ? S.flags + (kp - 1) : (const int32_t*)nullptr, S.flags + kp, (int)lbfgs_m,
-                       max_step_per_atom, grad_scale, grad_tol);
+                       max_step_per_atom, grad_scale, grad_tol, ck.q_bytes);
     if (sync) kp++;
   }
   HIP_TRY(hipGetLastError());

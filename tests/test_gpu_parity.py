@@ -442,3 +442,67 @@ def test_bonded_windows_of_the_smallest_molecules():
     torch.cuda.synchronize()
     assert torch.equal(few.x.repeat(300), many.x) and torch.equal(few.energy.repeat(300), many.energy)
     assert torch.equal(few.counters.repeat(300, 1), many.counters)
+
+
+def _few_and_many(families=("small", "ragged", "chain"), fill=300, n_confs=2):
+    """A batch of a few conformers, and the same conformers in front of `fill` more of a small
+    molecule (more than one per CU): (few batch, its x, many batch, its x), x on the device."""
+    from mlxmolkit_archive_amd import engine, workloads
+    wls = [workloads.build(f, n_mols=1 if f == "chain" else 3, n_confs=n_confs) for f in families]
+    p2 = conftest.mol_params("[H][H]", seed=4, k=1)
+    params, counts = [p for w in wls for p in w.params] + [p2[1]], [c for w in wls for c in w.conf_counts] + [1]
+    x = np.concatenate([w.x for w in wls] + [p2[2]])
+    f = workloads.build("small", n_mols=1, n_confs=fill)
+    return (engine.device_batch(params, counts), torch.from_numpy(x).cuda(),
+            engine.device_batch(params + f.params, counts + [fill]), torch.from_numpy(np.concatenate([x, f.x])).cuda())
+
+
+@pytest.mark.parametrize("mask", [0x7F, 0x20, 0x51])
+@pytest.mark.parametrize("family,diel", [(0, 1), (0, 2), (1, 1)])
+def test_single_points_do_not_depend_on_the_batch(family, diel, mask):
+    """Batches of at most one conformer per CU run in wide workgroups: bit for bit the energies,
+    terms and gradients that the same conformers have in a larger batch (small batches' are compared
+    with the oracle above); and energies are the same whether terms are asked for or not."""
+    from mlxmolkit_archive_amd import engine
+    db, x, db2, x2 = _few_and_many()
+    c, n = db.n_confs, x.numel()
+    got = []
+    for grad in (False, True):
+        for terms in (False, True):
+            a = engine.energy_grad(db, x, family=family, diel=diel, mask=mask, grad=grad, terms=terms)
+            b = engine.energy_grad(db2, x2, family=family, diel=diel, mask=mask, grad=grad, terms=terms)
+            torch.cuda.synchronize()
+            assert torch.equal(a[0], b[0][:c])
+            assert not grad or torch.equal(a[1], b[1][:n])
+            assert not terms or torch.equal(a[2], b[2][:c])
+            if terms:
+                # seven FP64 sums of at most a few thousand values each against one of all of them
+                assert torch.allclose(a[2].sum(1), a[0], rtol=0, atol=1e-10 * float(a[2].abs().max()))
+            got.append(a[0])
+    assert torch.equal(got[0], got[1]) and torch.equal(got[2], got[3])
+
+
+def test_descent_does_not_depend_on_the_batch():
+    """The Barzilai-Borwein descent of a few conformers (wide workgroups) and of the same
+    conformers in a batch of more than one per CU: the same geometries and energies, bit for bit,
+    over a run long enough for the energy guard and the step's dot products to matter."""
+    from mlxmolkit_archive_amd import engine
+    db, x, db2, x2 = _few_and_many()
+    for iters in (1, 3, 200):
+        a, b = engine.bb_fused(db, x, max_iters=iters), engine.bb_fused(db2, x2, max_iters=iters)
+        torch.cuda.synchronize()
+        assert torch.equal(a[0], b[0][:x.numel()]) and torch.equal(a[1], b[1][:db.n_confs])
+
+
+@pytest.mark.parametrize("families", [("small",), ("small", "chain")])
+def test_lockstep_does_not_depend_on_the_batch(families):
+    """The lock-step L-BFGS of a few conformers and of the same conformers in a batch of more than
+    one per CU (history in LDS for small molecules alone, in memory beside a chain)."""
+    from mlxmolkit_archive_amd import engine
+    db, x, db2, x2 = _few_and_many(families)
+    kw = dict(max_iters=60, grad_tol=0.0)
+    a, b = engine.multimol(db, x, **kw), engine.multimol(db2, x2, **kw)
+    torch.cuda.synchronize()
+    c = db.n_confs
+    assert torch.equal(a["x"], b["x"][:x.numel()]) and torch.equal(a["energy"], b["energy"][:c])
+    assert torch.equal(a["grad_norm"], b["grad_norm"][:c])
