@@ -2512,6 +2512,8 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
   // Stage term tables in LDS when asked and when they fit: all of them next to an LDS
   // Hessian; only the bonded ones beside a global Hessian, and only when that keeps the
   // unstaged kernel's workgroups per CU (there, occupancy hides the pair loads).
+  const int max_wg = std::max(1, 12 / (pl.nt / 64));  // workgroups per CU at most (below)
+  bool help_stage = false;  // helper kernels may stage: as many workgroups per CU as launch without
   if (o->table_lds_bytes > 0) {
     const int tl = pl.hm == 0 ? 1 : 2;
     const size_t with = nk_lds_bytes(o->algo, pl.hm, pl.nt, pl.max_n, m, (size_t)o->table_lds_bytes);
@@ -2523,7 +2525,11 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
       allow_lds(kt, with);
       if (k0) allow_lds(k0, pl.lds);
       take = k0 && hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc0, k0, pl.nt, pl.lds) == hipSuccess &&
-             hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc1, kt, pl.nt, with) == hipSuccess && pc1 >= pc0;
+             hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc1, kt, pl.nt, with) == hipSuccess;
+      help_stage = take && pc1 >= std::min(pc0, max_wg);
+      take = take && pc1 >= pc0;
+    } else {
+      help_stage = take;
     }
     if (take) {
       pl.tl = tl;
@@ -2533,8 +2539,11 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
   }
   // At most one conformer per CU: the time is the longest conformer's, so its workgroup gets
   // helper threads, and L-BFGS its history in LDS where that fits (both leave the results as
-  // they are). The bonded terms' energies take a word each; a bonded term has at least 12 table
-  // bytes, so table_lds_bytes bounds their number. Ten conformers of 48 atoms, BFGS,
+  // they are). The bonded tables are staged where a launch without helpers could (a caller whose
+  // reserve is smaller than a molecule's tables, and which the rule above spared, stays spared): ten
+  // conformers of 82 atoms 4.48 -> 4.65 ms without staging (L-BFGS), 5.50 -> 5.61 (BFGS). The bonded
+  // terms' energies take a word each; a bonded term has at least 12 table bytes, so
+  // table_lds_bytes bounds their number (eval_help takes more in windows). Ten conformers of 48 atoms, BFGS,
   // host work included: 4.28 -> 3.99 ms; 221 chains of 199-329 atoms, L-BFGS: 180 -> 127 ms (151 with
   // the history in LDS alone); with the bonded tasks' spread terms 3.95 and 116 ms. Above one
   // conformer per CU the waves of other conformers fill the CU and helpers would only displace them.
@@ -2544,7 +2553,7 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
       int hm, tl;
     } tries[] = {{0, 2}, {0, 0}, {pl.hm, 2}, {pl.hm, 0}};
     for (const auto& t : tries) {
-      if (t.hm == 0 && o->algo != MMFFHIP_LBFGS) continue;
+      if ((t.hm == 0 && o->algo != MMFFHIP_LBFGS) || (t.tl > 0 && !help_stage)) continue;
       const int tb = t.tl ? ((o->table_lds_bytes + 15) / 16) * 16 : 0;
       const size_t lds = nk_lds_bytes(o->algo, t.hm, pl.nt, pl.max_n, m, (size_t)tb, NK_HELP, eb);
       if (!nk_kernel(o->algo, t.hm, t.tl, pl.nt, NK_HELP) || lds > (size_t)di.lds) continue;
@@ -2566,7 +2575,7 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
   // Twelve waves per CU at most, whatever registers a kernel leaves free: the resident Hessians
   // stay in the Infinity Cache, a fourth wave per SIMD gains 1% at best (100,000 ragged conformers
   // 1,084 -> 1,075 ms, 2,500 small ones 13.6 -> 15.0), and callers size their buckets by this grid.
-  per_cu = std::min(per_cu, std::max(1, 12 / (pl.nt * pl.help / 64)));
+  per_cu = std::min(per_cu, std::max(1, max_wg / pl.help));
   pl.grid = std::max(1, std::min(b->n_confs, di.n_cu * per_cu));
   pl.slot_floats = 0;
   if (pl.hm != 0) {

@@ -506,3 +506,23 @@ def test_lockstep_does_not_depend_on_the_batch(families):
     c = db.n_confs
     assert torch.equal(a["x"], b["x"][:x.numel()]) and torch.equal(a["energy"], b["energy"][:c])
     assert torch.equal(a["grad_norm"], b["grad_norm"][:c])
+
+
+@pytest.mark.parametrize("use_lbfgs", [False, True])
+def test_reserve_too_small_to_stage_is_ignored(use_lbfgs):
+    """A table reserve that would cost workgroups per CU is ignored, so one smaller than the
+    molecule's tables does no harm there; the helper threads of a small batch do not change that: no
+    status 2, and the results of a launch without staging, bit for bit."""
+    from mlxmolkit_archive_amd import engine, workloads
+    wl = workloads.build("chain", n_mols=1, n_confs=2)
+    assert wl.params[0].n_atoms == 199  # 68 KB of LDS with BFGS, 29 KB with L-BFGS
+    db, x = engine.device_batch(wl.params, wl.conf_counts), torch.from_numpy(wl.x).cuda()
+    kw = dict(max_iters=25, grad_tol=1e-4, use_lbfgs=use_lbfgs, ls_grad=True)
+    want = engine.NkRunner(db, stage_tables=False, **kw).run(x)
+    r = engine.NkRunner(db, **kw)
+    reserve = 26000 if use_lbfgs else 16384  # three and two workgroups per CU become two and one
+    assert len(r.launches) == 1 and r.launches[0]["opts"].table_lds_bytes > reserve
+    r.launches[0]["opts"].table_lds_bytes = reserve
+    got = r.run(x)
+    torch.cuda.synchronize()
+    assert torch.equal(got.status, want.status) and torch.equal(got.x, want.x) and torch.equal(got.energy, want.energy)
