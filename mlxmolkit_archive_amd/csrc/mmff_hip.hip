@@ -1126,6 +1126,10 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
   // During an evaluation the bonded terms' energies lie in dgv, hd and the accumulators (at least
   // 12 floats per atom, which hold all but a cage molecule's at once, and never less than a task's
   // 64), none of which is live then; L-BFGS has that room where BFGS keeps its update.
+  // The full-matrix kernels have no registers for the next term's tables: loading them ahead took
+  // 112-132 bytes of scratch per lane at 64-256 threads, 20-44 without, and 8,000 ragged conformers of
+  // 256 threads 103.6 -> 98.3 ms (128 threads, medium: 24.7 -> 24.2; 640, ragged: 31.1 -> 27.9).
+  constexpr bool PREF = TL == 0 && HM != 1;
   constexpr bool ORDERED = HELP == 1 && (SYM || ALGO == MMFFHIP_LBFGS);
   float* ebuf = SYM ? dgv : UP;
   const int ebuf_n = SYM ? 2 * mn + NW * sacc_w : lbfgs_eb_floats(mn);
@@ -1244,7 +1248,7 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
       else if constexpr (ORDERED)
         return eval_ordered<FAM_TG, G, EV, NT>(TV, m, xs, gacc, P.diel, ebuf, ebuf_n);
       else
-        return eval_terms<FAM_TG, G, NT, TL == 0, EV>(TV, m, xs, gacc, P.diel);
+        return eval_terms<FAM_TG, G, NT, PREF, EV>(TV, m, xs, gacc, P.diel);
     };
     const std::true_type yes;
     const std::false_type no;
