@@ -526,3 +526,81 @@ def test_reserve_too_small_to_stage_is_ignored(use_lbfgs):
     got = r.run(x)
     torch.cuda.synchronize()
     assert torch.equal(got.status, want.status) and torch.equal(got.x, want.x) and torch.equal(got.energy, want.energy)
+
+
+def _water_box(n, k=2, seed=5):
+    """(params, flat coordinates of k conformers) of n water molecules on a 3.1 A grid: many atoms,
+    few bonded terms."""
+    from mlxmolkit_archive_amd.mmff_params import extract_mmff_params
+    from mlxmolkit_archive_amd.mol import mol_from_smiles
+    m = mol_from_smiles(".".join(["O"] * n))
+    m.set_conformers(np.zeros((1, m.GetNumAtoms(), 3)))
+    p = extract_mmff_params(m)
+    g = int(np.ceil(n ** (1 / 3)))
+    o = 3.1 * np.array([(i // g // g, i // g % g, i % g) for i in range(n)], np.float64)
+    x = np.zeros((p.n_atoms, 3))
+    x[:n] = o
+    h = np.zeros(n, int)
+    for i, j in zip(p.bond_idx1, p.bond_idx2):
+        a, b = (i, j) if i < n else (j, i)
+        x[b] = o[a] + (0.76, 0.59 * (1 - 2 * h[a]), 0.0)
+        h[a] += 1
+    assert (h == 2).all()
+    noise = np.random.default_rng(seed).normal(0.0, 0.05, (k, *x.shape))
+    return p, (x + noise).astype(np.float32).reshape(-1)
+
+
+def _plan(desc, o):
+    import ctypes
+    from mlxmolkit_archive_amd import _lib
+    g, b, lds, place = (ctypes.c_int32() for _ in range(4))
+    _lib.check(_lib.load().mmffhip_minimize_nk_plan(ctypes.byref(desc), ctypes.byref(o), ctypes.byref(g),
+                                                    ctypes.byref(b), ctypes.byref(lds), ctypes.byref(place)))
+    return dict(lds=lds.value, place=place.value)
+
+
+@pytest.mark.parametrize("reserve", [None, 20000])
+def test_helper_threads_with_the_history_in_memory(reserve):
+    """L-BFGS of 318 atoms with m = 16: a history that does not fit the LDS beside helper threads, with
+    the bonded tables staged (7 KB of them keep three workgroups per CU) or, given a reserve that does
+    not keep them, read from memory. Bit for bit the results inside a batch without helpers."""
+    from mlxmolkit_archive_amd import _lib, engine, workloads
+    p, x = _water_box(106)
+    f = workloads.build("small", n_mols=1, n_confs=300)
+    kw = dict(max_iters=25, grad_tol=1e-4, use_lbfgs=True, ls_grad=True, lbfgs_m=16)
+    r = engine.NkRunner(engine.device_batch([p], [2]), **kw)
+    ln, = r.launches
+    assert 7000 < ln["opts"].table_lds_bytes < 8000
+    if reserve:
+        ln["opts"].table_lds_bytes = reserve
+    n = 3 * p.n_atoms + 2
+    got = _plan(ln["desc"], ln["opts"])
+    # 832 bytes and 32 per coordinate, the pair energies' ring and the bonded energies; the tables
+    eb = (ln["opts"].table_lds_bytes // 12 + 64) // 64 * 64
+    assert got["place"] == _lib.HESS_GLOBAL
+    assert got["lds"] == 832 + 32 * n + 4 * (3072 + eb) + (0 if reserve else -(-ln["opts"].table_lds_bytes // 16) * 16)
+    few = r.run(torch.from_numpy(x).cuda())
+    many = engine.NkRunner(engine.device_batch([p] + f.params, [2, 300]), **kw).run(
+        torch.from_numpy(np.concatenate([x, f.x])).cuda())
+    torch.cuda.synchronize()
+    assert torch.equal(few.x, many.x[:len(x)]) and torch.equal(few.energy, many.energy[:2])
+    assert torch.equal(few.status, many.status[:2]) and torch.equal(few.counters, many.counters[:2])
+    assert (few.counters[:, 0] > 16).all() and torch.isfinite(few.energy).all()
+
+
+@pytest.mark.parametrize("waters", [171, 176])
+def test_lockstep_wide_workgroups_at_the_lds_limit(waters):
+    """The lock-step engine's wide workgroups where the LDS has room for one of an energy's two sums at
+    a time beside the history (513 atoms), and where the history goes to memory (528 atoms): bit for
+    bit the results in a batch of more than one conformer per CU."""
+    from mlxmolkit_archive_amd import engine, workloads
+    p, x = _water_box(waters)
+    f = workloads.build("small", n_mols=1, n_confs=300)
+    kw = dict(max_iters=20, grad_tol=0.0)
+    a = engine.multimol(engine.device_batch([p], [2]), torch.from_numpy(x).cuda(), **kw)
+    b = engine.multimol(engine.device_batch([p] + f.params, [2, 300]),
+                        torch.from_numpy(np.concatenate([x, f.x])).cuda(), **kw)
+    torch.cuda.synchronize()
+    assert torch.isfinite(a["energy"]).all() and not torch.equal(a["x"], torch.from_numpy(x).cuda())
+    assert torch.equal(a["x"], b["x"][:len(x)]) and torch.equal(a["energy"], b["energy"][:2])
+    assert torch.equal(a["grad_norm"], b["grad_norm"][:2])
