@@ -913,13 +913,14 @@ constexpr int RED_WORDS = 2 * (SUM_LANES / 64) * 8;  // doubles of a Reducer<SUM
 // Kernel: single-point energy / gradient / per-term energies, one workgroup per conformer.
 // Replaces mmff_energy_grad_metal(_mega) (mmff_metal_kernel.py:713-775); the TG family is
 // what the nk kernel evaluates (mmff_bfgs_header.metal).
-// xs_bytes: the positions' LDS, where the groups' sums meet once the positions are done with
+// The groups' sums meet in LDS behind the positions (xs_bytes), room values at a time, or where the
+// positions were when room is 0 (xs_bytes then hold one value at least)
 // The narrow kernels with kinds are held to 7 and 5 waves per SIMD (TG, MEGA), which they miss by a
 // register or two: 12,139 ragged MEGA energies with kinds 73.7 us, 80.1 at four
 template <int FAM, bool PT, int NT>
 __global__ void __launch_bounds__(NT, NT == 256 ? (FAM == FAM_TG ? 7 : 5) : 4) k_energy_grad(KBatch B, const float* __restrict__ x, double* e_out,
                                                     double* e_terms, float* g_out, uint32_t mask, int diel,
-                                                    int xs_bytes) {
+                                                    int xs_bytes, int room) {
   extern __shared__ __align__(16) unsigned char smem[];
   const int c = blockIdx.x;
   if (c >= B.n_confs) return;
@@ -939,9 +940,12 @@ __global__ void __launch_bounds__(NT, NT == 256 ? (FAM == FAM_TG ? 7 : 5) : 4) k
     sum = eval_tasks<FAM, true, true, PT, NT>(global_view(B, m), m, xs, gacc, diel, mask);
   else
     sum = eval_tasks<FAM, false, true, PT, NT>(global_view(B, m), m, xs, gacc, diel, mask);
-  double* buf = (double*)xs;
-  const int room = xs_bytes / (EX_WORDS * (int)sizeof(double));
-  if (NT > SUM_LANES) __syncthreads();  // the positions give way to the sums
+  double* buf = (double*)((char*)xs + xs_bytes);
+  if (NT > SUM_LANES && room == 0) {
+    __syncthreads();  // the positions give way to the sums
+    buf = (double*)xs;
+    room = xs_bytes / (EX_WORDS * (int)sizeof(double));
+  }
   const double e = group_energy<NT>(sum, buf, room, R);
   if constexpr (PT) {
     combine_groups<NT>(sum.kind, buf, room);
@@ -2371,12 +2375,17 @@ int check_batch(const mmffhip_batch* b) {
   return MMFFHIP_OK;
 }
 
-// LDS of k_energy_grad, of which xs_bytes are the positions' (wide workgroups: the sums' of energy
-// and kinds at once, which always fits where the narrow kernel does)
-size_t eg_lds(int nt, int max_atoms, bool terms, size_t limit, int& xs_bytes) {
-  const size_t rest = RED_WORDS * 8 + (size_t)3 * max_atoms * 8 + 16;
-  xs_bytes = (int)ex_area(nt, (size_t)3 * max_atoms * 4, terms ? 7 : 2, rest, limit);
-  return rest + xs_bytes;
+// LDS of k_energy_grad and its last two arguments; always fits a wide workgroup where it fits a
+// narrow one
+size_t eg_lds(int nt, int max_atoms, bool terms, size_t limit, int& xs_bytes, int& room) {
+  const size_t rest = RED_WORDS * 8 + (size_t)3 * max_atoms * 8 + 16, one = EX_WORDS * sizeof(double);
+  xs_bytes = (3 * max_atoms * 4 + 7) & ~7;
+  room = nt > SUM_LANES ? (terms ? 7 : 2) : 0;
+  if (rest + xs_bytes + room * one > limit) {
+    room = 0;
+    xs_bytes = (int)ex_area(nt, (size_t)3 * max_atoms * 4, 1, rest, limit);
+  }
+  return rest + xs_bytes + room * one;
 }
 
 // At most one conformer per CU: sixteen waves per conformer, whose latency is the call's; four
@@ -2386,23 +2395,18 @@ template <int FAM, bool PT>
 int launch_eg(const KBatch& kb, const float* x, double* e, double* et, float* g, uint32_t mask, int diel,
               hipStream_t s) {
   const DevInfo di = dev_info();
-  int xs_bytes = 0;
-  size_t lds = eg_lds(256, kb.max_atoms, PT, di.lds, xs_bytes);
+  int xs_bytes = 0, room = 0;
+  size_t lds = eg_lds(256, kb.max_atoms, PT, di.lds, xs_bytes, room);
   if (lds > (size_t)di.lds) return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
   int nt = 256;
   auto kernel = k_energy_grad<FAM, PT, 256>;
   if (kb.n_confs <= di.n_cu) {
-    int wide_xs = 0;
-    const size_t wide = eg_lds(1024, kb.max_atoms, PT, di.lds, wide_xs);
-    if (wide <= (size_t)di.lds) {
-      kernel = k_energy_grad<FAM, PT, 1024>;
-      nt = 1024;
-      lds = wide;
-      xs_bytes = wide_xs;
-    }
+    lds = eg_lds(1024, kb.max_atoms, PT, di.lds, xs_bytes, room);
+    kernel = k_energy_grad<FAM, PT, 1024>;
+    nt = 1024;
   }
   allow_lds((const void*)kernel, lds);
-  hipLaunchKernelGGL(kernel, dim3(kb.n_confs), dim3(nt), lds, s, kb, x, e, et, g, mask, diel, xs_bytes);
+  hipLaunchKernelGGL(kernel, dim3(kb.n_confs), dim3(nt), lds, s, kb, x, e, et, g, mask, diel, xs_bytes, room);
   HIP_TRY(hipGetLastError());
   return MMFFHIP_OK;
 }
