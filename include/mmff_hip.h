@@ -172,13 +172,15 @@ int mmffhip_minimize_nk_noalloc(const mmffhip_batch *b, const mmffhip_nk_opts *o
                                 void *stream);
 
 /* Barzilai-Borwein steepest descent of mmff_optimize_metal_fused (MEGA family).
- * e_out: energy of the last pre-step geometry, as the reference returns. */
+ * e_out: energy of the last pre-step geometry, as the reference returns. A conformer's results do
+ * not depend on the batch it is in. */
 int mmffhip_bb_fused(const mmffhip_batch *b, const float *x_in, float *x_out, double *e_out, int32_t max_iters,
                      float max_step, float grad_lr, void *stream);
 
 /* Lock-step host-L-BFGS of mmff_optimize_metal_multi_mol, run on the device in chunks of
  * eval_freq iterations. State lives in a caller workspace; counters in flags decide the
- * global early exit without host synchronisation, so the whole sequence is capturable. */
+ * global early exit without host synchronisation, so the whole sequence is capturable. That exit
+ * aside, a conformer's results do not depend on the batch it is in. */
 int mmffhip_multimol_workspace(const mmffhip_batch *b, int32_t lbfgs_m, size_t *bytes);
 int mmffhip_multimol_run(const mmffhip_batch *b, const float *x_in, float *x_best, double *e_final,
                          float *grad_norm, int32_t *per_conf_iters, int32_t *converged, int32_t *iters_used,

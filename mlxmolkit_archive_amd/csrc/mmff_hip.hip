@@ -2388,9 +2388,13 @@ size_t eg_lds(int nt, int max_atoms, bool terms, size_t limit, int& xs_bytes, in
   return rest + xs_bytes + room * one;
 }
 
-// At most one conformer per CU: sixteen waves per conformer, whose latency is the call's; four
-// otherwise. One conformer of a 245-atom chain 50 -> 24 us, 180 conformers of three chains (energies
-// alone) 34.5 -> 19.1 us; molecules of 60 atoms are bound by the host's 10 us per call either way.
+// At most one conformer per CU: sixteen waves per conformer, whose latency is the call's, from the
+// size on where that gains more than four groups' meeting in LDS costs; four waves otherwise. TG
+// energy and gradient of one conformer, us from launch to launch, four and sixteen waves: 9 atoms 3.6
+// and 4.2, 34 atoms 4.6 and 4.7, 82 atoms 8.0 and 6.4, 253 atoms 36.4 and 20.3; with kinds 4.4 and 5.8, 5.2
+// and 6.3, 8.6 and 7.9, 36.6 and 21.8. (The Python entry point's host work takes 10 us a call.) A
+// wide workgroup fills its CU, so with more conformers than CUs they queue: 300 conformers of 82
+// atoms 10.3 and 11.8 us, 768: 12.7 and 17.3.
 template <int FAM, bool PT>
 int launch_eg(const KBatch& kb, const float* x, double* e, double* et, float* g, uint32_t mask, int diel,
               hipStream_t s) {
@@ -2400,7 +2404,7 @@ int launch_eg(const KBatch& kb, const float* x, double* e, double* et, float* g,
   if (lds > (size_t)di.lds) return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
   int nt = 256;
   auto kernel = k_energy_grad<FAM, PT, 256>;
-  if (kb.n_confs <= di.n_cu) {
+  if (kb.n_confs <= di.n_cu && kb.max_atoms > (PT ? 64 : 40)) {
     lds = eg_lds(1024, kb.max_atoms, PT, di.lds, xs_bytes, room);
     kernel = k_energy_grad<FAM, PT, 1024>;
     nt = 1024;
@@ -2411,8 +2415,11 @@ int launch_eg(const KBatch& kb, const float* x, double* e, double* et, float* g,
   return MMFFHIP_OK;
 }
 
-// The launch of k_mm_chunk: wide workgroups when there is at most one conformer per CU; the history
-// in LDS when it fits there, or leaves three workgroups per CU.
+// The launch of k_mm_chunk: wide workgroups when there is at most one conformer per CU and the
+// molecules are not small, as in launch_eg (one conformer, 100 + 25 iterations, narrow and wide: 34 atoms 1.34
+// and 1.47 ms, 48 atoms 1.47 and 1.52, 82 atoms 1.89 and 1.76, 253 atoms 6.49 and 3.99; 257 conformers
+// of 82 atoms 2.29 and 3.46 ms); the history in LDS when it fits there, or leaves three workgroups
+// per CU.
 struct MMChunk {
   void (*kernel)(KBatch, MMState, int, int, int, int, const int32_t*, int32_t*, int, float, float, float, int);
   int nr;
@@ -2422,7 +2429,7 @@ struct MMChunk {
 MMChunk mm_chunk_plan(int n_confs, int mx, int m, const DevInfo& di) {
   const size_t limit = (size_t)di.lds;
   int q = 0;
-  if (n_confs <= di.n_cu) {
+  if (n_confs <= di.n_cu && mx > 3 * 56) {
     const size_t hl = mm_lds(1024, mx, m, true, limit, q);
     if (hl <= limit) return {k_mm_chunk<true, 1024>, 1024, hl, q};
     const size_t g = mm_lds(1024, mx, m, false, limit, q);
@@ -2553,8 +2560,10 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
   // terms' energies take a word each; a bonded term has at least 12 table bytes, so
   // table_lds_bytes bounds their number (eval_help takes more in windows). Ten conformers of 48 atoms, BFGS,
   // host work included: 4.28 -> 3.99 ms; 221 chains of 199-329 atoms, L-BFGS: 180 -> 127 ms (151 with
-  // the history in LDS alone); with the bonded tasks' spread terms 3.95 and 116 ms. Above one
-  // conformer per CU the waves of other conformers fill the CU and helpers would only displace them.
+  // the history in LDS alone); with the bonded tasks' spread terms 3.95 and 116 ms. A helped
+  // workgroup takes its CU's twelve waves, so with more conformers than CUs they queue: 257
+  // conformers of 82 atoms, without and with helpers, BFGS 4.28 and 5.70 ms, L-BFGS 4.05 and 5.89;
+  // 600: 6.25 and 10.1, 4.92 and 8.76.
   if (b->n_confs <= di.n_cu && o->table_lds_bytes > 0) {
     const int eb = (o->table_lds_bytes / 12 + 64) & ~63;
     const struct {
@@ -2583,6 +2592,8 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
   // Twelve waves per CU at most, whatever registers a kernel leaves free: the resident Hessians
   // stay in the Infinity Cache, a fourth wave per SIMD gains 1% at best (100,000 ragged conformers
   // 1,084 -> 1,075 ms, 2,500 small ones 13.6 -> 15.0), and callers size their buckets by this grid.
+  // (L-BFGS, which has no Hessian and 109 registers, would gain from sixteen: 8,000 medium conformers
+  // 63.9 -> 54.5 ms, 2,000 chains the same.)
   per_cu = std::min(per_cu, std::max(1, max_wg / pl.help));
   pl.grid = std::max(1, std::min(b->n_confs, di.n_cu * per_cu));
   pl.slot_floats = 0;
@@ -2831,9 +2842,11 @@ int mmffhip_bb_fused(const mmffhip_batch* b, const float* x_in, float* x_out, do
   };
   if (plan(256) > (size_t)di.lds) return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
   KBatch kb = to_kbatch(b);
-  // at most one conformer per CU: sixteen waves each, as in launch_eg. 60 ragged conformers,
-  // 200 steps: 2.19 -> 1.50 ms
-  const int nt = b->n_confs <= di.n_cu && plan(1024) <= (size_t)di.lds ? 1024 : 256;
+  // at most one conformer per CU and molecules that are not small: sixteen waves each, as in
+  // launch_eg. One conformer, 200 steps, four waves and sixteen: 9 atoms 0.46 and 0.53 ms, 33 atoms
+  // 0.57 and 0.57, 82 atoms 1.39 and 0.94, 253 atoms 7.22 and 3.86; 600 conformers of 82 atoms 2.31
+  // and 2.84
+  const int nt = b->n_confs <= di.n_cu && b->max_atoms > 32 && plan(1024) <= (size_t)di.lds ? 1024 : 256;
   const size_t lds = plan(nt);
   const auto kernel = nt == 1024 ? k_bb_fused<1024> : k_bb_fused<256>;
   allow_lds((const void*)kernel, lds);

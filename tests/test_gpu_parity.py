@@ -494,10 +494,11 @@ def test_descent_does_not_depend_on_the_batch():
         assert torch.equal(a[0], b[0][:x.numel()]) and torch.equal(a[1], b[1][:db.n_confs])
 
 
-@pytest.mark.parametrize("families", [("small",), ("small", "chain")])
+@pytest.mark.parametrize("families", [("small",), ("medium",), ("small", "chain")])
 def test_lockstep_does_not_depend_on_the_batch(families):
     """The lock-step L-BFGS of a few conformers and of the same conformers in a batch of more than
-    one per CU (history in LDS for small molecules alone, in memory beside a chain)."""
+    one per CU (history in LDS for small molecules alone, in memory beside a chain; a few small
+    molecules run in narrow workgroups, medium ones and the chain in wide ones)."""
     from mlxmolkit_archive_amd import engine
     db, x, db2, x2 = _few_and_many(families)
     kw = dict(max_iters=60, grad_tol=0.0)
