@@ -433,8 +433,8 @@ __device__ __forceinline__ double eval_terms(const TView& TV, const MolDesc& m, 
 // quarter of the list, so one group after another is one walk over it.
 // 12,139 ragged MEGA energies and gradients: generic loop 143 us, tasks of consecutive terms 123, of
 // spread terms 103, without the sums of kinds 97.5; the Barzilai-Borwein descent of 1,000
-// conformers: 6.08, 4.59, 4.00 ms, with the sums by groups 4.07; the lock-step L-BFGS: 7.00, 6.28,
-// 6.37 ms.
+// conformers: 6.08, 4.59, 4.00 ms, with the sums by groups 4.05; the lock-step L-BFGS: 7.00, 6.28,
+// 6.34 ms.
 constexpr int SUM_LANES = 256, SUM_GROUPS = 4;
 
 // A lane's energy sums: bonded terms, pairs, and each kind of term when PT
@@ -486,20 +486,27 @@ __device__ __forceinline__ LaneSums<PT> eval_tasks(const TView& V, const MolDesc
     const float2 p = V.bond_p[u];
     return t_bond<FAM, G>(xs, acc, (int)(ij & 0xffff), (int)(ij >> 16), p.x, p.y);
   };
+  // a wave's tasks of a group: every NW-th from its first
+  auto first_task = [&](int h) { return GW * h + ((h & 1) ? GW - 1 - wg : wg); };
+  int h = h0, t = first_task(h);
+  double e = 0.0;
+  // task t of kind c, whose tasks are first .. end - 1 and whose terms are n
+  auto one = [&](int c, int first, int end, int n, auto term, double& k) {
+    const int u = lane * (end - first) + (t - first);
+    if ((mask >> c & 1u) && u < n) {
+      const float v = term(u);
+      e += v;
+      if (PT) k += v;
+    }
+  };
+  auto next_group = [&]() {
+    sum.b += e;
+    e = 0.0;
+    if (++h < h1) t = first_task(h);
+  };
+  if constexpr (PT) {
 #pragma unroll 1
-  for (int h = h0; h < h1 && GW * h < t5; h++) {
-    int t = GW * h + ((h & 1) ? GW - 1 - wg : wg);  // a wave's tasks in this group: every NW-th from here
-    double e = 0.0;
-    // task t of kind c, whose tasks are first .. end - 1 and whose terms are n
-    auto one = [&](int c, int first, int end, int n, auto term, double& k) {
-      const int u = lane * (end - first) + (t - first);
-      if ((mask >> c & 1u) && u < n) {
-        const float v = term(u);
-        e += v;
-        if (PT) k += v;
-      }
-    };
-    if constexpr (PT) {
+    while (t < t5) {
       // a loop for each kind, so that one sum of kinds is in the making at a time
       auto all = [&](int c, int first, int end, int n, auto term) {
         double k = 0.0;
@@ -511,17 +518,21 @@ __device__ __forceinline__ LaneSums<PT> eval_tasks(const TView& V, const MolDesc
       all(1, t2, t3, m.na, ang);
       all(3, t3, t4, m.noop, oop);
       all(0, t4, t5, m.nb, bond);
-    } else {
-      double k;
-      for (; t < t5; t += NW) {
-        if (t < t1) one(4, 0, t1, m.ntor, tor, k);
-        else if (t < t2) one(2, t1, t2, m.nsb, sb, k);
-        else if (t < t3) one(1, t2, t3, m.na, ang, k);
-        else if (t < t4) one(3, t3, t4, m.noop, oop, k);
-        else one(0, t4, t5, m.nb, bond, k);
-      }
+      next_group();
     }
-    sum.b += e;
+  } else {
+    // one loop over the groups' tasks and one over their pairs below (a loop in a loop each: the
+    // descent of 1,000 conformers 4.07 ms, so 4.05)
+    double k;
+    while (t < t5) {
+      if (t < t1) one(4, 0, t1, m.ntor, tor, k);
+      else if (t < t2) one(2, t1, t2, m.nsb, sb, k);
+      else if (t < t3) one(1, t2, t3, m.na, ang, k);
+      else if (t < t4) one(3, t3, t4, m.noop, oop, k);
+      else one(0, t4, t5, m.nb, bond, k);
+      t += NW;
+      if (t >= t5) next_group();
+    }
   }
   if (!(mask & 96u) || m.npair <= 0) return sum;
   // eval_pairs' walk, two pairs per lane and step
@@ -553,21 +564,21 @@ __device__ __forceinline__ LaneSums<PT> eval_tasks(const TView& V, const MolDesc
   unsigned s = min(h0 * per, steps);
   const unsigned end = min(h1 * per, steps), full = min(end, steps - 1);
   if (s < end) {
-    unsigned u = s * STEP + (threadIdx.x & (SUM_LANES - 1)), stop = ALL ? per : end;  // this group's end
+    unsigned u = s * STEP + (threadIdx.x & (SUM_LANES - 1)), left = per;  // steps left of this group
     Pair pa = row(u), pb = row(u + SUM_LANES);
-    for (;; stop += per) {
-      for (const unsigned lim = min(stop, full); s < lim; s++) {
-        const Pair na = row(u + STEP), nb = row(u + STEP + SUM_LANES);
-        term(pa);
-        term(pb);
-        pa = na;
-        pb = nb;
-        u += STEP;
+    for (; s < full; s++) {
+      const Pair na = row(u + STEP), nb = row(u + STEP + SUM_LANES);
+      term(pa);
+      term(pb);
+      pa = na;
+      pb = nb;
+      u += STEP;
+      if (ALL && --left == 0) {
+        close();
+        left = per;
       }
-      if (!ALL || s < stop) break;  // the list's last step, if any is left, is this group's too
-      close();
     }
-    if (s < end) {
+    if (s < end) {  // the list's last step
       if (u < np) term(pa);
       if (u + SUM_LANES < np) term(pb);
     }
@@ -1931,6 +1942,8 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
 // BB fused steepest descent, MEGA family: mmff_metal_kernel.py:845-1075.
 // NR: threads of the workgroup. The first 256 do everything but the evaluation, which all share.
 // g_bytes: the gradient's LDS, where the groups' sums meet during an evaluation.
+// A step waits for the cleared sums, the energy and the step's dot products; 1,000 conformers 4.11 ms
+// with two more barriers, 4.07 with these three.
 template <int NR>
 __global__ void __launch_bounds__(NR) k_bb_fused(KBatch B, const float* __restrict__ x_in, float* x_out,
                                                  double* e_out, int max_it, float max_step, float grad_lr,
@@ -1979,22 +1992,27 @@ __global__ void __launch_bounds__(NR) k_bb_fused(KBatch B, const float* __restri
       }
       R.template run<2, 0>(v2);
       if (v2[1] > 1e-20) alpha = fminf(fmaxf((float)(v2[0] / v2[1]), 1e-6f), 0.3f);
+    } else {
+      __syncthreads();
     }
     E_prev = E;
-    for (int i = tid; i < n; i += NT) {
-      pp[i] = xs[i];
-      pg[i] = g[i];
-    }
-    __syncthreads();
-    for (int a = tid; a < m.n_atoms; a += NT) {  // per-atom capped step :1063-1071
+    // per-atom capped step :1063-1071; g is behind the barrier above, and the one behind the clearing
+    // of gacc follows before anybody reads what is written here
+    for (int a = tid; a < m.n_atoms; a += NT) {
+      float *x = xs + 3 * a, *xp = pp + 3 * a, *gp = pg + 3 * a;
       const float gx = g[3 * a], gy = g[3 * a + 1], gz = g[3 * a + 2];
       const float gn = sqrtf(gx * gx + gy * gy + gz * gz + 1e-30f);
       const float s = fminf(max_step / gn, alpha);
-      xs[3 * a] -= s * gx;
-      xs[3 * a + 1] -= s * gy;
-      xs[3 * a + 2] -= s * gz;
+      xp[0] = x[0];
+      xp[1] = x[1];
+      xp[2] = x[2];
+      gp[0] = gx;
+      gp[1] = gy;
+      gp[2] = gz;
+      x[0] -= s * gx;
+      x[1] -= s * gy;
+      x[2] -= s * gz;
     }
-    __syncthreads();
   }
   __syncthreads();
   for (int i = tid; i < n; i += NT) x_out[off + i] = xs[i];
@@ -2214,7 +2232,6 @@ __global__ void __launch_bounds__(NR, NR > 256 ? 1 : 4) k_mm_chunk(KBatch B, MMS
       xn[3 * a + 1] = xs[3 * a + 1] + dy * f;
       xn[3 * a + 2] = xs[3 * a + 2] + dz * f;
     }
-    __syncthreads();
     mm_eval<NR>(B, m, xn, gacc, R, E, n, (double*)q, room);
     // push (s, y, rho) into the ring (:385-399); rho = 0 on bad curvature
     int sl;
@@ -2242,9 +2259,8 @@ __global__ void __launch_bounds__(NR, NR > 256 ? 1 : 4) k_mm_chunk(KBatch B, MMS
     if (tid == 0) {
       const double r = sy[0] > 1e-10 ? 1.0 / (sy[0] + 1e-30) : 0.0;
       if (HL) lrho[sl] = r;
-      S.rho[(size_t)sl * B.n_confs + c] = r;
+      S.rho[(size_t)sl * B.n_confs + c] = r;  // read behind the next step's first reduction
     }
-    __syncthreads();
   }
   if (do_sync) {
     // best-x guard (:408-412) and convergence (:354-359 main, :477-481 polish)
