@@ -2408,7 +2408,7 @@ size_t eg_lds(int nt, int max_atoms, bool terms, size_t limit, int& xs_bytes, in
 // size on where that gains more than four groups' meeting in LDS costs; four waves otherwise. TG
 // energy and gradient of one conformer, us from launch to launch, four and sixteen waves: 9 atoms 3.6
 // and 4.2, 34 atoms 4.6 and 4.7, 82 atoms 8.0 and 6.4, 253 atoms 36.4 and 20.3; with kinds 4.4 and 5.8, 5.2
-// and 6.3, 8.6 and 7.9, 36.6 and 21.8. (The Python entry point's host work takes 10 us a call.) A
+// and 6.3, 8.6 and 7.9, 36.6 and 21.8. (The Python entry point's host work takes 7.5 us a call.) A
 // wide workgroup fills its CU, so with more conformers than CUs they queue: 300 conformers of 82
 // atoms 10.3 and 11.8 us, 768: 12.7 and 17.3.
 template <int FAM, bool PT>

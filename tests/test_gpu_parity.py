@@ -605,3 +605,20 @@ def test_lockstep_wide_workgroups_at_the_lds_limit(waters):
     assert torch.isfinite(a["energy"]).all() and not torch.equal(a["x"], torch.from_numpy(x).cuda())
     assert torch.equal(a["x"], b["x"][:len(x)]) and torch.equal(a["energy"], b["energy"][:2])
     assert torch.equal(a["grad_norm"], b["grad_norm"][:2])
+
+
+def test_calls_follow_the_current_stream():
+    """The stream handle that calls take is torch's current stream's: the default one, a side stream's
+    inside its context, also in nested ones, or the one given."""
+    from mlxmolkit_archive_amd import _lib
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    want = lambda: int(torch.cuda.current_stream().cuda_stream)  # noqa: E731
+    base = _lib.stream_ptr()
+    assert base == want()
+    with torch.cuda.stream(a):
+        assert _lib.stream_ptr() == want() == int(a.cuda_stream) != base
+        with torch.cuda.stream(b):
+            assert _lib.stream_ptr() == want() == int(b.cuda_stream)
+            assert _lib.stream_ptr(a) == int(a.cuda_stream)
+        assert _lib.stream_ptr() == int(a.cuda_stream)
+    assert _lib.stream_ptr() == want() == base
