@@ -1091,13 +1091,16 @@ __device__ __forceinline__ float h_init(const float* pc, float psc, int i, int j
 // pairs read from global memory (2). Global-Hessian kernels of up to 256 threads are compiled
 // for three waves per SIMD (at most 168 VGPRs), so three workgroups share a CU: their LDS
 // use is small, and the extra resident conformers hide memory latency better than the
-// registers the compiler would otherwise use (medium workload: 172.6 against 178.5 ms).
+// registers the compiler would otherwise use (medium workload: 172.6 against 178.5 ms). One wave with
+// everything in LDS is held to them too, where it would take 178-186: 18,000 conformers of 9-14 atoms
+// 4.38 -> 3.67 ms (L-BFGS 6.66 -> 5.29), 8,000 of 26 atoms, which LDS limits first, 11.1 and 11.2.
 // HELP: a conformer's workgroup has HELP * NT threads, of which the first NT do all that NT threads
 // do and the others share the term evaluation (eval_help): same results, shorter iterations.
 // For batches of at most one conformer per CU, whose time is the longest conformer's chain of
 // iterations. Three times 256 threads keep three waves per SIMD and their 168 registers.
 template <int ALGO, int HM, int TL, int NT, int HELP = 1>
-__global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256) ? (HELP > 1 ? 1 : 3) : 1)
+__global__ void __launch_bounds__(
+    NT * HELP, HELP == 1 && (((HM == 1 || HM == 3) && NT <= 256) || (TL == 1 && NT == 64)) ? 3 : 1)
     k_minimize_nk(KBatch B, NkParams P) {
   constexpr bool HLDS = HM == 0;    // LDS-resident (also selects the LDS L-BFGS history)
   constexpr bool PACKED = HM == 0 || HM == 2;  // packed upper triangle, select read + column-pair write-back
@@ -1540,9 +1543,9 @@ __global__ void __launch_bounds__(NT * HELP, ((HM == 1 || HM == 3) && NT <= 256)
           float4* H4 = (float4*)H;
           // The next block's four rows are loaded while this one is used: a step is one load
           // latency long otherwise, with three waves per SIMD to cover it. 100,000 ragged
-          // conformers 1,134 -> 1,095 ms. (The 16 registers for it came free with the uniform
-          // reduction results and the shorter pair loop; before them it spilled 76-244 bytes per
-          // lane and lost 5%.)
+          // conformers 1,134 -> 1,095 ms. (Before the uniform reduction results and the shorter pair
+          // loop its 16 registers spilled 76-244 bytes per lane and lost 5%; now they cost the kernels
+          // of 128 and 256 threads with staged tables 20 and 28 bytes, the others none.)
           //
           // one block of a lane's walk: its quads, whether it is kept, and its first row
           struct Item {

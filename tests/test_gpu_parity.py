@@ -622,3 +622,30 @@ def test_calls_follow_the_current_stream():
             assert _lib.stream_ptr(a) == int(a.cuda_stream)
         assert _lib.stream_ptr() == int(a.cuda_stream)
     assert _lib.stream_ptr() == want() == base
+
+
+@pytest.mark.parametrize("use_lbfgs", [False, True])
+def test_one_wave_with_everything_in_lds(use_lbfgs):
+    """One wave per conformer with matrix (or history) and tables in LDS: for small molecules, whose LDS
+    leaves the room, registers for twelve workgroups per CU. BFGS has the bits of the same kernel
+    without staged tables; L-BFGS, which has no such kernel, stays within 1e-4 A of two waves' over
+    three iterations (steps of at most an angstrom, whose FP64 sums in another order move them by
+    about an FP32 rounding each)."""
+    from mlxmolkit_archive_amd import _lib, engine
+    _, p, x = conftest.mol_params("CCO", seed=4, k=2)
+    db, xd = engine.device_batch([p], [600]), torch.from_numpy(np.tile(x, 300)).cuda()
+    kw = dict(max_iters=3 if use_lbfgs else 200, grad_tol=1e-4, use_lbfgs=use_lbfgs, ls_grad=True, min_fill=0)
+    r = engine.NkRunner(db, buckets=((1 << 20, 64, _lib.HESS_LDS),), **kw)
+    ln, = r.launches
+    assert ln["opts"].table_lds_bytes > 0 and ln["placement"] == _lib.HESS_LDS
+    n_cu = torch.cuda.get_device_properties(0).multi_processor_count
+    assert engine.resident_workgroups(ln["desc"], ln["opts"]) == 12 * n_cu
+    got = r.run(xd)
+    want = engine.NkRunner(db, buckets=((1 << 20, 128 if use_lbfgs else 64, _lib.HESS_LDS),), stage_tables=False,
+                           **kw).run(xd)
+    torch.cuda.synchronize()
+    assert not torch.equal(got.x, xd)
+    if use_lbfgs:
+        assert torch.allclose(got.x, want.x, rtol=0, atol=1e-4)
+    else:
+        assert torch.equal(got.x, want.x) and torch.equal(got.energy, want.energy) and (got.status == 0).all()
