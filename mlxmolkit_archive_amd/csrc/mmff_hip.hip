@@ -2363,11 +2363,12 @@ struct DevInfo {
 };
 
 DevInfo dev_info() {
-  static thread_local DevInfo cache[16];
+  constexpr int CACHED = 64;  // a node of eight GPUs in eight partitions each
+  static thread_local DevInfo cache[CACHED];
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return DevInfo{};
-  if (dev < 0 || dev >= 16) return DevInfo{};
-  DevInfo& di = cache[dev];
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return DevInfo{};
+  DevInfo fresh;
+  DevInfo& di = dev < CACHED ? cache[dev] : fresh;
   if (!di.ok) {
     hipDeviceProp_t p;
     if (hipGetDeviceProperties(&p, dev) == hipSuccess) {
