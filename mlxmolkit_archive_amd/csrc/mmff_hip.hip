@@ -926,10 +926,9 @@ constexpr int RED_WORDS = 2 * (SUM_LANES / 64) * 8;  // doubles of a Reducer<SUM
 // what the nk kernel evaluates (mmff_bfgs_header.metal).
 // The groups' sums meet in LDS behind the positions (xs_bytes), room values at a time, or where the
 // positions were when room is 0 (xs_bytes then hold one value at least)
-// The narrow kernels with kinds are held to 7 and 5 waves per SIMD (TG, MEGA), which they miss by a
-// register or two: 12,139 ragged MEGA energies with kinds 73.7 us, 80.1 at four
+// Registers let 8 (TG) and 6 (MEGA) waves onto a SIMD, 7 and 5 with kinds.
 template <int FAM, bool PT, int NT>
-__global__ void __launch_bounds__(NT, NT == 256 ? (FAM == FAM_TG ? 7 : 5) : 4) k_energy_grad(KBatch B, const float* __restrict__ x, double* e_out,
+__global__ void __launch_bounds__(NT) k_energy_grad(KBatch B, const float* __restrict__ x, double* e_out,
                                                     double* e_terms, float* g_out, uint32_t mask, int diel,
                                                     int xs_bytes, int room) {
   extern __shared__ __align__(16) unsigned char smem[];
