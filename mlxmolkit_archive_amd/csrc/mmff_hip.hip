@@ -433,8 +433,8 @@ __device__ __forceinline__ double eval_terms(const TView& TV, const MolDesc& m, 
 // quarter of the list, so one group after another is one walk over it.
 // 12,139 ragged MEGA energies and gradients: generic loop 143 us, tasks of consecutive terms 123, of
 // spread terms 103, without the sums of kinds 97.5; the Barzilai-Borwein descent of 1,000
-// conformers: 6.08, 4.59, 4.00 ms, with the sums by groups 4.05; the lock-step L-BFGS: 7.00, 6.28,
-// 6.34 ms.
+// conformers: 6.08, 4.59, 4.00 ms, and again 4.00 with the sums by groups; the lock-step L-BFGS: 7.00,
+// 6.28, 6.26 ms.
 constexpr int SUM_LANES = 256, SUM_GROUPS = 4;
 
 // A lane's energy sums: bonded terms, pairs, and each kind of term when PT
@@ -1943,23 +1943,24 @@ __global__ void __launch_bounds__(
 // ------------------------------------------------------------------------------------
 // BB fused steepest descent, MEGA family: mmff_metal_kernel.py:845-1075.
 // NR: threads of the workgroup. The first 256 do everything but the evaluation, which all share.
-// g_bytes: the gradient's LDS, where the groups' sums meet during an evaluation.
-// A step waits for the cleared sums, the energy and the step's dot products; 1,000 conformers 4.11 ms
-// with two more barriers, 4.07 with these three.
+// ex_bytes: LDS where the groups' sums meet during an evaluation.
+// The gradient is taken from its sums where it is used, and the pass that moves an atom clears them,
+// so a step waits for the positions, the energy and the step's dot products only. 1,000 conformers: 4.11 ms
+// with a gradient and a clearing pass of their own and three more barriers, 4.00 so.
 template <int NR>
 __global__ void __launch_bounds__(NR) k_bb_fused(KBatch B, const float* __restrict__ x_in, float* x_out,
                                                  double* e_out, int max_it, float max_step, float grad_lr,
-                                                 int g_bytes) {
+                                                 int ex_bytes) {
   extern __shared__ __align__(16) unsigned char smem[];
   constexpr int NT = SUM_LANES;
   const int c = blockIdx.x;
   if (c >= B.n_confs) return;
   const int tid = NR == NT || threadIdx.x < NT ? (int)threadIdx.x : 1 << 30;
-  const int mx = 3 * B.max_atoms, room = g_bytes / (EX_WORDS * (int)sizeof(double));
+  const int mx = 3 * B.max_atoms, room = ex_bytes / (EX_WORDS * (int)sizeof(double));
   double* red = (double*)smem;
   unsigned long long* gacc = (unsigned long long*)(red + RED_WORDS);
-  float* g = (float*)(gacc + mx);
-  float* xs = (float*)((char*)g + g_bytes);
+  double* buf = (double*)(gacc + mx);
+  float* xs = (float*)((char*)buf + ex_bytes);
   float* pp = xs + mx;
   float* pg = pp + mx;
   const MolDesc m = load_desc(B.mol_desc + 16 * B.conf_mol[c]);
@@ -1969,42 +1970,41 @@ __global__ void __launch_bounds__(NR) k_bb_fused(KBatch B, const float* __restri
     xs[i] = x_in[off + i];
     pp[i] = xs[i];
     pg[i] = 0.f;
+    gacc[i] = 0ull;
   }
   Reducer<NT, 8, (NR > NT)> R{red, 0};
   float alpha = grad_lr;
   double E_prev = 1e30, E = 0.0;
   for (int it = 0; it < max_it; it++) {
-    for (int i = threadIdx.x; i < n; i += NR) gacc[i] = 0ull;
     __syncthreads();
-    E = group_energy<NR>(eval_tasks<FAM_MEGA, true, false, false, NR>(global_view(B, m), m, xs, gacc, 1, 0x7fu), (double*)g,
-                         room, R);
+    E = group_energy<NR>(eval_tasks<FAM_MEGA, true, false, false, NR>(global_view(B, m), m, xs, gacc, 1, 0x7fu), buf, room, R);
     if (it > 0 && E > E_prev + 1.0) {  // energy guard :1031-1038
-      for (int i = tid; i < n; i += NT) xs[i] = pp[i];
+      for (int i = tid; i < n; i += NT) {
+        xs[i] = pp[i];
+        gacc[i] = 0ull;
+      }
       alpha = fmaxf(alpha * 0.5f, 1e-7f);
       E = E_prev;
       continue;
     }
-    for (int i = tid; i < n; i += NT) g[i] = from_fx(gacc[i]);
     if (it > 0) {  // BB step :1041-1052
       double v2[2] = {0.0, 0.0};
       for (int i = tid; i < n; i += NT) {
-        const float si = xs[i] - pp[i], yi = g[i] - pg[i];
+        const float si = xs[i] - pp[i], yi = from_fx(gacc[i]) - pg[i];
         v2[0] += (double)si * si;
         v2[1] += (double)si * yi;
       }
       R.template run<2, 0>(v2);
       if (v2[1] > 1e-20) alpha = fminf(fmaxf((float)(v2[0] / v2[1]), 1e-6f), 0.3f);
-    } else {
-      __syncthreads();
     }
     E_prev = E;
-    // per-atom capped step :1063-1071; g is behind the barrier above, and the one behind the clearing
-    // of gacc follows before anybody reads what is written here
-    for (int a = tid; a < m.n_atoms; a += NT) {
+    for (int a = tid; a < m.n_atoms; a += NT) {  // per-atom capped step :1063-1071
       float *x = xs + 3 * a, *xp = pp + 3 * a, *gp = pg + 3 * a;
-      const float gx = g[3 * a], gy = g[3 * a + 1], gz = g[3 * a + 2];
+      unsigned long long* ga = gacc + 3 * a;
+      const float gx = from_fx(ga[0]), gy = from_fx(ga[1]), gz = from_fx(ga[2]);
       const float gn = sqrtf(gx * gx + gy * gy + gz * gz + 1e-30f);
       const float s = fminf(max_step / gn, alpha);
+      ga[0] = ga[1] = ga[2] = 0ull;
       xp[0] = x[0];
       xp[1] = x[1];
       xp[2] = x[2];
@@ -2043,10 +2043,10 @@ struct MMState {
   size_t total;
 };
 
+// the gradient sums come cleared; starts with a barrier, and ends with one
 template <int NR, class Red>
 __device__ void mm_eval(const KBatch& B, const MolDesc& m, float* xs, unsigned long long* gacc, Red& R, double& E,
-                        int n, double* buf = nullptr, int room = 0) {
-  for (int i = threadIdx.x; i < n; i += NR) gacc[i] = 0ull;
+                        double* buf = nullptr, int room = 0) {
   __syncthreads();
   E = group_energy<NR>(eval_tasks<FAM_MEGA, true, false, false, NR>(global_view(B, m), m, xs, gacc, 1, 0x7fu), buf, room, R);
 }
@@ -2066,10 +2066,13 @@ __global__ void __launch_bounds__(NT) k_mm_init(KBatch B, MMState S, const float
   float* xs = (float*)(gacc + mx);
   const MolDesc m = load_desc(B.mol_desc + 16 * B.conf_mol[c]);
   const int n = 3 * m.n_atoms, off = B.conf_off[c];
-  for (int i = threadIdx.x; i < n; i += NT) xs[i] = mode == 0 ? x_in[off + i] : S.bx[off + i];
+  for (int i = threadIdx.x; i < n; i += NT) {
+    xs[i] = mode == 0 ? x_in[off + i] : S.bx[off + i];
+    gacc[i] = 0ull;
+  }
   Reducer<NT> R{red, 0};
   double E;
-  mm_eval<NT>(B, m, xs, gacc, R, E, n);
+  mm_eval<NT>(B, m, xs, gacc, R, E);
   for (int i = threadIdx.x; i < n; i += NT) {
     S.x[off + i] = xs[i];
     S.g[off + i] = from_fx(gacc[i]) * gsc;
@@ -2106,9 +2109,10 @@ size_t mm_lds(int nr, int mx, int m, bool hl, size_t limit, int& q_bytes) {
 
 // HL: the (s, y) history is worked on in LDS for the launch's iterations (and written through to
 // the workspace, which the next launch reads); from memory, each of an iteration's 2 len + 1
-// dependent passes waited for its loads. Each lane meets only its own coordinates of it, so it
-// needs no barrier. 128 registers put four workgroups on a CU. 1,000 conformers of 69 atoms on
-// average, 200 + 50 iterations: 6.28 ms, 10.7 ms with the history read from memory and one loop
+// dependent passes waited for its loads. Each lane meets only its own coordinates of it (but for
+// the step over atoms, which comes behind the reductions' barriers), so it needs no barrier of its
+// own. 128 registers put four workgroups on a CU. 1,000 conformers of 69 atoms on
+// average, 200 + 50 iterations: 6.26 ms, 10.7 ms with the history read from memory and one loop
 // over all term types. Of that, measured before the reductions by readlane and the spread terms:
 // 7.4 ms; 9.1 ms with three workgroups per CU, 10.5 ms with the history in memory. Dropped: the
 // recursion in one wave while the others wait (the same sums without barriers: 7.6 against 7.4 ms,
@@ -2149,6 +2153,7 @@ __global__ void __launch_bounds__(NR, NR > 256 ? 1 : 4) k_mm_chunk(KBatch B, MMS
   for (int i = tid; i < n; i += NT) {
     xs[i] = S.x[off + i];
     gs[i] = S.g[off + i];
+    gacc[i] = 0ull;
   }
   auto rho = [&](int k) { return HL ? lrho[k] : S.rho[(size_t)k * B.n_confs + c]; };
   if (HL) {
@@ -2167,10 +2172,11 @@ __global__ void __launch_bounds__(NR, NR > 256 ? 1 : 4) k_mm_chunk(KBatch B, MMS
     // two-loop direction, mmff_metal_optimizer.py:47-74 (history oldest -> newest), with each
     // axpy fused into the next dot product's pass, gamma's dots into the first pass and the
     // gamma scaling into the first loop's last axpy: the same FP32 updates of q and FP64 dot
-    // products as running the passes one by one (bit-identical), in 2 len + 1 passes.
+    // products as running the passes one by one (bit-identical), in 2 len + 1 passes with the step.
+    int sl = head + len - 1;  // newest entry
+    if (sl >= M) sl -= M;
+    float cf = 0.f;
     if (len > 0) {
-      int sl = head + len - 1;  // newest entry
-      if (sl >= M) sl -= M;
       double v3[3];
       block_dots<NT, 3>(R, tid, n, v3, [&](int i, double (&p)[3]) {
         const float qv = gs[i];
@@ -2207,36 +2213,30 @@ __global__ void __launch_bounds__(NR, NR > 256 ? 1 : 4) k_mm_chunk(KBatch B, MMS
           p[0] += (double)y * qv;
         });  // its barrier also makes alf visible
       }
-      for (int h = 0; h < len; h++) {  // q += (alpha_h - beta_h) s_h, then y_{h+1}.q
-        const float cf = (float)(alf[h] - rho(sl) * yr[0]);
+      for (int h = 0;; h++) {  // q += (alpha_h - beta_h) s_h, then y_{h+1}.q
+        cf = (float)(alf[h] - rho(sl) * yr[0]);
+        if (h + 1 == len) break;  // the last axpy goes with the step
         const int sn = sl + 1 == M ? 0 : sl + 1;
-        if (h + 1 < len) {
-          block_dots<NT, 1>(R, tid, n, yr, [&](int i, double (&p)[1]) {
-            const float r = q[i] + cf * hS[sl * HT + i];
-            q[i] = r;
-            p[0] += (double)hY[sn * HT + i] * r;
-          });
-        } else {
-          for (int i = tid; i < n; i += NT) q[i] += cf * hS[sl * HT + i];
-        }
+        block_dots<NT, 1>(R, tid, n, yr, [&](int i, double (&p)[1]) {
+          const float r = q[i] + cf * hS[sl * HT + i];
+          q[i] = r;
+          p[0] += (double)hY[sn * HT + i] * r;
+        });
         sl = sn;
       }
-    } else {
-      for (int i = tid; i < n; i += NT) q[i] = gs[i];
     }
-    __syncthreads();
     // d = -q with the per-atom cap of max_step (:365-373); x_new = x + d
+    auto dir = [&](int i) { return len > 0 ? -(q[i] + cf * hS[sl * HT + i]) : -gs[i]; };
     for (int a = tid; a < m.n_atoms; a += NT) {
-      const float dx = -q[3 * a], dy = -q[3 * a + 1], dz = -q[3 * a + 2];
+      const float dx = dir(3 * a), dy = dir(3 * a + 1), dz = dir(3 * a + 2);
       const float disp = sqrtf(dx * dx + dy * dy + dz * dz + 1e-30f);
       const float f = fminf(max_step / disp, 1.0f);
       xn[3 * a] = xs[3 * a] + dx * f;
       xn[3 * a + 1] = xs[3 * a + 1] + dy * f;
       xn[3 * a + 2] = xs[3 * a + 2] + dz * f;
     }
-    mm_eval<NR>(B, m, xn, gacc, R, E, n, (double*)q, room);
+    mm_eval<NR>(B, m, xn, gacc, R, E, (double*)q, room);
     // push (s, y, rho) into the ring (:385-399); rho = 0 on bad curvature
-    int sl;
     if (len >= M) {
       sl = head;
       head = head + 1 == M ? 0 : head + 1;
@@ -2247,6 +2247,7 @@ __global__ void __launch_bounds__(NR, NR > 256 ? 1 : 4) k_mm_chunk(KBatch B, MMS
     double sy[1];
     block_dots<NT, 1>(R, tid, n, sy, [&](int i, double (&p)[1]) {
       const float gn = from_fx(gacc[i]) * gsc;
+      gacc[i] = 0ull;  // for the next evaluation
       const float s = xn[i] - xs[i], y = gn - gs[i];
       hS[sl * HT + i] = s;
       hY[sl * HT + i] = y;
@@ -2853,24 +2854,22 @@ int mmffhip_bb_fused(const mmffhip_batch* b, const float* x_in, float* x_out, do
   if (!x_in || !x_out || !e_out) return fail(MMFFHIP_ERR_ARG, "x_in, x_out and e_out are required");
   if (max_iters < 0) return fail(MMFFHIP_ERR_ARG, "max_iters must be >= 0");
   const DevInfo di = dev_info();
-  int g_bytes = 0;
-  auto plan = [&](int nt) {
-    const size_t rest = RED_WORDS * 8 + (size_t)3 * b->max_atoms * (8 + 3 * 4) + 16;
-    g_bytes = (int)ex_area(nt, (size_t)3 * b->max_atoms * 4, 2, rest, di.lds);
-    return rest + g_bytes;
-  };
-  if (plan(256) > (size_t)di.lds) return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
+  const size_t rest = RED_WORDS * 8 + (size_t)3 * b->max_atoms * (8 + 3 * 4) + 16;
+  // the largest molecule is what it was when the LDS held the gradient too
+  if (rest + (size_t)3 * b->max_atoms * 4 > (size_t)di.lds)
+    return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
   KBatch kb = to_kbatch(b);
   // at most one conformer per CU and molecules that are not small: sixteen waves each, as in
   // launch_eg. One conformer, 200 steps, four waves and sixteen: 9 atoms 0.46 and 0.53 ms, 33 atoms
   // 0.57 and 0.57, 82 atoms 1.39 and 0.94, 253 atoms 7.22 and 3.86; 600 conformers of 82 atoms 2.31
   // and 2.84
-  const int nt = b->n_confs <= di.n_cu && b->max_atoms > 32 && plan(1024) <= (size_t)di.lds ? 1024 : 256;
-  const size_t lds = plan(nt);
-  const auto kernel = nt == 1024 ? k_bb_fused<1024> : k_bb_fused<256>;
-  allow_lds((const void*)kernel, lds);
-  hipLaunchKernelGGL(kernel, dim3(b->n_confs), dim3(nt), lds, (hipStream_t)stream, kb, x_in, x_out, e_out,
-                     (int)max_iters, max_step, grad_lr, g_bytes);
+  const size_t wide_ex = ex_area(1024, 0, 2, rest, di.lds);
+  const bool wide = b->n_confs <= di.n_cu && b->max_atoms > 32 && rest + wide_ex <= (size_t)di.lds;
+  const size_t ex = wide ? wide_ex : 0;
+  const auto kernel = wide ? k_bb_fused<1024> : k_bb_fused<256>;
+  allow_lds((const void*)kernel, rest + ex);
+  hipLaunchKernelGGL(kernel, dim3(b->n_confs), dim3(wide ? 1024 : 256), rest + ex, (hipStream_t)stream, kb, x_in, x_out,
+                     e_out, (int)max_iters, max_step, grad_lr, (int)ex);
   HIP_TRY(hipGetLastError());
   return MMFFHIP_OK;
 }
