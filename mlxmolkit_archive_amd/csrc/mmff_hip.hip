@@ -2410,11 +2410,11 @@ size_t eg_lds(int nt, int max_atoms, bool terms, size_t limit, int& xs_bytes, in
 
 // At most one conformer per CU: sixteen waves per conformer, whose latency is the call's, from the
 // size on where that gains more than four groups' meeting in LDS costs; four waves otherwise. TG
-// energy and gradient of one conformer, us from launch to launch, four and sixteen waves: 9 atoms 3.6
-// and 4.2, 34 atoms 4.6 and 4.7, 82 atoms 8.0 and 6.4, 253 atoms 36.4 and 20.3; with kinds 4.4 and 5.8, 5.2
-// and 6.3, 8.6 and 7.9, 36.6 and 21.8. (The Python entry point's host work takes 7.5 us a call.) A
-// wide workgroup fills its CU, so with more conformers than CUs they queue: 300 conformers of 82
-// atoms 10.3 and 11.8 us, 768: 12.7 and 17.3.
+// energy and gradient of one conformer, us from launch to launch in a graph, four and sixteen waves: 9 atoms
+// 3.1 and 3.6, 34 atoms 3.6 and 3.9, 42 atoms 4.2 and 3.9, 82 atoms 7.4 and 5.5, 253 atoms 38.0 and 19.7; with kinds
+// 3.6 and 5.2, 4.3 and 5.7, 4.9 and 5.7, 8.0 and 7.2, 38.4 and 21.5 (63 atoms 6.0 and 6.1). (The Python entry point's host
+// work takes 7.5 us a call.) A wide workgroup fills its CU, so with more conformers than CUs they
+// queue: 300 conformers of 82 atoms 9.6 and 10.3 us, 768: 11.8 and 15.4.
 template <int FAM, bool PT>
 int launch_eg(const KBatch& kb, const float* x, double* e, double* et, float* g, uint32_t mask, int diel,
               hipStream_t s) {
@@ -2436,10 +2436,10 @@ int launch_eg(const KBatch& kb, const float* x, double* e, double* et, float* g,
 }
 
 // The launch of k_mm_chunk: wide workgroups when there is at most one conformer per CU and the
-// molecules are not small, as in launch_eg (one conformer, 100 + 25 iterations, narrow and wide: 34 atoms 1.34
-// and 1.47 ms, 48 atoms 1.47 and 1.52, 82 atoms 1.89 and 1.76, 253 atoms 6.49 and 3.99; 257 conformers
-// of 82 atoms 2.29 and 3.46 ms); the history in LDS when it fits there, or leaves three workgroups
-// per CU.
+// molecules are not small, as in launch_eg (one conformer, 100 + 25 iterations, narrow and wide: 9 atoms 0.63
+// and 0.74 ms, 34 atoms 1.19 and 1.37, 57 atoms 1.43 and 1.45, 63 atoms 1.47 and 1.46, 82 atoms 1.77 and 1.61, 253
+// atoms 6.64 and 3.90; 300 conformers of 82 atoms 2.17 and 3.25 ms); the history in LDS when it fits
+// there, or leaves three workgroups per CU.
 struct MMChunk {
   void (*kernel)(KBatch, MMState, int, int, int, int, const int32_t*, int32_t*, int, float, float, float, int);
   int nr;
@@ -2449,7 +2449,7 @@ struct MMChunk {
 MMChunk mm_chunk_plan(int n_confs, int mx, int m, const DevInfo& di) {
   const size_t limit = (size_t)di.lds;
   int q = 0;
-  if (n_confs <= di.n_cu && mx > 3 * 56) {
+  if (n_confs <= di.n_cu && mx > 3 * 60) {
     const size_t hl = mm_lds(1024, mx, m, true, limit, q);
     if (hl <= limit) return {k_mm_chunk<true, 1024>, 1024, hl, q};
     const size_t g = mm_lds(1024, mx, m, false, limit, q);
@@ -2860,11 +2860,12 @@ int mmffhip_bb_fused(const mmffhip_batch* b, const float* x_in, float* x_out, do
     return fail(MMFFHIP_ERR_SIZE, "molecule too large for the LDS of one workgroup");
   KBatch kb = to_kbatch(b);
   // at most one conformer per CU and molecules that are not small: sixteen waves each, as in
-  // launch_eg. One conformer, 200 steps, four waves and sixteen: 9 atoms 0.46 and 0.53 ms, 33 atoms
-  // 0.57 and 0.57, 82 atoms 1.39 and 0.94, 253 atoms 7.22 and 3.86; 600 conformers of 82 atoms 2.31
-  // and 2.84
+  // launch_eg. One conformer, 200 steps, four waves and sixteen: 9 atoms 0.43 and 0.55 ms, 33 atoms
+  // 0.46 and 0.58 (one step of pairs), 36 atoms 0.57 and 0.59, 39 atoms 0.58 and 0.59 or 0.68 and 0.63 (a chain; three
+  // rings), 48 atoms 0.69 and 0.66, 82 atoms 1.28 and 0.91, 253 atoms 7.35 and 3.98; 300 conformers of 82 atoms 1.68
+  // and 1.84
   const size_t wide_ex = ex_area(1024, 0, 2, rest, di.lds);
-  const bool wide = b->n_confs <= di.n_cu && b->max_atoms > 32 && rest + wide_ex <= (size_t)di.lds;
+  const bool wide = b->n_confs <= di.n_cu && b->max_atoms > 38 && rest + wide_ex <= (size_t)di.lds;
   const size_t ex = wide ? wide_ex : 0;
   const auto kernel = wide ? k_bb_fused<1024> : k_bb_fused<256>;
   allow_lds((const void*)kernel, rest + ex);
