@@ -1087,7 +1087,8 @@ __device__ __forceinline__ float h_init(const float* pc, float psc, int i, int j
 
 // HM: where the dense inverse Hessian lives -- 0 packed in LDS, 1 full in HBM, 2 packed in HBM
 // TL: term tables read from global memory (0), staged in LDS (1), or bonded tables staged and
-// pairs read from global memory (2). Global-Hessian kernels of up to 256 threads are compiled
+// pairs read from global memory (2; 3: likewise, but a molecule whose bonded tables are larger than
+// the reserve has them read from global memory too, by a second copy of the evaluation). Global-Hessian kernels of up to 256 threads are compiled
 // for three waves per SIMD (at most 168 VGPRs), so three workgroups share a CU: their LDS
 // use is small, and the extra resident conformers hide memory latency better than the
 // registers the compiler would otherwise use (medium workload: 172.6 against 178.5 ms). One wave with
@@ -1200,8 +1201,9 @@ __global__ void __launch_bounds__(
     while (lsh2 < 3 && (np << (lsh2 + 1)) <= NT) lsh2++;
     const float* pc = P.precond ? P.precond + (size_t)(off / 3) * 9 : nullptr;
     TView TV;
+    const bool fits = !TL || table_lds_bytes(m.nb, m.na, m.nsb, m.noop, m.ntor, TL == 1 ? m.npair : 0) <= (size_t)P.tbytes;
     if (TL) {
-      if (table_lds_bytes(m.nb, m.na, m.nsb, m.noop, m.ntor, TL == 1 ? m.npair : 0) > (size_t)P.tbytes) {
+      if (TL != 3 && !fits) {
         // tables larger than the reserved LDS: report and skip (the planner never does this)
         for (int i = tid; i < n; i += NT) P.x_out[off + i] = P.x_in[off + i];
         if (tid == 0) {
@@ -1211,7 +1213,7 @@ __global__ void __launch_bounds__(
         }
         continue;
       }
-      TV = stage_tables(B, m, tstage, tid, NT, TL == 1);
+      TV = stage_tables(B, m, tstage, fits ? tid : 1 << 30, NT, TL == 1);
     } else {
       TV = global_view(B, m);
     }
@@ -1260,9 +1262,11 @@ __global__ void __launch_bounds__(
 
     auto evaluate = [&](auto grad, auto energy) {
       constexpr bool G = decltype(grad)::value, EV = decltype(energy)::value;
-      if constexpr (HELP > 1)
+      if constexpr (HELP > 1) {
+        if (TL == 3 && !fits)
+          return eval_help<FAM_TG, G, EV, NT, HELP>(global_view(B, m), m, xs, gacc, P.diel, eb, P.eb_floats, ring);
         return eval_help<FAM_TG, G, EV, NT, HELP>(TV, m, xs, gacc, P.diel, eb, P.eb_floats, ring);
-      else if constexpr (ORDERED)
+      } else if constexpr (ORDERED)
         return eval_ordered<FAM_TG, G, EV, NT>(TV, m, xs, gacc, P.diel, ebuf, ebuf_n);
       else
         return eval_terms<FAM_TG, G, NT, PREF, EV>(TV, m, xs, gacc, P.diel);
@@ -2484,7 +2488,8 @@ const void* nk_kernel_ptr() {
 // kernels with NK_HELP threads per lane of 256
 constexpr int NK_HELP = 3;
 #define NK_HELP_EACH(X) \
-  X(0, 3, 2, 256) X(0, 3, 0, 256) X(1, 0, 2, 256) X(1, 0, 0, 256) X(1, 1, 2, 256) X(1, 1, 0, 256)
+  X(0, 3, 2, 256) X(0, 3, 3, 256) X(0, 3, 0, 256)                                                       \
+  X(1, 0, 2, 256) X(1, 0, 0, 256) X(1, 1, 2, 256) X(1, 1, 0, 256)
 
 #define NK_FOR_EACH(X)                                                                                   \
   X(0, 0, 1, 64) X(0, 0, 1, 128) X(0, 0, 1, 192) X(0, 0, 1, 256) X(0, 0, 1, 384) X(0, 0, 1, 512)        \
@@ -2548,7 +2553,7 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
   // Hessian; only the bonded ones beside a global Hessian, and only when that keeps the
   // unstaged kernel's workgroups per CU (there, occupancy hides the pair loads).
   const int max_wg = std::max(1, 12 / (pl.nt / 64));  // workgroups per CU at most (below)
-  bool help_stage = false;  // helper kernels may stage: as many workgroups per CU as launch without
+  bool help_stage = false;  // a launch without helpers could stage: as many workgroups per CU as launch without
   if (o->table_lds_bytes > 0) {
     const int tl = pl.hm == 0 ? 1 : 2;
     const size_t with = nk_lds_bytes(o->algo, pl.hm, pl.nt, pl.max_n, m, (size_t)o->table_lds_bytes);
@@ -2574,9 +2579,12 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
   }
   // At most one conformer per CU: the time is the longest conformer's, so its workgroup gets
   // helper threads, and L-BFGS its history in LDS where that fits (both leave the results as
-  // they are). The bonded tables are staged where a launch without helpers could (a caller whose
-  // reserve is smaller than a molecule's tables, and which the rule above spared, stays spared): ten
-  // conformers of 82 atoms 4.48 -> 4.65 ms without staging (L-BFGS), 5.50 -> 5.61 (BFGS). The bonded
+  // they are). The bonded tables are staged: ten conformers of 82 atoms 4.65 -> 4.48 ms (L-BFGS), 5.61 ->
+  // 5.50 (BFGS). Where the rule above does not stage, a caller whose reserve is smaller than a molecule's
+  // tables gets results all the same and must keep getting them: there BFGS takes the kernel that reads such
+  // tables from memory (six ragged conformers 15.7 ms, 16.1 unstaged; its second copy of the evaluation
+  // costs other batches up to 2%, so they keep the plain one), and L-BFGS, which staging gains nothing
+  // there, none. The bonded
   // terms' energies take a word each; a bonded term has at least 12 table bytes, so
   // table_lds_bytes bounds their number (eval_help takes more in windows). Ten conformers of 48 atoms, BFGS,
   // host work included: 4.28 -> 3.99 ms; 221 chains of 199-329 atoms, L-BFGS: 180 -> 127 ms (151 with
@@ -2585,12 +2593,12 @@ int make_nk_plan(const mmffhip_batch* b, const mmffhip_nk_opts* o, NkPlan& pl) {
   // conformers of 82 atoms, without and with helpers, BFGS 4.28 and 5.70 ms, L-BFGS 4.05 and 5.89;
   // 600: 6.25 and 10.1, 4.92 and 8.76.
   if (b->n_confs <= di.n_cu && o->table_lds_bytes > 0) {
-    const int eb = (o->table_lds_bytes / 12 + 64) & ~63;
+    const int eb = (o->table_lds_bytes / 12 + 64) & ~63, stage = help_stage ? 2 : 3;
     const struct {
       int hm, tl;
-    } tries[] = {{0, 2}, {0, 0}, {pl.hm, 2}, {pl.hm, 0}};
+    } tries[] = {{0, stage}, {0, 0}, {pl.hm, stage}, {pl.hm, 0}};
     for (const auto& t : tries) {
-      if ((t.hm == 0 && o->algo != MMFFHIP_LBFGS) || (t.tl > 0 && !help_stage)) continue;
+      if (t.hm == 0 && o->algo != MMFFHIP_LBFGS) continue;
       const int tb = t.tl ? ((o->table_lds_bytes + 15) / 16) * 16 : 0;
       const size_t lds = nk_lds_bytes(o->algo, t.hm, pl.nt, pl.max_n, m, (size_t)tb, NK_HELP, eb);
       if (!nk_kernel(o->algo, t.hm, t.tl, pl.nt, NK_HELP) || lds > (size_t)di.lds) continue;

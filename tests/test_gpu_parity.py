@@ -649,3 +649,26 @@ def test_one_wave_with_everything_in_lds(use_lbfgs):
         assert torch.allclose(got.x, want.x, rtol=0, atol=1e-4)
     else:
         assert torch.equal(got.x, want.x) and torch.equal(got.energy, want.energy) and (got.status == 0).all()
+
+
+@pytest.mark.parametrize("cut", [0, 32, 4096])
+def test_helpers_stage_beyond_the_other_launches_rule(cut):
+    """BFGS of molecules whose bonded tables a launch without helpers would leave in memory: helper
+    threads stage those that fit the reserve and read the others where they are, molecule by
+    molecule. Bit for bit the results without helpers and staging, with a reserve of all of the
+    largest tables, a little less, and one between the two molecules'."""
+    from mlxmolkit_archive_amd import engine, workloads
+    wls = [workloads.build(f, n_mols=1, n_confs=2) for f in ("chain", "ragged")]
+    params, counts = [p for w in wls for p in w.params], [c for w in wls for c in w.conf_counts]
+    db, x = engine.device_batch(params, counts), torch.from_numpy(np.concatenate([w.x for w in wls])).cuda()
+    kw = dict(max_iters=15, grad_tol=1e-4, ls_grad=True)
+    want = engine.NkRunner(db, stage_tables=False, **kw).run(x)
+    r = engine.NkRunner(db, **kw)
+    ln, = r.launches
+    small, big = sorted(int(v) for v in engine.table_lds_bytes(db.host, pairs=False))
+    assert ln["opts"].table_lds_bytes == big and small < big - 4096
+    ln["opts"].table_lds_bytes = big - cut
+    got = r.run(x)
+    torch.cuda.synchronize()
+    assert (got.status != 2).all() and torch.isfinite(got.energy).all()
+    assert torch.equal(got.status, want.status) and torch.equal(got.x, want.x) and torch.equal(got.energy, want.energy)
