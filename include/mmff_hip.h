@@ -114,7 +114,9 @@ typedef struct {
                               only the bonded tables (pairs stay in global memory), and only
                               when that keeps the workgroups per CU. Ignored when they do not
                               fit. A conformer whose staged tables need more gets status 2 and
-                              E = NaN */
+                              E = NaN. (Where that rule ignores it, a batch of at most one conformer
+                              per compute unit may stage the tables that fit and read the others
+                              where they are) */
   const int32_t *xcd_offsets; /* optional host array of 9 rising offsets from 0 to n_confs that
                                  split `order` into 8 per-XCD work queues: a workgroup on XCD x
                                  (workgroups go to the 8 XCDs round-robin) takes conformers from
